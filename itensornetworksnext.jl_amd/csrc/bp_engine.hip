@@ -29,6 +29,7 @@
 #include "vertex64.h"
 #include "vertex64l.h"
 #include "vertex4.h"
+#include "pair.h"
 #include "adjoint.h"
 #include "vertex_adjoint.h"
 #include "contract.h"
@@ -330,11 +331,17 @@ struct bp_context {
     // polish of every context.  Built on first use for the current topology and mask.
     Vertex64Plan v64;
     Vertex64LPlan v64l;         // bond dimensions 9..16 (vertex64l.h), when the D <= 8 plan
-    int v64_kind = 0;           // declines: 1 the D <= 8 kernel, 2 the large-bond one
+    int v64_kind = 0;           // declines: 1 the D <= 8 kernel, 2 the large-bond one, 3 the
+                                // pair kernel in the D <= 8 kernel's place
     bool v64_tried = false;     // plan attempted (v64_plan_ok tells the outcome)
     bool v64_plan_ok = false;
     bool v64_sites = false;     // padded FP64 slices match the current sites
     bool v64_ok = false;        // plan and slices ready
+
+    // pair kernel (pair.hip) in complex FP64 (complex contexts) or FP64 (the sweeps of FP64
+    // contexts, the FP64 polish of the others); built on first use for the current topology
+    PairPlan pair;
+    bool pair_tried = false, pair_ok = false;
 
     // cached sweep graphs (16 sweeps + bookkeeping), one per starting buffer parity; valid
     // while graph_epoch equals the process-wide plan epoch (which moves whenever a captured
@@ -441,6 +448,8 @@ static void free_all(bp_context *c) {
     vertex64l_release(&c->v64l);
     c->v64_kind = 0;
     c->v64_tried = c->v64_plan_ok = c->v64_sites = c->v64_ok = false;
+    pair_release(&c->pair);
+    c->pair_tried = c->pair_ok = false;
     for (auto &b : c->gb)
         if (b.d_slots) (void)hipFree(b.d_slots);
     c->gb.clear();
@@ -570,14 +579,45 @@ static void free_buckets(bp_context *c) {
     c->gb_path = -1;
 }
 
-// Buckets of the generic slots of `path` (all slots, or the slots outside the vertex bucket).
+// The pair kernel (pair.hip) sweeps the vertices it takes on the automatic path of FP64 and
+// complex contexts; a forced generic path and unnormalised updates stay on the generic
+// kernel.  Measured per sweep against it: see pair_plan_build.
+static bool pair_used(const bp_context *c) {
+    return c->pair_ok && c->normalize && c->path == BP_PATH_AUTO &&
+           (c->dtype == BP_F64 || c->is_cplx());
+}
+
+// Plan of the pair kernel for this topology.  Allocates: never called inside a capture.
+static int ensure_pair(bp_context *c) {
+    if (c->pair_tried || !c->have_topo) return BP_OK;
+    c->pair_tried = true;
+    const int rc = pair_plan_build(&c->pair, c->is_cplx() ? PAIR_C128 : PAIR_F64, c->plain, c->nv,
+                                   c->nnet, c->port_off.data(), c->port_edge.data(),
+                                   c->edge_dim.data(), c->phys_dim.data(), c->port_rev.data(),
+                                   c->vnet.data(), c->site_off.data(), c->msg_off.data());
+    if (rc != 0 && rc != 4) return set_err(BP_ERR_HIP, "pair kernel plan failed");
+    c->pair_ok = rc == 0;
+    bump_epoch();
+    return BP_OK;
+}
+
+// What the buckets of a path are built for: the path, and whether the pair kernel takes its
+// vertices out of them.
+static int bucket_id(const bp_context *c, int path) {
+    return path * 2 + (path == BP_PATH_GENERIC && pair_used(c) ? 1 : 0);
+}
+
+// Buckets of the generic slots of `path` (all slots, or the slots that neither the vertex
+// bucket nor the pair kernel takes).
 static int build_buckets(bp_context *c, int path) {
-    if (c->gb_path == path) return BP_OK;
+    if (c->gb_path == bucket_id(c, path)) return BP_OK;
     free_buckets(c);
-    if (path == BP_PATH_VERTEX) { c->gb_path = path; return BP_OK; }
+    if (path == BP_PATH_VERTEX) { c->gb_path = bucket_id(c, path); return BP_OK; }
     std::vector<int> all;
     const std::vector<int> *slots = &c->vplan.gen_slots;
-    if (path != BP_PATH_MIXED) {
+    if (path == BP_PATH_GENERIC && pair_used(c)) {
+        slots = &c->pair.rest;
+    } else if (path != BP_PATH_MIXED) {
         all.resize(c->nports);
         for (int q = 0; q < c->nports; ++q) all[q] = q;
         slots = &all;
@@ -616,7 +656,7 @@ static int build_buckets(bp_context *c, int path) {
         }
         RETCHK(upload(&b.d_slots, b.slots));
     }
-    c->gb_path = path;
+    c->gb_path = bucket_id(c, path);
     return BP_OK;
 }
 
@@ -705,6 +745,8 @@ static int launch_edge_scalars(bp_context *c, const T *msgs) {
 // kernel, or the vertex bucket plus the generic kernel for the remaining networks.
 
 
+static constexpr double PAIR_MFMA_MAX = 400.0;
+
 // The FP64 vertex plan for this context's networks (bond dimensions enabled: the context's
 // vertex mask in FP64 contexts; 6..8 and 9..16 for the polish of FP32/BF16 contexts): the
 // D <= 8 kernel (vertex64.h) when every network's largest bond dimension is 6..8, else the
@@ -729,13 +771,23 @@ static int ensure_v64(bp_context *c) {
                                      lmask) == 0)
                 c->v64_kind = 2;
         }
+        // The pair kernel in its place where it is the faster one: its time grows with the
+        // products it pads to 16 x 16, the other's is that of bond dimension 8.  us per sweep,
+        // d = 2, pair / other: D = 6 (324 products per slice) 23 / 36 at 16x16 and 71 / 82 at
+        // 32x32; D = 7 (832) 33 / 36 and 118 / 83; D = 8 of degree 3 (152) 21 / 41 at 8x16 hex
+        RETCHK(ensure_pair(c));
+        if (c->v64_kind == 1 && c->pair_ok && c->pair.covers && pair_mfma_per_slice(&c->pair) <= PAIR_MFMA_MAX) {
+            vertex64_release(&c->v64);
+            c->v64_kind = 3;
+        }
         c->v64_plan_ok = c->v64_kind != 0;
         c->v64_tried = true;
         c->v64_sites = false;
         bump_epoch();
     }
     if (c->v64_plan_ok && c->have_sites && !c->v64_sites) {
-        const int rc = c->v64_kind == 1
+        const int rc = c->v64_kind == 3 ? 0  // reads the master copy
+                       : c->v64_kind == 1
                            ? vertex64_upload_sites(&c->v64, c->stream, c->d_sites64, c->d_site_off,
                                                    c->d_port_off, c->d_port_edge, c->d_edge_dim)
                            : vertex64l_upload_sites(&c->v64l, c->stream, c->d_sites64,
@@ -758,8 +810,12 @@ static void v64_invalidate(bp_context *c) {
 }
 
 // One FP64 sweep on the context's FP64 vertex kernel (ensure_v64 has made it ready).
-static int v64_sweep(bp_context *c, const double *src, double *dst, const NetCtl &ctl) {
-    const int rc = c->v64_kind == 1
+static int v64_sweep(bp_context *c, const double *src, double *dst, const NetCtl &ctl,
+                     const SweepFold &fold = SweepFold{}) {
+    const int rc = c->v64_kind == 3
+                       ? pair_sweep(&c->pair, c->stream, c->d_sites64, src, dst, ctl,
+                                    c->d_res_fid, c->d_res_abs, fold)
+                   : c->v64_kind == 1
                        ? vertex64_sweep(&c->v64, c->stream, c->d_msg_off, src, dst, ctl,
                                         c->d_res_fid, c->d_res_abs)
                        : vertex64l_sweep(&c->v64l, c->stream, c->d_msg_off, src, dst, ctl,
@@ -792,8 +848,9 @@ static int prepare_sweep(bp_context *c) {
     const int path = resolve_path(c);
     if (path < 0) return BP_OK;  // reported by sweep_once
     RETCHK(gen_set_lds_limits());
+    if (path == BP_PATH_GENERIC) RETCHK(ensure_pair(c));
     RETCHK(build_buckets(c, path));
-    if (c->vplan_ok && c->fold_n != c->nnet) {
+    if ((c->vplan_ok || c->pair_ok) && c->fold_n != c->nnet) {
         // folded residual accumulators, FOLD_BUFS rotating buffers (outside any graph
         // capture); every run starts by clearing them (k_reset_nets)
         const size_t nb = sizeof(unsigned long long) * FOLD_BUFS * FOLD_SLOTS * (size_t)c->nnet;
@@ -868,13 +925,15 @@ static const float *generic_sites32(const bp_context *c) {
 }
 
 // One Jacobi sweep on the working dtype: reads d_msg[cur], writes d_msg[cur^1].
-// Whether the residual reduction can ride on the sweep kernel: the D <= 8 four-port kernel
-// alone updates every message of every network.
-static bool fold_possible(const bp_context *c) {
-    return c->vplan_ok && c->vplan.all && c->vplan.nv_k3 == 0 && c->vplan.nv16 == 0 &&
+// Whether the residual reduction can ride on the sweep kernel: one kernel (the D <= 8
+// four-port kernel, or the pair kernel) updates every message of every network.
+static bool fold_possible(const bp_context *c, int path) {
+    if (!c->d_fold_acc || c->fold_n != c->nnet || !c->fold_on) return false;
+    if (path == BP_PATH_GENERIC) return pair_used(c) && c->pair.covers;
+    if (c->dtype == BP_F64) return c->v64_kind == 3;
+    return path == BP_PATH_VERTEX && c->vplan_ok && c->vplan.all && c->vplan.nv_k3 == 0 && c->vplan.nv16 == 0 &&
            c->vplan.ns_total() == 0 &&
-           c->path != BP_PATH_GENERIC && c->d_fold_acc && c->fold_n == c->nnet &&
-           c->vplan.nv > 0 && c->vplan.d_lead && c->fold_on;
+           c->path != BP_PATH_GENERIC && c->vplan.nv > 0 && c->vplan.d_lead;
 }
 
 // One Jacobi sweep; with `folded` non-null and the bookkeeping foldable, the sweep kernel
@@ -886,26 +945,28 @@ static int sweep_once(bp_context *c, const NetCtl &done, bool *folded = nullptr,
     const int path = resolve_path(c);
     if (path < 0) return set_err(BP_ERR_UNSUPPORTED, "vertex path not available: %s",
                                  c->vplan.why.c_str());
-    if (c->gb_path != path)  // normally done by prepare_sweep, outside any graph capture
+    if (c->gb_path != bucket_id(c, path))  // normally done by prepare_sweep, outside any graph capture
         RETCHK(prepare_sweep(c));
     void *src = c->d_msg[c->cur], *dst = c->d_msg[c->cur ^ 1];
     SweepFold fold{};
     if (folded) *folded = false;
-    if (folded && done.enabled && path == BP_PATH_VERTEX && fold_possible(c)) {
+    const bool pair = path == BP_PATH_GENERIC && pair_used(c);  // of its own, not as the FP64
+                                                                // vertex path's kernel
+    if (folded && done.enabled && fold_possible(c, path)) {
         const size_t stride = FOLD_SLOTS * (size_t)c->fold_n;
         fold.acc = c->d_fold_acc + (size_t)(k % FOLD_BUFS) * stride;
         fold.rp = c->d_runp;
         fold.prev = apply_prev ? c->d_fold_acc + (size_t)((k + FOLD_BUFS - 1) % FOLD_BUFS) * stride
                                : nullptr;
         fold.clear = c->d_fold_acc + (size_t)((k + 1) % FOLD_BUFS) * stride;
-        fold.lead = c->vplan.d_lead;
+        fold.lead = pair || c->dtype == BP_F64 ? c->pair.d_lead : c->vplan.d_lead;
         fold.iter = c->d_iter;
         fold.delta = c->d_delta;
         fold.at = c->d_at;
         *folded = true;
     }
     if (path == BP_PATH_VERTEX && c->dtype == BP_F64) {
-        RETCHK(v64_sweep(c, (const double *)src, (double *)dst, done));
+        RETCHK(v64_sweep(c, (const double *)src, (double *)dst, done, fold));
     } else if (path == BP_PATH_VERTEX || path == BP_PATH_MIXED) {
         RETCHK(vertex_sweep(&c->vplan, c->stream, c->topo(), c->d_vsites, src, dst, done,
                             c->d_res_fid, c->d_res_abs, fold));
@@ -918,6 +979,9 @@ static int sweep_once(bp_context *c, const NetCtl &done, bool *folded = nullptr,
             return set_err(BP_ERR_HIP, "small-bond sweep launch failed");
         HIPCHK(hipGetLastError());
     }
+    if (pair && pair_sweep(&c->pair, c->stream, c->d_sites, src, dst, done, c->d_res_fid,
+                           c->d_res_abs, fold) != 0)
+        return set_err(BP_ERR_HIP, "pair sweep launch failed");
     if (path != BP_PATH_VERTEX) {
         if (c->is_cplx())
             RETCHK(launch_buckets<cplx>(c, (const cplx *)c->d_sites, (const cplx *)src,
@@ -1182,6 +1246,8 @@ int bp_set_topology(bp_context *c, int nv, int ne, const int *port_off, const in
     if (c->d_msg64[1]) { (void)hipFree(c->d_msg64[1]); c->d_msg64[1] = nullptr; }
     c->fp64_active = false;
     c->cur = 0;
+    pair_release(&c->pair);
+    c->pair_tried = c->pair_ok = false;
     RETCHK(rebuild_vertex_plan(c));
     c->have_topo = true;
     c->have_sites = false;
@@ -2314,13 +2380,21 @@ int bp_polish_fp64(bp_context *c, int nsweeps, double *out_delta) {
         c->fp64_active = true;
     }
     // FP64 sweeps on an FP64 vertex kernel when one covers the networks (largest bond
-    // dimensions 6..8 or 9..16 in FP32/BF16 contexts), else on the generic kernel
+    // dimensions 6..8 or 9..16 in FP32/BF16 contexts), on the pair kernel when that does, else
+    // on the generic kernel
     if (c->normalize) RETCHK(ensure_v64(c));
     const bool v64 = c->normalize && c->v64_ok && c->path != BP_PATH_GENERIC;
+    const bool pair = c->normalize && c->path == BP_PATH_AUTO && c->pair_ok &&
+                      c->pair.rest.empty();
     for (int i = 0; i < nsweeps; ++i) {
         if (v64) {
             RETCHK(v64_sweep(c, c->d_msg64[c->cur64], c->d_msg64[c->cur64 ^ 1],
                              make_ctl(c, false)));
+        } else if (pair) {
+            if (pair_sweep(&c->pair, c->stream, c->d_sites64, c->d_msg64[c->cur64],
+                           c->d_msg64[c->cur64 ^ 1], make_ctl(c, false), c->d_res_fid,
+                           c->d_res_abs, SweepFold{}) != 0)
+                return set_err(BP_ERR_HIP, "pair sweep launch failed");
         } else {
             RETCHK(launch_update_generic<double>(c, c->d_sites64, c->d_msg64[c->cur64],
                                                  c->d_msg64[c->cur64 ^ 1], make_ctl(c, false), 0,

@@ -169,6 +169,37 @@ __device__ __forceinline__ double wave_max_v(double v) {
     return vmax_nan(h.first, h.second);
 }
 
+// Whether network `net` is stopped for this sweep.  With fold.prev set, the previous sweep's
+// stopping rule (StopWhenConverged on the maximum of its FOLD_SLOTS accumulators) is applied
+// first: every wave of every work item of the network computes the same decision (a racing
+// read of the lead's done flag sees 0 or 1, and either way ends stopped), and the lead item
+// records the iteration, delta, done and at.  StopAfterIteration is left to the kernel that
+// ends the sequence: no sequence runs past maxiter.  The lead item also clears fold.clear.
+__device__ __forceinline__ bool vx_fold_begin(const NetCtl &ctl, const SweepFold &fold, int net,
+                                              int u) {
+    const int lane = threadIdx.x & 63;
+    const bool lead = fold.lead && fold.lead[net] == u;
+    if (lead && fold.clear && threadIdx.x < FOLD_SLOTS)
+        fold.clear[(long long)net * FOLD_SLOTS + threadIdx.x] = 0ull;
+    const bool was = ctl.enabled && ctl.done[net];
+    if (!fold.prev) return was;
+    const unsigned long long b =
+        lane < FOLD_SLOTS ? fold.prev[(long long)net * FOLD_SLOTS + lane] : 0ull;
+    const double m = wave_max_v(__longlong_as_double((long long)b));
+    const double tol = fold.rp->tol;
+    const bool newly = !was && tol >= 0.0 && m < tol;
+    if (lead && threadIdx.x == 0 && !was) {
+        const int it = fold.iter[net] + 1;
+        fold.iter[net] = it;
+        fold.delta[net] = m;
+        if (newly) {
+            ctl.done[net] = 1;
+            fold.at[net] = it;
+        }
+    }
+    return was || newly;
+}
+
 // Neumaier-compensated running sum of doubles (the log-norm accumulations).
 struct NeuSum {
     double s = 0.0, c = 0.0;

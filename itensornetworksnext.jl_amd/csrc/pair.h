@@ -1,0 +1,58 @@
+// pair.h -- sweep kernel for vertices of degree <= 4 and bond dimensions <= 8, FP64, complex
+// FP64 or FP32, in the unpadded site layout of the generic kernel (kernel: pair.hip).
+#pragma once
+
+#include <string>
+#include <vector>
+
+#include "common.h"
+
+#define PAIR_MAXD 8        // largest bond dimension
+#define PAIR_SIDE 64       // largest pair dimension (two bonds of PAIR_MAXD)
+#define PAIR_MAXWAVES 8    // waves per workgroup
+
+enum { PAIR_F64 = 0, PAIR_C128 = 1, PAIR_F32 = 2 };
+
+// One vertex as the kernel reads it.  Its ports are split into two pairs of consecutive
+// tensor axes, positions (0, 1) and (2, 3): degree 4 (p0 p1)(p2 p3), degree 3 (p0 p1)(p2),
+// degree 2 (p0)(p1), degree 1 (p0)().  An absent position has dimension 1 and slot -1.
+struct PairRec {
+    long long site;     // element offset of the site tensor
+    long long in[4];    // element offset of the incoming message per position
+    long long out[4];   // element offset of the outgoing message
+    int slot[4];        // outgoing message slot
+    int dim[4];
+    int d, net;
+    int n[2];           // pair dimensions dim[0] dim[1], dim[2] dim[3]
+    int vertex, pad;
+};
+
+struct PairPlan {
+    int dtype = PAIR_F64;
+    std::vector<PairRec> recs;       // one per vertex of positive degree
+    std::vector<int> rec_of;         // vertex -> record, -1 when the vertex does not qualify
+    std::vector<int> rest;           // message slots of the other vertices
+    PairRec *d_recs = nullptr;
+    int *d_lead = nullptr;           // per network: its first record
+    bool covers = false;             // it takes every vertex of every network
+    int nt = 0;                      // 16-wide tiles of the largest pair dimension
+    int chunk = 0, split = 0;        // slices staged in LDS at once; waves sharing a tile's slices
+    int waves = 0;
+    int slice_elems = 0, env_elems = 0;  // LDS elements per plane
+    size_t lds_bytes = 0;
+};
+
+void pair_release(PairPlan *p);
+// 0 on success, 4 when no vertex qualifies, other values on a device error
+int pair_plan_build(PairPlan *p, int dtype, int plain, int nv, int nnet, const int *port_off,
+                    const int *port_edge, const int *edge_dim, const int *phys_dim,
+                    const int *port_rev, const int *vnet, const long long *site_off,
+                    const long long *msg_off);
+// 16x16x4 products per physical slice of a vertex, on average: the kernel's time grows with it
+double pair_mfma_per_slice(const PairPlan *p);
+// One launch over records [0, n) when `items` is null (every message of every record), else
+// over n work items of `items` (record * 4 + position: one message each).  src == dst is
+// allowed for messages that no work item of the launch reads.
+int pair_sweep(const PairPlan *p, hipStream_t st, const void *sites, const void *src, void *dst,
+               const NetCtl &ctl, double *res_fid, double *res_abs, const SweepFold &fold,
+               const int *items = nullptr, int n = 0);
