@@ -2140,6 +2140,75 @@ int bp_iterate_diff(bp_context *c, const double *other, double *out) {
     return BP_OK;
 }
 
+// The updates of one sequential sweep, regrouped into levels that keep the sweep's results:
+// an update comes after the earlier updates of the messages it reads, and after the earlier
+// readers and writers of the message it writes, so the updates of one level touch disjoint
+// messages and run as one launch.  Over the forest cover of an L x L lattice (4 L (L - 1)
+// updates) there are about 4 L levels.  `items` holds the slots level by level, a level's
+// pair-kernel items (record * 4 + position) before its generic slots.
+struct SeqLevel {
+    int begin, pairs, end;
+};
+
+static void seq_levels(const bp_context *c, const int *order, int n, bool pair,
+                       std::vector<int> *items, std::vector<SeqLevel> *levels) {
+    std::vector<int> wrote(c->nports, -1), read(c->nports, -1), level(n);
+    int nl = 0;
+    for (int i = 0; i < n; ++i) {
+        const int q = order[i], u = c->owner[q];
+        int l = std::max(wrote[q], read[q]) + 1;
+        for (int j = c->port_off[u]; j < c->port_off[u + 1]; ++j)
+            if (j != q) l = std::max(l, wrote[c->port_rev[j]] + 1);
+        for (int j = c->port_off[u]; j < c->port_off[u + 1]; ++j)
+            if (j != q) read[c->port_rev[j]] = std::max(read[c->port_rev[j]], l);
+        wrote[q] = l;
+        level[i] = l;
+        nl = std::max(nl, l + 1);
+    }
+    auto pair_item = [&](int q) {
+        if (!pair) return -1;
+        const int u = c->owner[q], r = c->pair.rec_of[u];
+        if (r < 0) return -1;
+        for (int t = 0; t < 4; ++t)
+            if (c->pair.recs[r].slot[t] == q) return 4 * r + t;
+        return -1;
+    };
+    std::vector<std::vector<int>> pairs(nl), rest(nl);
+    for (int i = 0; i < n; ++i) {
+        const int it = pair_item(order[i]);
+        if (it >= 0) pairs[level[i]].push_back(it);
+        else rest[level[i]].push_back(order[i]);
+    }
+    for (int l = 0; l < nl; ++l) {
+        SeqLevel v;
+        v.begin = (int)items->size();
+        items->insert(items->end(), pairs[l].begin(), pairs[l].end());
+        v.pairs = (int)items->size();
+        items->insert(items->end(), rest[l].begin(), rest[l].end());
+        v.end = (int)items->size();
+        levels->push_back(v);
+    }
+}
+
+// One level of a sequential sweep, in place on m.
+static int seq_launch(bp_context *c, const SeqLevel &v, const int *d_items, void *m,
+                      const NetCtl &ctl) {
+    if (v.pairs > v.begin &&
+        pair_sweep(&c->pair, c->stream, c->d_sites, m, m, ctl, c->d_res_fid, c->d_res_abs,
+                   SweepFold{}, d_items + v.begin, v.pairs - v.begin) != 0)
+        return set_err(BP_ERR_HIP, "pair update launch failed");
+    if (v.end == v.pairs) return BP_OK;
+    const int n = v.end - v.pairs, *list = d_items + v.pairs;
+    if (c->is_cplx())
+        return launch_update_generic<cplx>(c, (const cplx *)c->d_sites, (const cplx *)m,
+                                           (cplx *)m, ctl, 0, n, list, gen_flags(c, false));
+    if (c->dtype == BP_F64)
+        return launch_update_generic<double>(c, (const double *)c->d_sites, (const double *)m,
+                                             (double *)m, ctl, 0, n, list, gen_flags(c, false));
+    return launch_update_generic<float>(c, generic_sites32(c), (const float *)m, (float *)m, ctl,
+                                        0, n, list, gen_flags(c, c->dtype == BP_BF16));
+}
+
 int bp_run_sequential(bp_context *c, const int *order, int norder, int maxiter, double tol,
                       int criterion, int *out_sweeps, double *out_delta, int *out_at) {
     RETCHK(ready(c));
@@ -2154,13 +2223,20 @@ int bp_run_sequential(bp_context *c, const int *order, int norder, int maxiter, 
     c->fp64_active = false;
     const int cap = maxiter > 0 ? maxiter : 100000;
     const size_t es = c->elt();
+    if (c->dtype == BP_F64 || c->is_cplx()) RETCHK(ensure_pair(c));
+    std::vector<int> items;
+    std::vector<SeqLevel> levels;
+    seq_levels(c, order, norder, pair_used(c), &items, &levels);
     void *prev = nullptr;
+    int *d_items = nullptr;
     HIPCHK(hipMalloc(&prev, es * std::max<long long>(c->nmsg, 1)));
+    int rc = upload(&d_items, items);
     std::vector<double> res(c->nports);
     const NetCtl off = make_ctl(c, false);
-    int it = 0, at = -1, rc = BP_OK;
+    int it = 0, at = -1;
     double delta = INFINITY;
-    HIPCHK(hipEventRecord(c->ev0, c->stream));
+    if (rc == BP_OK && hipEventRecord(c->ev0, c->stream) != hipSuccess)
+        rc = set_err(BP_ERR_HIP, "event record failed");
     while (rc == BP_OK && it < cap) {
         if (hipMemcpyAsync(prev, c->d_msg[c->cur], es * c->nmsg, hipMemcpyDeviceToDevice,
                            c->stream) != hipSuccess) {
@@ -2168,20 +2244,8 @@ int bp_run_sequential(bp_context *c, const int *order, int norder, int maxiter, 
             break;
         }
         void *m = c->d_msg[c->cur];
-        for (int i = 0; i < norder && rc == BP_OK; ++i) {
-            if (c->is_cplx())
-                rc = launch_update_generic<cplx>(c, (const cplx *)c->d_sites, (const cplx *)m,
-                                                 (cplx *)m, off, order[i], order[i] + 1, nullptr,
-                                                 gen_flags(c, false));
-            else if (c->dtype == BP_F64)
-                rc = launch_update_generic<double>(c, (const double *)c->d_sites,
-                                                   (const double *)m, (double *)m, off, order[i],
-                                                   order[i] + 1, nullptr, gen_flags(c, false));
-            else
-                rc = launch_update_generic<float>(c, generic_sites32(c), (const float *)m,
-                                                  (float *)m, off, order[i], order[i] + 1,
-                                                  nullptr, gen_flags(c, c->dtype == BP_BF16));
-        }
+        for (size_t l = 0; l < levels.size() && rc == BP_OK; ++l)
+            rc = seq_launch(c, levels[l], d_items, m, off);
         if (rc != BP_OK) break;
         ++it;
         if (tol >= 0.0) {
@@ -2209,6 +2273,7 @@ int bp_run_sequential(bp_context *c, const int *order, int norder, int maxiter, 
     (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
     c->last_ms = ms;
     (void)hipFree(prev);
+    if (d_items) (void)hipFree(d_items);
     if (rc != BP_OK) return rc;
     if (out_sweeps) *out_sweeps = it;
     if (out_delta) *out_delta = delta;
