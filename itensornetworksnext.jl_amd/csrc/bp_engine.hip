@@ -85,14 +85,15 @@ static double *g_scratch_ptr[BP_SCRATCH_DEVICES] = {};
 
 // ------------------------------------------------------------------ small kernels
 
+// 16 lanes per message (a workgroup per message: 59 us for 261 120 of 3 x 3)
 template <typename T>
-__global__ void k_init_messages(DevTopo tp, T *m, int kind) {
-    const int q = blockIdx.x;
+__global__ __launch_bounds__(256) void k_init_messages(DevTopo tp, T *m, int kind) {
+    const int q = blockIdx.x * 16 + threadIdx.x / 16;
     if (q >= tp.nports) return;
     const long long off = tp.msg_off[q];
     const int len = (int)(tp.msg_off[q + 1] - off);
     const int D = tp.edge_dim[tp.port_edge[q]];
-    for (int i = threadIdx.x; i < len; i += blockDim.x) {
+    for (int i = threadIdx.x % 16; i < len; i += 16) {
         T v = T(1);
         if (kind == BP_INIT_IDENTITY && !tp.plain) v = (i / D == i % D) ? T(1) : T(0);
         m[off + i] = v;
@@ -164,6 +165,29 @@ __global__ __launch_bounds__(1024) void k_reduce_nets(const int *pbeg, const dou
     }
 }
 
+// The maxima of k_reduce_nets for networks of many slots: RED_SLOTS slots a workgroup, folded
+// into the network's accumulators (k_reduce_folded applies the rule).
+#define RED_SLOTS 4096
+__global__ __launch_bounds__(256) void k_reduce_parts(const int *pbeg, const double *res_fid,
+                                                      const double *res_abs, const RunParams *rp,
+                                                      const int *done, unsigned long long *acc) {
+    __shared__ double red[4];
+    const int n = blockIdx.y;
+    const int q0 = pbeg[n] + blockIdx.x * RED_SLOTS, q1 = min(q0 + RED_SLOTS, pbeg[n + 1]);
+    if (q0 >= q1 || done[n]) return;  // uniform over the workgroup
+    const double *res = rp->crit == BP_CRIT_FIDELITY ? res_fid : res_abs;
+    double m = 0.0;
+    for (int q = q0 + threadIdx.x; q < q1; q += 256) m = fold_max(m, res[q]);
+    m = wave_max_v(m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < 4; ++k) m = fold_max(m, red[k]);
+        atomicMax(acc + (long long)n * FOLD_SLOTS + blockIdx.x % FOLD_SLOTS,
+                  (unsigned long long)__double_as_longlong(m));
+    }
+}
+
 // Per-slot distance between two message buffers (one wave per slot): the reference's
 // iterate_diff term 1 - |<a^, b^>|^2 (beliefpropagation.jl:261-267) and max |a - b|.
 template <typename Ta, typename Tb>
@@ -193,53 +217,95 @@ __global__ void k_diff_slots(DevTopo tp, const Ta *a, const Tb *b, double *res_f
     }
 }
 
-// BP log-norm per network (one workgroup per network): Neumaier-compensated (NeuSum)
-// sum log|Z_v| - sum log|Z_e| with the reference's complex promotion and -Inf rule
-// (messagecache.jl:185-201).
+// BP log-norm per network: sum log Z_v - sum log Z_e, Neumaier-compensated, with the
+// reference's complex promotion and -Inf rule (messagecache.jl:185-201).  Real terms: log|z|
+// and pi times the number of negative vertex terms minus that of negative edge terms; complex
+// terms (CX): the principal logarithm log|z| + i arg z of every term.  Any Z_e = 0 gives -Inf,
+// a Z_v = 0 a real part of -Inf.
+//
+// Many workgroups per network (LN_TERMS terms each) leave their sums in `parts`, and one wave
+// per network joins them.  A single workgroup per network took 1.14 ms for 326 656 terms, and
+// its serial last sum 15 of the 20 us of a small network.
+#define LN_TERMS 4096
+#define LN_PARTS 64  // workgroups per network at most
 
-__global__ __launch_bounds__(BP_BLOCK) void k_lognorm_nets(DevTopo tp, const int *vbeg,
-                                                            const int *pbeg, const double *zv,
-                                                            const double *ze, double *out_re,
-                                                            double *out_im) {
-    __shared__ double ss[BP_BLOCK], cc[BP_BLOCK];
-    __shared__ int cnt[4];
+struct LnPart {
+    double s, c;    // compensated sum of the real parts
+    double a, ac;   // complex: of the angles; real: a = number of negative terms (signed)
+    int zv0, ze0;   // a zero vertex / edge term was seen
+};
+
+__device__ __forceinline__ void ln_join(NeuSum &t, double s, double c) {
+    t.add(s);
+    t.c += c;
+}
+
+// wave64 sum of the lanes' parts (every lane gets it)
+__device__ __forceinline__ LnPart ln_wave(LnPart p) {
+    for (int o = 32; o > 0; o >>= 1) {
+        NeuSum t, u;
+        t.s = p.s, t.c = p.c, u.s = p.a, u.c = p.ac;
+        ln_join(t, __shfl_xor(p.s, o, 64), __shfl_xor(p.c, o, 64));
+        ln_join(u, __shfl_xor(p.a, o, 64), __shfl_xor(p.ac, o, 64));
+        p.s = t.s, p.c = t.c, p.a = u.s, p.ac = u.c;
+        p.zv0 |= __shfl_xor(p.zv0, o, 64);
+        p.ze0 |= __shfl_xor(p.ze0, o, 64);
+    }
+    return p;
+}
+
+template <bool CX>
+__device__ __forceinline__ void ln_out(const LnPart &p, double *re, double *im) {
+    double r = p.s + p.c, i = CX ? p.a + p.ac : M_PI * p.a;
+    if (p.ze0) { r = -INFINITY; i = 0.0; }
+    else if (p.zv0) r = -INFINITY;
+    *re = r;
+    *im = i;
+}
+
+template <bool CX>
+__global__ __launch_bounds__(256) void k_lognorm_parts(DevTopo tp, const int *vbeg,
+                                                       const int *pbeg, const double *zv,
+                                                       const double *ze, LnPart *parts,
+                                                       double *out_re, double *out_im) {
+    __shared__ LnPart wp[4];
+    const int n = blockIdx.y, step = gridDim.x * 256;
+    NeuSum acc, ang;
+    LnPart p{};
+    auto term = [&](const double *z, int i, double sign, int &zero) {
+        const double x = CX ? z[2 * (long long)i] : z[i], y = CX ? z[2 * (long long)i + 1] : 0.0;
+        if (x == 0.0 && y == 0.0) { zero = 1; return; }
+        if constexpr (CX) {
+            ang.add(sign * atan2(y, x));
+            acc.add(sign * log(hypot(x, y)));
+        } else {
+            if (x < 0.0) ang.add(sign);
+            acc.add(sign * log(fabs(x)));
+        }
+    };
+    for (int u = vbeg[n] + blockIdx.x * 256 + threadIdx.x; u < vbeg[n + 1]; u += step)
+        term(zv, u, 1.0, p.zv0);
+    for (int q = pbeg[n] + blockIdx.x * 256 + threadIdx.x; q < pbeg[n + 1]; q += step)
+        if (q <= tp.port_rev[q]) term(ze, tp.port_edge[q], -1.0, p.ze0);
+    p.s = acc.s, p.c = acc.c, p.a = ang.s, p.ac = ang.c;
+    p = ln_wave(p);
+    if ((threadIdx.x & 63) == 0) wp[threadIdx.x >> 6] = p;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    p = threadIdx.x < 4 ? wp[threadIdx.x] : LnPart{};
+    p = ln_wave(p);
+    if (threadIdx.x != 0) return;
+    if (gridDim.x == 1) ln_out<CX>(p, out_re + n, out_im + n);
+    else parts[n * (long long)LN_PARTS + blockIdx.x] = p;
+}
+
+template <bool CX>
+__global__ __launch_bounds__(64) void k_lognorm_join(const LnPart *parts, int np, double *out_re,
+                                                     double *out_im) {
     const int n = blockIdx.x;
-    if (threadIdx.x < 4) cnt[threadIdx.x] = 0;
-    __syncthreads();
-    NeuSum acc;
-    int negv = 0, nege = 0, zv0 = 0, ze0 = 0;
-    for (int u = vbeg[n] + threadIdx.x; u < vbeg[n + 1]; u += blockDim.x) {
-        const double x = zv[u];
-        if (x == 0.0) { zv0 = 1; continue; }
-        if (x < 0.0) ++negv;
-        acc.add(log(fabs(x)));
-    }
-    for (int q = pbeg[n] + threadIdx.x; q < pbeg[n + 1]; q += blockDim.x) {
-        if (q > tp.port_rev[q]) continue;
-        const double x = ze[tp.port_edge[q]];
-        if (x == 0.0) { ze0 = 1; continue; }
-        if (x < 0.0) ++nege;
-        acc.add(-log(fabs(x)));
-    }
-    ss[threadIdx.x] = acc.s;
-    cc[threadIdx.x] = acc.c;
-    atomicAdd(&cnt[0], negv);
-    atomicAdd(&cnt[1], nege);
-    atomicOr(&cnt[2], zv0);
-    atomicOr(&cnt[3], ze0);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        NeuSum t;
-        for (int i = 0; i < (int)blockDim.x; ++i) t.add(ss[i]);
-        double c = 0.0;
-        for (int i = 0; i < (int)blockDim.x; ++i) c += cc[i];
-        double re = t.s + (t.c + c);
-        double im = M_PI * (double)(cnt[0] - cnt[1]);
-        if (cnt[3]) { re = -INFINITY; im = 0.0; }
-        else if (cnt[2]) re = -INFINITY;
-        out_re[n] = re;
-        out_im[n] = im;
-    }
+    LnPart p = (int)threadIdx.x < np ? parts[n * (long long)LN_PARTS + threadIdx.x] : LnPart{};
+    p = ln_wave(p);
+    if (threadIdx.x == 0) ln_out<CX>(p, out_re + n, out_im + n);
 }
 
 // ------------------------------------------------------------------ context
@@ -304,7 +370,9 @@ struct bp_context {
     int cur64 = 0;
     bool fp64_active = false;  // messages currently live in d_msg64[cur64]
     double *d_res_fid = nullptr, *d_res_abs = nullptr;
-    double *d_zv = nullptr, *d_ze = nullptr, *d_lre = nullptr, *d_lim = nullptr;
+    double *d_zv = nullptr, *d_ze = nullptr;
+    double *d_lre = nullptr;       // log-norms: nnet real parts, nnet imaginary parts
+    LnPart *d_lnp = nullptr;       // partial sums of the log-norms (networks of many terms)
     int *d_done = nullptr, *d_iter = nullptr, *d_at = nullptr;
     double *d_delta = nullptr;
     unsigned long long *d_fold_acc = nullptr;  // per network (folded residual reduction)
@@ -438,7 +506,7 @@ static void free_all(bp_context *c) {
                     c->d_phys_dim, c->d_owner, c->d_vnet, c->d_vbeg, c->d_pbeg, c->d_site_off,
                     c->d_msg_off, c->d_sites64, c->d_sites, c->d_msg[0], c->d_msg[1],
                     c->d_msg64[0], c->d_msg64[1], c->d_res_fid, c->d_res_abs, c->d_zv, c->d_ze,
-                    c->d_lre, c->d_lim, c->d_delta, c->d_ws,
+                    c->d_lre, c->d_lnp, c->d_delta, c->d_ws,
                     c->d_vsites, c->d_sites_bf, c->d_runp, c->d_fold_acc};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -726,14 +794,25 @@ static int launch_vertex_scalars(bp_context *c, const T *sites, const T *msgs) {
 
 template <typename T>
 static int launch_edge_scalars(bp_context *c, const T *msgs) {
-    const int blocks = (c->nports + 255) / 256;
+    // lanes per message: 4 for messages of up to 16 entries, else 16
+    const int G = c->maxD * (c->plain ? 1 : c->maxD) <= 16 ? 4 : 16;
+    const int blocks = (int)(((long long)c->nports * G + 255) / 256);
     if (blocks > 0) {
-        if constexpr (std::is_same<T, cplx>::value)
-            hipLaunchKernelGGL(k_edge_scalars_cplx, dim3(blocks), dim3(256), 0, c->stream,
-                               c->topo(), msgs, c->d_ze);
-        else
-            hipLaunchKernelGGL(k_edge_scalars<T>, dim3(blocks), dim3(256), 0, c->stream,
-                               c->topo(), msgs, c->d_ze);
+        if constexpr (std::is_same<T, cplx>::value) {
+            if (G == 4)
+                hipLaunchKernelGGL(k_edge_scalars_cplx<4>, dim3(blocks), dim3(256), 0, c->stream,
+                                   c->topo(), msgs, c->d_ze);
+            else
+                hipLaunchKernelGGL(k_edge_scalars_cplx<16>, dim3(blocks), dim3(256), 0, c->stream,
+                                   c->topo(), msgs, c->d_ze);
+        } else {
+            if (G == 4)
+                hipLaunchKernelGGL((k_edge_scalars<T, 4>), dim3(blocks), dim3(256), 0, c->stream,
+                                   c->topo(), msgs, c->d_ze);
+            else
+                hipLaunchKernelGGL((k_edge_scalars<T, 16>), dim3(blocks), dim3(256), 0, c->stream,
+                                   c->topo(), msgs, c->d_ze);
+        }
     }
     HIPCHK(hipGetLastError());
     return BP_OK;
@@ -850,7 +929,7 @@ static int prepare_sweep(bp_context *c) {
     RETCHK(gen_set_lds_limits());
     if (path == BP_PATH_GENERIC) RETCHK(ensure_pair(c));
     RETCHK(build_buckets(c, path));
-    if ((c->vplan_ok || c->pair_ok) && c->fold_n != c->nnet) {
+    if (c->fold_n != c->nnet) {
         // folded residual accumulators, FOLD_BUFS rotating buffers (outside any graph
         // capture); every run starts by clearing them (k_reset_nets)
         const size_t nb = sizeof(unsigned long long) * FOLD_BUFS * FOLD_SLOTS * (size_t)c->nnet;
@@ -909,8 +988,19 @@ static int launch_reduce_folded(bp_context *c, int k) {
     return BP_OK;
 }
 
-// Per-network bookkeeping after a sweep: one workgroup of 1024 threads per network.
+// Per-network bookkeeping after a sweep: one workgroup of 1024 threads per network, or, for
+// networks of more than 4 x 4096 slots, many workgroups and a thread per network (261 120
+// slots: 79 us on one workgroup, against 5 + 4 us).
 static int launch_reduce(bp_context *c) {
+    int most = 0;
+    for (int n = 0; n < c->nnet; ++n) most = std::max(most, c->pbeg[n + 1] - c->pbeg[n]);
+    if (most > 4 * RED_SLOTS && c->d_fold_acc && c->fold_n == c->nnet && c->nnet < 65536) {
+        hipLaunchKernelGGL(k_reduce_parts, dim3((most + RED_SLOTS - 1) / RED_SLOTS, c->nnet),
+                           dim3(256), 0, c->stream, c->d_pbeg, c->d_res_fid, c->d_res_abs,
+                           c->d_runp, c->d_done, c->d_fold_acc);
+        HIPCHK(hipGetLastError());
+        return launch_reduce_folded(c, 0);
+    }
     hipLaunchKernelGGL(k_reduce_nets, dim3(c->nnet), dim3(1024), 0, c->stream, c->d_pbeg,
                        c->d_res_fid, c->d_res_abs, c->d_runp, c->d_done, c->d_iter, c->d_delta,
                        c->d_at);
@@ -926,11 +1016,13 @@ static const float *generic_sites32(const bp_context *c) {
 
 // One Jacobi sweep on the working dtype: reads d_msg[cur], writes d_msg[cur^1].
 // Whether the residual reduction can ride on the sweep kernel: one kernel (the D <= 8
-// four-port kernel, or the pair kernel) updates every message of every network.
+// four-port kernel, the pair kernel, or a small-bond kernel on one network) updates every
+// message of every network.
 static bool fold_possible(const bp_context *c, int path) {
     if (!c->d_fold_acc || c->fold_n != c->nnet || !c->fold_on) return false;
     if (path == BP_PATH_GENERIC) return pair_used(c) && c->pair.covers;
     if (c->dtype == BP_F64) return c->v64_kind == 3;
+    if (path == BP_PATH_VERTEX && c->vplan_ok && c->vplan.small_single) return true;
     return path == BP_PATH_VERTEX && c->vplan_ok && c->vplan.all && c->vplan.nv_k3 == 0 && c->vplan.nv16 == 0 &&
            c->vplan.ns_total() == 0 &&
            c->path != BP_PATH_GENERIC && c->vplan.nv > 0 && c->vplan.d_lead;
@@ -959,7 +1051,9 @@ static int sweep_once(bp_context *c, const NetCtl &done, bool *folded = nullptr,
         fold.prev = apply_prev ? c->d_fold_acc + (size_t)((k + FOLD_BUFS - 1) % FOLD_BUFS) * stride
                                : nullptr;
         fold.clear = c->d_fold_acc + (size_t)((k + 1) % FOLD_BUFS) * stride;
-        fold.lead = pair || c->dtype == BP_F64 ? c->pair.d_lead : c->vplan.d_lead;
+        fold.lead = pair || c->dtype == BP_F64 ? c->pair.d_lead
+                    : c->vplan.small_single    ? c->vplan.d_vs_lead
+                                               : c->vplan.d_lead;
         fold.iter = c->d_iter;
         fold.delta = c->d_delta;
         fold.at = c->d_at;
@@ -975,7 +1069,7 @@ static int sweep_once(bp_context *c, const NetCtl &done, bool *folded = nullptr,
         RETCHK(vertex16_sweep(&c->vplan, c->stream, c->topo(), src, dst, done, c->d_res_fid,
                               c->d_res_abs));
         if (vertex_s_sweep(&c->vplan, c->stream, c->topo(), src, dst, done, c->d_res_fid,
-                           c->d_res_abs) != 0)
+                           c->d_res_abs, fold) != 0)
             return set_err(BP_ERR_HIP, "small-bond sweep launch failed");
         HIPCHK(hipGetLastError());
     }
@@ -1232,8 +1326,8 @@ int bp_set_topology(bp_context *c, int nv, int ne, const int *port_off, const in
     RETCHK(dev_alloc((void **)&c->d_res_abs, sizeof(double) * np));
     RETCHK(dev_alloc((void **)&c->d_zv, sizeof(double) * c->hw() * nv));
     RETCHK(dev_alloc((void **)&c->d_ze, sizeof(double) * c->hw() * std::max(ne, 1)));
-    RETCHK(dev_alloc((void **)&c->d_lre, sizeof(double) * nnet));
-    RETCHK(dev_alloc((void **)&c->d_lim, sizeof(double) * nnet));
+    RETCHK(dev_alloc((void **)&c->d_lre, sizeof(double) * 2 * nnet));
+    RETCHK(dev_alloc((void **)&c->d_lnp, sizeof(LnPart) * LN_PARTS * (size_t)nnet));
     // per-network run state in one block (one copy back per run): delta, done, iter, at
     RETCHK(dev_alloc((void **)&c->d_delta, run_state_bytes(nnet)));
     c->d_done = (int *)(c->d_delta + nnet);
@@ -1332,14 +1426,14 @@ int bp_init_messages(bp_context *c, int kind, const double *host) {
         if (c->nports == 0) {
             // no edges: nothing to initialise
         } else if (c->is_cplx())
-            hipLaunchKernelGGL(k_init_messages<cplx>, dim3(c->nports), dim3(64), 0, c->stream,
-                               c->topo(), (cplx *)c->d_msg[0], kind);
+            hipLaunchKernelGGL(k_init_messages<cplx>, dim3((c->nports + 15) / 16), dim3(256), 0,
+                               c->stream, c->topo(), (cplx *)c->d_msg[0], kind);
         else if (c->dtype == BP_F64)
-            hipLaunchKernelGGL(k_init_messages<double>, dim3(c->nports), dim3(64), 0, c->stream,
-                               c->topo(), (double *)c->d_msg[0], kind);
+            hipLaunchKernelGGL(k_init_messages<double>, dim3((c->nports + 15) / 16), dim3(256), 0,
+                               c->stream, c->topo(), (double *)c->d_msg[0], kind);
         else
-            hipLaunchKernelGGL(k_init_messages<float>, dim3(c->nports), dim3(64), 0, c->stream,
-                               c->topo(), (float *)c->d_msg[0], kind);
+            hipLaunchKernelGGL(k_init_messages<float>, dim3((c->nports + 15) / 16), dim3(256), 0,
+                               c->stream, c->topo(), (float *)c->d_msg[0], kind);
         HIPCHK(hipGetLastError());
     } else {
         return set_err(BP_ERR_ARG, "unknown init kind %d", kind);
@@ -2304,31 +2398,68 @@ static int v64l_scalars(bp_context *c, const void *m, bool is64, bool *done) {
     return BP_OK;
 }
 
+// Vertex scalars on the pair kernel when it takes every vertex, on the automatic path.
+static int pair_zv(bp_context *c, const void *sites, const void *m, bool *done) {
+    *done = false;
+    if (c->path != BP_PATH_AUTO) return BP_OK;
+    RETCHK(ensure_pair(c));
+    if (!c->pair_ok || !c->pair.all) return BP_OK;
+    if (pair_scalars(&c->pair, c->stream, sites, m, c->d_zv) != 0)
+        return set_err(BP_ERR_HIP, "vertex scalar launch failed");
+    *done = true;
+    return BP_OK;
+}
+
+// Vertex scalars of FP32 contexts whose vertices are all on the vertex kernels, each bucket by
+// its own kernel: Z_u = <G_{u, port 0}, m_in,0> from the unnormalised message out of port 0.
+// 65 536 vertices at D = 3: 937 us on the generic kernel.
+static int vertex_zv(bp_context *c, const float *m, bool *done) {
+    *done = false;
+    const VertexPlan &p = c->vplan;
+    if (c->dtype != BP_F32 || !c->vplan_ok || !p.all || c->path == BP_PATH_GENERIC ||
+        (p.nv > 0 && !c->d_vsites))
+        return BP_OK;
+    if (p.nv16 > 0)  // the large-bond finisher leaves out padded ports, port 0 included
+        for (int u = 0; u < c->nv; ++u)
+            if (c->port_off[u] == c->port_off[u + 1]) return BP_OK;
+    if (p.nv > 0) {
+        if (vd_set_limits(p.d) != 0) return BP_OK;
+        const VdCtx vc{&c->vplan, c->stream, c->topo(), (const float *)c->d_vsites};
+        if (vd_msg(vc, m, nullptr, OP_I, 1.0, nullptr, 0, nullptr, nullptr, nullptr, nullptr,
+                   c->d_zv) != 0)
+            return set_err(BP_ERR_HIP, "vertex scalar launch failed");
+    }
+    const NetCtl off = make_ctl(c, false);
+    if (vertex_s_sweep(&c->vplan, c->stream, c->topo(), m, nullptr, off, nullptr, nullptr,
+                       SweepFold{}, c->d_zv) != 0 ||
+        vertex16_sweep(&c->vplan, c->stream, c->topo(), m, nullptr, off, nullptr, nullptr,
+                       c->d_zv) != BP_OK)
+        return set_err(BP_ERR_HIP, "vertex scalar launch failed");
+    *done = true;
+    return BP_OK;
+}
+
 static int scalars(bp_context *c) {
     bool is64 = false;
     const void *m = current_msgs(c, &is64);
     if (c->is_cplx()) {
-        RETCHK(launch_vertex_scalars<cplx>(c, (const cplx *)c->d_sites64, (const cplx *)m));
+        bool zdone = false;
+        RETCHK(pair_zv(c, c->d_sites64, m, &zdone));
+        if (!zdone)
+            RETCHK(launch_vertex_scalars<cplx>(c, (const cplx *)c->d_sites64, (const cplx *)m));
         RETCHK(launch_edge_scalars<cplx>(c, (const cplx *)m));
         return BP_OK;
     }
     // largest bond dimensions 9..16: FP64 scalars on the large-bond kernel, in every dtype
     bool done = false;
     RETCHK(v64l_scalars(c, m, is64, &done));
+    if (is64 && !done) RETCHK(pair_zv(c, c->d_sites64, m, &done));
     if (is64) {
         if (!done) RETCHK(launch_vertex_scalars<double>(c, c->d_sites64, (const double *)m));
         RETCHK(launch_edge_scalars<double>(c, (const double *)m));
         return BP_OK;
     }
-    if (!done && vertex_adjoint_ok(c, false) && vd_set_limits(c->vplan.d) == 0) {
-        // FP32 networks on the D <= 8 vertex kernels: the message-form dual kernel without
-        // overrides gives Z_u = <G_{u, port 0}, m_in,0> from the unnormalised port-0 result
-        const VdCtx vc{&c->vplan, c->stream, c->topo(), (const float *)c->d_vsites};
-        if (vd_msg(vc, (const float *)m, nullptr, OP_I, 1.0, nullptr, 0, nullptr, nullptr,
-                   nullptr, nullptr, c->d_zv) != 0)
-            return set_err(BP_ERR_HIP, "vertex scalar launch failed");
-        done = true;
-    }
+    if (!done) RETCHK(vertex_zv(c, (const float *)m, &done));
     if (!done) RETCHK(launch_vertex_scalars<float>(c, (const float *)c->d_sites, (const float *)m));
     RETCHK(launch_edge_scalars<float>(c, (const float *)m));
     return BP_OK;
@@ -2362,20 +2493,39 @@ int bp_lognorm(bp_context *c, double *out_re, double *out_im) {
     if (!out_re) return set_err(BP_ERR_ARG, "NULL argument");
     HIPCHK(hipSetDevice(c->device));
     RETCHK(scalars(c));
-    if (c->is_cplx())
-        hipLaunchKernelGGL(k_lognorm_nets_cplx, dim3(c->nnet), dim3(BP_BLOCK), 0, c->stream,
-                           c->topo(), c->d_vbeg, c->d_pbeg, c->d_zv, c->d_ze, c->d_lre, c->d_lim);
-    else
-        hipLaunchKernelGGL(k_lognorm_nets, dim3(c->nnet), dim3(BP_BLOCK), 0, c->stream,
-                           c->topo(), c->d_vbeg, c->d_pbeg, c->d_zv, c->d_ze, c->d_lre,
-                           c->d_lim);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(out_re, c->d_lre, sizeof(double) * c->nnet, hipMemcpyDeviceToHost,
-                          c->stream));
-    if (out_im)
-        HIPCHK(hipMemcpyAsync(out_im, c->d_lim, sizeof(double) * c->nnet, hipMemcpyDeviceToHost,
-                              c->stream));
+    int most = 0;
+    for (int n = 0; n < c->nnet; ++n)
+        most = std::max(most, c->vbeg[n + 1] - c->vbeg[n] + c->pbeg[n + 1] - c->pbeg[n]);
+    const int np = std::max(1, std::min(LN_PARTS, most / LN_TERMS));
+    double *lim = c->d_lre + c->nnet;
+    for (int n0 = 0; n0 < c->nnet; n0 += 65535) {  // networks sit on the grid's second axis
+        const dim3 grid(np, std::min(c->nnet - n0, 65535));
+        LnPart *parts = c->d_lnp + (size_t)n0 * LN_PARTS;
+        if (c->is_cplx())
+            hipLaunchKernelGGL(k_lognorm_parts<true>, grid, dim3(256), 0, c->stream, c->topo(),
+                               c->d_vbeg + n0, c->d_pbeg + n0, c->d_zv, c->d_ze, parts,
+                               c->d_lre + n0, lim + n0);
+        else
+            hipLaunchKernelGGL(k_lognorm_parts<false>, grid, dim3(256), 0, c->stream, c->topo(),
+                               c->d_vbeg + n0, c->d_pbeg + n0, c->d_zv, c->d_ze, parts,
+                               c->d_lre + n0, lim + n0);
+        HIPCHK(hipGetLastError());
+    }
+    if (np > 1) {
+        if (c->is_cplx())
+            hipLaunchKernelGGL(k_lognorm_join<true>, dim3(c->nnet), dim3(64), 0, c->stream,
+                               c->d_lnp, np, c->d_lre, lim);
+        else
+            hipLaunchKernelGGL(k_lognorm_join<false>, dim3(c->nnet), dim3(64), 0, c->stream,
+                               c->d_lnp, np, c->d_lre, lim);
+        HIPCHK(hipGetLastError());
+    }
+    std::vector<double> out(2 * (size_t)c->nnet);
+    HIPCHK(hipMemcpyAsync(out.data(), c->d_lre, sizeof(double) * out.size(),
+                          hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    std::memcpy(out_re, out.data(), sizeof(double) * c->nnet);
+    if (out_im) std::memcpy(out_im, out.data() + c->nnet, sizeof(double) * c->nnet);
     return BP_OK;
 }
 

@@ -124,6 +124,19 @@ __device__ __forceinline__ double row_partner(double v) {
     return __hiloint2double(hi, lo);
 }
 
+// sum over an aligned group of G = 4 or 16 lanes (every lane gets it)
+template <int G>
+__device__ __forceinline__ double group_sum(double v) {
+    static_assert(G == 4 || G == 16, "lanes per group");
+    v += row_partner<1>(v);
+    v += row_partner<2>(v);
+    if constexpr (G == 16) {
+        v += row_partner<4>(v);
+        v += row_partner<8>(v);
+    }
+    return v;
+}
+
 // Both members of a pair of 16-lane rows (rows 0 and 1, rows 2 and 3) or of the two 32-lane
 // halves, through v_permlane16_swap / v_permlane32_swap (VALU): with both operands v, the
 // swap returns v of the pair's first member in [0] and of its second in [1], on every lane.

@@ -203,20 +203,29 @@ __global__ __launch_bounds__(BP_BLOCK) void k_vertex_scalar_cplx(
 }
 
 // Z_e = sum_i m_uv[i] m_vu[i] (both shared names contracted, no conjugate,
-// messagecache.jl:153-157), one thread per port pair; interleaved complex output.
-__global__ void k_edge_scalars_cplx(DevTopo tp, const cplx *__restrict__ msgs,
-                                    double *__restrict__ ze) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= tp.nports) return;
-    const int r = tp.port_rev[q];
-    if (q > r) return;
-    const long long a = tp.msg_off[q], b = tp.msg_off[r];
-    const int len = (int)(tp.msg_off[q + 1] - a);
+// messagecache.jl:153-157), G lanes per port pair; interleaved complex output.
+template <int G>
+__global__ __launch_bounds__(256) void k_edge_scalars_cplx(DevTopo tp,
+                                                           const cplx *__restrict__ msgs,
+                                                           double *__restrict__ ze) {
+    const int q = (blockIdx.x * 256 + threadIdx.x) / G;
     cplx s(0.0);
-    for (int i = 0; i < len; ++i) s += msgs[a + i] * msgs[b + i];
-    const int e = tp.port_edge[q];
-    ze[2 * e] = s.re;
-    ze[2 * e + 1] = s.im;
+    int r = 0;
+    if (q < tp.nports) {
+        r = tp.port_rev[q];
+        if (q <= r) {
+            const long long a = tp.msg_off[q], b = tp.msg_off[r];
+            const int len = (int)(tp.msg_off[q + 1] - a);
+            for (int i = threadIdx.x % G; i < len; i += G) s += msgs[a + i] * msgs[b + i];
+        }
+    }
+    s.re = group_sum<G>(s.re);
+    s.im = group_sum<G>(s.im);
+    if (threadIdx.x % G == 0 && q < tp.nports && q <= r) {
+        const int e = tp.port_edge[q];
+        ze[2 * e] = s.re;
+        ze[2 * e + 1] = s.im;
+    }
 }
 
 // Per-slot distance between two complex message buffers (one wave per slot):
@@ -246,59 +255,5 @@ __global__ void k_diff_slots_cplx(DevTopo tp, const cplx *a, const cplx *b, doub
     if (threadIdx.x == 0) {
         res_fid[q] = 1.0 - (dr * dr + di * di) / (aa * bb);
         res_abs[q] = mx;
-    }
-}
-
-// BP log-norm per network with complex terms (one workgroup per network):
-// sum log Z_v - sum log Z_e with the principal logarithm log|z| + i arg z of every term,
-// real parts Neumaier-compensated; any Z_e = 0 gives -Inf, a Z_v = 0 gives a real part of
-// -Inf (messagecache.jl:185-201).
-__global__ __launch_bounds__(BP_BLOCK) void k_lognorm_nets_cplx(DevTopo tp, const int *vbeg,
-                                                                 const int *pbeg,
-                                                                 const double *zv,
-                                                                 const double *ze,
-                                                                 double *out_re,
-                                                                 double *out_im) {
-    __shared__ double ss[BP_BLOCK], cc[BP_BLOCK], ii[BP_BLOCK];
-    __shared__ int flag[2];
-    const int n = blockIdx.x;
-    if (threadIdx.x < 2) flag[threadIdx.x] = 0;
-    __syncthreads();
-    NeuSum acc, ang;
-    int zv0 = 0, ze0 = 0;
-    for (int u = vbeg[n] + threadIdx.x; u < vbeg[n + 1]; u += blockDim.x) {
-        const double x = zv[2 * u], y = zv[2 * u + 1];
-        ang.add(atan2(y, x));
-        if (x == 0.0 && y == 0.0) { zv0 = 1; continue; }
-        acc.add(log(hypot(x, y)));
-    }
-    for (int q = pbeg[n] + threadIdx.x; q < pbeg[n + 1]; q += blockDim.x) {
-        if (q > tp.port_rev[q]) continue;
-        const int e = tp.port_edge[q];
-        const double x = ze[2 * e], y = ze[2 * e + 1];
-        if (x == 0.0 && y == 0.0) { ze0 = 1; continue; }
-        ang.add(-atan2(y, x));
-        acc.add(-log(hypot(x, y)));
-    }
-    ss[threadIdx.x] = acc.s;
-    cc[threadIdx.x] = acc.c;
-    ii[threadIdx.x] = ang.s + ang.c;
-    atomicOr(&flag[0], zv0);
-    atomicOr(&flag[1], ze0);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        NeuSum t, a;
-        double c = 0.0;
-        for (int i = 0; i < (int)blockDim.x; ++i) {
-            t.add(ss[i]);
-            c += cc[i];
-            a.add(ii[i]);
-        }
-        double re = t.s + (t.c + c);
-        double im = a.s + a.c;
-        if (flag[1]) { re = -INFINITY; im = 0.0; }
-        else if (flag[0]) re = -INFINITY;
-        out_re[n] = re;
-        out_im[n] = im;
     }
 }

@@ -322,16 +322,23 @@ __global__ __launch_bounds__(BP_BLOCK) void k_vertex_scalar_generic(
     }
 }
 
-// Z_e = <m_uv, m_vu> for every undirected edge (one thread per port pair).
-template <typename T>
-__global__ void k_edge_scalars(DevTopo tp, const T *__restrict__ msgs, double *__restrict__ ze) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= tp.nports) return;
-    const int r = tp.port_rev[q];
-    if (q > r) return;
-    const long long a = tp.msg_off[q], b = tp.msg_off[r];
-    const int len = (int)(tp.msg_off[q + 1] - a);
+// Z_e = <m_uv, m_vu> for every undirected edge, G lanes per port pair (G = 4 or 16; a thread
+// per pair read 16 x 16 messages one cache line an entry: 50 us for 1 104 edges).
+template <typename T, int G>
+__global__ __launch_bounds__(256) void k_edge_scalars(DevTopo tp, const T *__restrict__ msgs,
+                                                      double *__restrict__ ze) {
+    const int q = (blockIdx.x * 256 + threadIdx.x) / G;
     double s = 0.0;
-    for (int i = 0; i < len; ++i) s += (double)msgs[a + i] * (double)msgs[b + i];
-    ze[tp.port_edge[q]] = s;
+    int r = 0;
+    if (q < tp.nports) {
+        r = tp.port_rev[q];
+        if (q <= r) {
+            const long long a = tp.msg_off[q], b = tp.msg_off[r];
+            const int len = (int)(tp.msg_off[q + 1] - a);
+            for (int i = threadIdx.x % G; i < len; i += G)
+                s += (double)msgs[a + i] * (double)msgs[b + i];
+        }
+    }
+    s = group_sum<G>(s);
+    if (threadIdx.x % G == 0 && q < tp.nports && q <= r) ze[tp.port_edge[q]] = s;
 }

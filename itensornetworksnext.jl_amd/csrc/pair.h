@@ -34,7 +34,8 @@ struct PairPlan {
     std::vector<int> rest;           // message slots of the other vertices
     PairRec *d_recs = nullptr;
     int *d_lead = nullptr;           // per network: its first record
-    bool covers = false;             // it takes every vertex of every network
+    bool covers = false;             // it takes every message of every network
+    bool all = false;                // and every vertex (no isolated ones)
     int nt = 0;                      // 16-wide tiles of the largest pair dimension
     int chunk = 0, split = 0;        // slices staged in LDS at once; waves sharing a tile's slices
     int waves = 0;
@@ -56,3 +57,6 @@ double pair_mfma_per_slice(const PairPlan *p);
 int pair_sweep(const PairPlan *p, hipStream_t st, const void *sites, const void *src, void *dst,
                const NetCtl &ctl, double *res_fid, double *res_abs, const SweepFold &fold,
                const int *items = nullptr, int n = 0);
+// Vertex scalars of every record at the messages `msgs`: zv[vertex] (complex: interleaved).
+int pair_scalars(const PairPlan *p, hipStream_t st, const void *sites, const void *msgs,
+                 double *zv);

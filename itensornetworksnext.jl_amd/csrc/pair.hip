@@ -78,7 +78,7 @@ __global__ __launch_bounds__(64 * PAIR_MAXWAVES) void k_pair(
     const typename PairTy<TY>::E *__restrict__ sites, const typename PairTy<TY>::E *mold,
     typename PairTy<TY>::E *mnew, NetCtl ctl, double *__restrict__ res_fid,
     double *__restrict__ res_abs, SweepFold fold, int chunk, int split, int slice_elems,
-    int env_elems) {
+    int env_elems, double *__restrict__ zv) {
     using P = PairTy<TY>;
     using E = typename P::E;
     using V = typename P::V;
@@ -93,7 +93,8 @@ __global__ __launch_bounds__(64 * PAIR_MAXWAVES) void k_pair(
 
     const int item = blockIdx.x;
     const int ri = items ? items[item] >> 2 : item;
-    const int mask = items ? 1 << (items[item] & 3) : 15;
+    // positions to update; the vertex scalar comes from position 0's unnormalised message
+    const int mask = zv ? 1 : items ? 1 << (items[item] & 3) : 15;
     const PairRec &rec = recs[ri];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nthr = blockDim.x;
     const int W = nthr >> 6;
@@ -341,6 +342,21 @@ __global__ __launch_bounds__(64 * PAIR_MAXWAVES) void k_pair(
             if constexpr (CX) xi += __shfl_down(xi, k * DD, 64);
         }
         const bool real = lane < DD;
+        if (zv) {
+            if constexpr (CX) {
+                const E mr = ml[lane & 63], mi = ml[64 + (lane & 63)];
+                const double zr = wave_sum_v(real ? x * mr - xi * mi : 0.0);
+                const double zi = wave_sum_v(real ? x * mi + xi * mr : 0.0);
+                if (lane == 0) {
+                    zv[2 * rec.vertex] = zr;
+                    zv[2 * rec.vertex + 1] = zi;
+                }
+            } else {
+                const double z = wave_sum_v(real ? (double)x * (double)ml[lane] : 0.0);
+                if (lane == 0) zv[rec.vertex] = z;
+            }
+            continue;
+        }
         const long long mo = rec.out[p] + lane;
         double fid, mx;
         if constexpr (CX) {
@@ -459,6 +475,7 @@ int pair_plan_build(PairPlan *p, int dtype, int plain, int nv, int nnet, const i
     }
     if (p->recs.empty()) return 4;
     p->covers = p->rest.empty();
+    p->all = (int)p->recs.size() == nv;
     for (int n = 0; n < nnet; ++n) p->covers = p->covers && lead[n] >= 0;
     p->nt = (maxn + 15) / 16;
     // one tile column per half leaves two waves: share the slices between two more
@@ -514,14 +531,14 @@ double pair_mfma_per_slice(const PairPlan *p) {
 template <int TY>
 static int pair_go(const PairPlan *p, hipStream_t st, const void *sites, const void *src,
                    void *dst, const NetCtl &ctl, double *rf, double *ra, const SweepFold &fold,
-                   const int *items, int n) {
+                   const int *items, int n, double *zv) {
     using E = typename PairTy<TY>::E;
     const int blocks = items ? n : (int)p->recs.size();
     if (blocks == 0) return 0;
 #define PAIR_GO(NT)                                                                               \
     hipLaunchKernelGGL((k_pair<TY, NT>), dim3(blocks), dim3(64 * p->waves), p->lds_bytes, st,      \
                        p->d_recs, items, (const E *)sites, (const E *)src, (E *)dst, ctl, rf, ra, \
-                       fold, p->chunk, p->split, p->slice_elems, p->env_elems)
+                       fold, p->chunk, p->split, p->slice_elems, p->env_elems, zv)
     switch (p->nt) {
         case 1: PAIR_GO(1); break;
         case 2: PAIR_GO(2); break;
@@ -532,12 +549,25 @@ static int pair_go(const PairPlan *p, hipStream_t st, const void *sites, const v
     return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
+static int pair_any(const PairPlan *p, hipStream_t st, const void *sites, const void *src,
+                    void *dst, const NetCtl &ctl, double *rf, double *ra, const SweepFold &fold,
+                    const int *items, int n, double *zv) {
+    if (p->dtype == PAIR_F64)
+        return pair_go<PAIR_F64>(p, st, sites, src, dst, ctl, rf, ra, fold, items, n, zv);
+    if (p->dtype == PAIR_C128)
+        return pair_go<PAIR_C128>(p, st, sites, src, dst, ctl, rf, ra, fold, items, n, zv);
+    return pair_go<PAIR_F32>(p, st, sites, src, dst, ctl, rf, ra, fold, items, n, zv);
+}
+
 int pair_sweep(const PairPlan *p, hipStream_t st, const void *sites, const void *src, void *dst,
                const NetCtl &ctl, double *res_fid, double *res_abs, const SweepFold &fold,
                const int *items, int n) {
-    if (p->dtype == PAIR_F64)
-        return pair_go<PAIR_F64>(p, st, sites, src, dst, ctl, res_fid, res_abs, fold, items, n);
-    if (p->dtype == PAIR_C128)
-        return pair_go<PAIR_C128>(p, st, sites, src, dst, ctl, res_fid, res_abs, fold, items, n);
-    return pair_go<PAIR_F32>(p, st, sites, src, dst, ctl, res_fid, res_abs, fold, items, n);
+    return pair_any(p, st, sites, src, dst, ctl, res_fid, res_abs, fold, items, n, nullptr);
+}
+
+int pair_scalars(const PairPlan *p, hipStream_t st, const void *sites, const void *msgs,
+                 double *zv) {
+    NetCtl off{};
+    return pair_any(p, st, sites, msgs, nullptr, off, nullptr, nullptr, SweepFold{}, nullptr, 0,
+                    zv);
 }

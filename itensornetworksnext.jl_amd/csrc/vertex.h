@@ -97,6 +97,9 @@ struct VertexPlan {
     int *d_vs_out[3] = {};   // per item and port: outgoing slot (-1: padded port)
     int *d_vs_dim[3] = {};   // per item: the four ports' bond dimensions, one byte each
     int *d_vs_net[3] = {}, *d_vs_list[3] = {};
+    int *d_vs_lead = nullptr;  // one zero: the lead group of a run on one network (SweepFold)
+    // one network, every vertex of it in one small-bond bucket
+    bool small_single = false;
     float *d_vs_sites[3] = {};
     int ns_total() const { return ns[0] + ns[1] + ns[2]; }
 };
@@ -126,6 +129,9 @@ static void vertex_plan_release(VertexPlan *p) {
     p->nv16 = 0;
     if (p->d_vsites_y) (void)hipFree(p->d_vsites_y);
     p->d_vsites_y = nullptr;
+    if (p->d_vs_lead) (void)hipFree(p->d_vs_lead);
+    p->d_vs_lead = nullptr;
+    p->small_single = false;
     for (int k = 0; k < 3; ++k) {
         void *sm[7] = {p->d_vs_ino[k], p->d_vs_outo[k], p->d_vs_out[k], p->d_vs_dim[k],
                        p->d_vs_net[k], p->d_vs_list[k], p->d_vs_sites[k]};
@@ -323,6 +329,9 @@ static int vertex_plan_build(VertexPlan *p, int dtype, int plain, int nv, const 
         if (!rc) rc = vx_upload(&p->d_vs_list[k], vlist_s[k]);
         p->ns[k] = n;
     }
+    p->small_single = nv > 0 && vnet[nv - 1] == 0 &&
+                      (p->ns[0] == nv || p->ns[1] == nv || p->ns[2] == nv);
+    if (!rc && p->small_single) rc = vx_upload(&p->d_vs_lead, std::vector<int>(1, 0));
     if (rc) {
         p->why = "allocation failed";
         vertex_plan_release(p);

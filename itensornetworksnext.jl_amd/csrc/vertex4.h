@@ -80,12 +80,26 @@ __device__ __forceinline__ void vs_mode_0(float (&X)[VsShape<DP>::RP], const flo
     }
 }
 
-template <int DP>
+// ZV: the vertex scalars zv[vlist[item]] at the messages mold instead of a sweep: the
+// unnormalised message out of port 0 meets the one into it (a padded port 0: e0 e0^T).
+//
+// fold: the stopping rule of a run on one network whose vertices are all in one bucket, folded
+// as in the D <= 8 kernels (work item: the wave's group).  With one 1024-thread workgroup
+// reading the residuals back after each sweep, a 256x256 D = 3 sweep took 44 + 79 us.
+__device__ __forceinline__ void vs_fold_end(const SweepFold &fold, int g, double fm) {
+    if (!fold.acc) return;
+    fm = wave_max_v(fm);
+    if ((threadIdx.x & 63) == 0)
+        atomicMax(fold.acc + (g % FOLD_SLOTS), (unsigned long long)__double_as_longlong(fm));
+}
+
+template <int DP, bool ZV>
 __global__ __launch_bounds__(64) void k_vertex_s(
     const float *__restrict__ vs_sites, const float *__restrict__ mold, float *__restrict__ mnew,
     const int *__restrict__ vs_ino, const int *__restrict__ vs_outo,
     const int *__restrict__ vs_out, const int *__restrict__ vs_dim, const int *__restrict__ vnet,
-    NetCtl ctl, double *__restrict__ res_fid, double *__restrict__ res_abs, int nitems, int d) {
+    NetCtl ctl, double *__restrict__ res_fid, double *__restrict__ res_abs, int nitems, int d,
+    SweepFold fold, const int *__restrict__ vlist, double *__restrict__ zv) {
     using Shp = VsShape<DP>;
     constexpr int R = Shp::R, RP = Shp::RP, M2 = Shp::M2;
     __shared__ float msm[16 * 4 * M2];   // [vi][port][p * DP + b], padded incoming messages
@@ -123,8 +137,9 @@ __global__ __launch_bounds__(64) void k_vertex_s(
 #pragma unroll
         for (int r = 0; r < RP; ++r) A[r] = 0.f;
     }
-    const bool live = inr && !(ctl.enabled && ctl.done[vnet[b]]);
-    const bool done2 = mine && ctl.enabled && ctl.done[net2];
+    const bool stopped = fold.acc && vx_fold_begin(ctl, fold, 0, g);
+    const bool live = inr && !(fold.acc ? stopped : ctl.enabled && ctl.done[vnet[b]]);
+    const bool done2 = mine && (fold.acc ? stopped : ctl.enabled && ctl.done[net2]);
     // the incoming message of (vi2, port), zero-padded to DP x DP (padded port: e0 e0^T)
     {
         float *dst = msm + (vi2 * 4 + port) * M2;
@@ -163,6 +178,7 @@ __global__ __launch_bounds__(64) void k_vertex_s(
         float E[RP], o[M2];
 
         // ---- phase A: E = A x0 m0 x1 m1
+        if constexpr (!ZV) {
 #pragma unroll
         for (int r = 0; r < RP; ++r) E[r] = A[r];
         vs_mode_0<DP>(E, c0);
@@ -215,6 +231,7 @@ __global__ __launch_bounds__(64) void k_vertex_s(
                         o[a * DP + ap] = fmaf(G[t * DP + a], A[(p1 * DP + t) * DP + ap], o[a * DP + ap]);
         }
         store(o, 3);
+        }
 
         // ---- phase B: E = A x2 m2 x3 m3
 #pragma unroll
@@ -222,6 +239,7 @@ __global__ __launch_bounds__(64) void k_vertex_s(
         vs_mode_in<DP, 2>(E, c2);
         vs_mode_in<DP, 3>(E, c3);
         // out1 = open_1(E x0 m0, A), the port-0 product fused entry by entry
+        if constexpr (!ZV) {
 #pragma unroll
         for (int e = 0; e < M2; ++e) o[e] = 0.f;
 #pragma unroll
@@ -236,6 +254,7 @@ __global__ __launch_bounds__(64) void k_vertex_s(
                 for (int ap = 0; ap < DP; ++ap) o[a * DP + ap] = fmaf(gv, A[ap * DP * DP + t], o[a * DP + ap]);
             }
         store(o, 1);
+        }
         // out0 = open_0(E x1 m1, A) on the matrix cores: with a = G (row a = lane i) and
         // b = A (column a' = lane j), register i of lane j collects out0[i][j]
         vs_mode_in<DP, 1>(E, c1);
@@ -249,41 +268,55 @@ __global__ __launch_bounds__(64) void k_vertex_s(
     }
     __syncthreads();
 
+    if constexpr (ZV) {  // one lane per vertex
+        if (!mine || port != 0) return;
+        double z = 0.0;
+#pragma unroll
+        for (int e = 0; e < M2; ++e) {
+            float v = 0.f;
+            for (int t = 0; t < d; ++t) v += part[((vi2 * d + t) * 4) * M2 + e];
+            z += (double)v * (double)msm[(vi2 * 4) * M2 + e];
+        }
+        zv[vlist[b2]] = z;
+        return;
+    }
     // ---- one lane per message: sum over slices, normalise, residuals, write
-    if (qout < 0) return;
-    if (done2) {
+    double fm = 0.0;
+    if (qout >= 0 && done2) {
         for (int e = 0; e < Dm * Dm; ++e) mnew[outo + e] = mold[outo + e];
         res_fid[qout] = 0.0;
         res_abs[qout] = 0.0;
-        return;
-    }
-    float x[M2];
-    double S = 0.0;
+    } else if (qout >= 0) {
+        float x[M2];
+        double S = 0.0;
 #pragma unroll
-    for (int e = 0; e < M2; ++e) {
-        float v = 0.f;
-        for (int s = 0; s < d; ++s) v += part[((vi2 * d + s) * 4 + port) * M2 + e];
-        x[e] = v;
-        S += (double)v;  // entries beyond the bond dimension are exactly zero
-    }
-    double dn = 0.0, nn = 0.0, oo = 0.0, mx = 0.0;
+        for (int e = 0; e < M2; ++e) {
+            float v = 0.f;
+            for (int t = 0; t < d; ++t) v += part[((vi2 * d + t) * 4 + port) * M2 + e];
+            x[e] = v;
+            S += (double)v;  // entries beyond the bond dimension are exactly zero
+        }
+        double dn = 0.0, nn = 0.0, oo = 0.0, mx = 0.0;
 #pragma unroll
-    for (int e = 0; e < M2; ++e) {
-        const int a = e / DP, ap = e % DP;
-        if (a >= Dm || ap >= Dm) continue;
-        const float xf = (float)(S != 0.0 ? (double)x[e] / S : (double)x[e]);
-        const long long o = outo + a * Dm + ap;
-        const double xo = (double)mold[o];
-        mnew[o] = xf;
-        dn += (double)xf * xo;
-        nn += (double)xf * (double)xf;
-        oo += xo * xo;
-        const double df = fabs((double)xf - xo);
-        mx = (df > mx || df != df) ? df : mx;
+        for (int e = 0; e < M2; ++e) {
+            const int a = e / DP, ap = e % DP;
+            if (a >= Dm || ap >= Dm) continue;
+            const float xf = (float)(S != 0.0 ? (double)x[e] / S : (double)x[e]);
+            const long long o = outo + a * Dm + ap;
+            const double xo = (double)mold[o];
+            mnew[o] = xf;
+            dn += (double)xf * xo;
+            nn += (double)xf * (double)xf;
+            oo += xo * xo;
+            const double df = fabs((double)xf - xo);
+            mx = (df > mx || df != df) ? df : mx;
+        }
+        const double c = dn / sqrt(nn * oo);
+        res_fid[qout] = 1.0 - c * c;
+        res_abs[qout] = mx;
+        fm = fold_max(0.0, fold.acc && fold.rp->crit != 0 ? mx : 1.0 - c * c);
     }
-    const double c = dn / sqrt(nn * oo);
-    res_fid[qout] = 1.0 - c * c;
-    res_abs[qout] = mx;
+    vs_fold_end(fold, g, fm);
 }
 
 // ---------------------------------------------------------------- bond dimension <= 2
@@ -337,11 +370,13 @@ __device__ __forceinline__ float4 t2_load_msg(const float *m, long long off, int
     return make_float4(D == 1 ? m[off] : 0.f, 0.f, 0.f, 0.f);
 }
 
+template <bool ZV>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_vertex_t2(
     const float *__restrict__ vs_sites, const float *__restrict__ mold, float *__restrict__ mnew,
     const int *__restrict__ vs_ino, const int *__restrict__ vs_outo,
     const int *__restrict__ vs_out, const int *__restrict__ vs_dim, const int *__restrict__ vnet,
-    NetCtl ctl, double *__restrict__ res_fid, double *__restrict__ res_abs, int nitems, int d) {
+    NetCtl ctl, double *__restrict__ res_fid, double *__restrict__ res_abs, int nitems, int d,
+    SweepFold fold, const int *__restrict__ vlist, double *__restrict__ zv) {
     // 4 KiB of LDS: the incoming messages [vi * 4 + port], then, once every lane holds its
     // four, the per-slice results [lane * 4 + port], so that eight one-wave workgroups share
     // a SIMD (64 registers).
@@ -372,7 +407,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         msm[mi] = v;
     }
     wave_lds_sync();  // one wave per workgroup
-    const bool live = inr && !(ctl.enabled && ctl.done[vnet[b]]);
+    const bool stopped = fold.acc && vx_fold_begin(ctl, fold, 0, g);
+    const bool live = inr && !(fold.acc ? stopped : ctl.enabled && ctl.done[vnet[b]]);
     float m[4][4];  // vi * 4 + j < 256 for every lane
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -390,6 +426,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
     if (live) {
         float E[16], G[16], o[4];
         // phase A: E = A x0 m0 x1 m1; out2 = open_2(E x3 m3, A), out3 = open_3(E x2 m2, A)
+        if constexpr (!ZV) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) E[r] = A[r];
         t2_mode<0>(E, m[0]);
@@ -402,6 +439,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         t2_mode<2>(E, m[2]);
         t2_open<3>(E, A, o);
         put(3, o);
+        }
         // phase B: E = A x2 m2 x3 m3; out0 = open_0(E x1 m1, A), out1 = open_1(E x0 m0, A)
 #pragma unroll
         for (int r = 0; r < 16; ++r) E[r] = A[r];
@@ -411,17 +449,36 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         for (int r = 0; r < 16; ++r) G[r] = E[r];
         t2_mode<1>(G, m[1]);
         t2_open<0>(G, A, o);
+        if constexpr (ZV) {  // this slice's share of the vertex scalar
+            o[0] = o[0] * m[0][0];
+            o[1] = o[1] * m[0][1];
+            o[2] = o[2] * m[0][2];
+            o[3] = o[3] * m[0][3];
+        }
         put(0, o);
-        t2_mode<0>(E, m[0]);
-        t2_open<1>(E, A, o);
-        put(1, o);
+        if constexpr (!ZV) {
+            t2_mode<0>(E, m[0]);
+            t2_open<1>(E, A, o);
+            put(1, o);
+        }
     } else {
         const float z[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < 4; ++j) put(j, z);
     }
     wave_lds_sync();
+    if constexpr (ZV) {
+        if (!inr || s != 0) return;
+        double z = 0.0;
+        for (int t = 0; t < d; ++t) {
+            const float4 pv = part[(vi * d + t) * 4];
+            z += ((double)pv.x + (double)pv.y) + ((double)pv.z + (double)pv.w);
+        }
+        zv[vlist[b]] = z;
+        return;
+    }
     // one lane per outgoing message: sum over the vertex's slices, normalise, residuals
+    double fm = 0.0;
     for (int mi = lane; mi < nm; mi += 64) {
         const int v2 = mi / 4, j = mi & 3, bb = g * W2 + v2;
         if (bb >= nitems) continue;
@@ -431,7 +488,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         const long long mo = vs_outo[4 * bb + j];
         const float4 xo4 = t2_load_msg(mold, mo, D);
         const float xo[4] = {xo4.x, xo4.y, xo4.z, xo4.w};
-        if (ctl.enabled && ctl.done[vnet[bb]]) {
+        if (fold.acc ? stopped : ctl.enabled && ctl.done[vnet[bb]]) {
             for (int e = 0; e < D * D; ++e) mnew[mo + e] = xo[e];
             res_fid[qout] = 0.0;
             res_abs[qout] = 0.0;
@@ -471,7 +528,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         const double c = dn / sqrt(nn * oo);
         res_fid[qout] = 1.0 - c * c;
         res_abs[qout] = mx;
+        fm = fold_max(fm, fold.acc && fold.rp->crit != 0 ? mx : 1.0 - c * c);
     }
+    vs_fold_end(fold, g, fm);
 }
 
 // Sites of the bond-dimension <= 2 bucket in the lane-per-slice layout.
@@ -576,23 +635,27 @@ static int vertex_s_upload_sites(VertexPlan *p, hipStream_t st, const double *d_
     return 0;
 }
 
+// The small-bond buckets' part of a sweep (with zv, the vertex scalars at the messages src
+// instead; nothing else is written).
 static int vertex_s_sweep(const VertexPlan *p, hipStream_t st, DevTopo tp, const void *src,
-                          void *dst, const NetCtl &ctl, double *res_fid, double *res_abs) {
+                          void *dst, const NetCtl &ctl, double *res_fid, double *res_abs,
+                          const SweepFold &fold = SweepFold{}, double *zv = nullptr) {
     for (int k = 0; k < 3; ++k) {
         if (p->ns[k] == 0) continue;
         const int ng = vertex_s_groups(p, k);
-#define VS_GO(DPV)                                                                               \
-    hipLaunchKernelGGL((k_vertex_s<DPV>), dim3(ng), dim3(64), 0, st, p->d_vs_sites[k],             \
+#define VS_GO(...)                                                                               \
+    hipLaunchKernelGGL((__VA_ARGS__), dim3(ng), dim3(64), 0, st, p->d_vs_sites[k],                 \
                        (const float *)src, (float *)dst, p->d_vs_ino[k], p->d_vs_outo[k],        \
                        p->d_vs_out[k], p->d_vs_dim[k], p->d_vs_net[k], ctl, res_fid, res_abs,    \
-                       p->ns[k], p->d)
-        if (k == 0)
-            hipLaunchKernelGGL(k_vertex_t2, dim3(ng), dim3(64), 0, st, p->d_vs_sites[k],
-                               (const float *)src, (float *)dst, p->d_vs_ino[k], p->d_vs_outo[k],
-                               p->d_vs_out[k], p->d_vs_dim[k], p->d_vs_net[k], ctl, res_fid,
-                               res_abs, p->ns[k], p->d);
-        else if (k == 1) VS_GO(3);
-        else VS_GO(4);
+                       p->ns[k], p->d, fold, p->d_vs_list[k], zv)
+        switch (2 * k + (zv ? 1 : 0)) {
+            case 0: VS_GO(k_vertex_t2<false>); break;
+            case 1: VS_GO(k_vertex_t2<true>); break;
+            case 2: VS_GO(k_vertex_s<3, false>); break;
+            case 3: VS_GO(k_vertex_s<3, true>); break;
+            case 4: VS_GO(k_vertex_s<4, false>); break;
+            default: VS_GO(k_vertex_s<4, true>); break;
+        }
 #undef VS_GO
         if (hipGetLastError() != hipSuccess) return 2;
     }
