@@ -2728,6 +2728,13 @@ static int local_impl(bp_context *c, const double *ops_v, const double *ops_firs
     HIPCHK(hipSetDevice(c->device));
     bool is64 = false;
     const void *m = current_msgs(c, &is64);
+    if (vertex_adjoint_ok(c, is64)) {
+        const VdCtx vc{&c->vplan, c->stream, c->topo(), (const float *)c->d_vsites};
+        const int rv = vadj_local(&c->adj, vc, c->ne, (const float *)m, c->nsite, c->nmsg, ops_v,
+                                  ops_first, ops_second, ld, energy, go, adj_tol, adj_maxiter,
+                                  out_iters, out_res);
+        return rv == BP_OK ? BP_OK : set_err(rv, "local energy/gradient failed (status %d)", rv);
+    }
     const int rc = adjoint_local(&c->adj, c->stream, c->topo(), c->ne, c->max_site, c->max_mats,
                                  c->maxD, is64 ? BP_F64 : c->dtype,
                                  is64 ? (const void *)c->d_sites64 : (const void *)c->d_sites, m,
