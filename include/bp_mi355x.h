@@ -267,6 +267,9 @@ int bp_local_energy_device(bp_context *ctx, const double *ops_v, const double *o
  *   "fold_bookkeeping" 1 (default): when one D <= 8 vertex launch covers every network, the
  *                      sweep kernels also do the per-network convergence bookkeeping;
  *                      0: a separate bookkeeping kernel after every sweep (same results);
+ *   "pair_run"         longest wait in us (default 250000) inside the launches that run many
+ *                      sweeps of a small FP64 or complex network at once, after which the run
+ *                      is repeated launch by launch; 0: launch by launch (same messages);
  *   "normalize"        1 (default): every update divides the new message by its sum when
  *                      the sum is nonzero; 0: messages are kept unnormalised, as
  *                      SimpleMessageUpdate(; normalize = false) (beliefpropagation.jl:237-253);

@@ -117,12 +117,12 @@ __global__ void k_round_bf16(const double *in, float *out, long long n) {
 // run's stopping parameters (passed by value, so no host copy precedes the sweeps).
 __global__ void k_reset_nets(int nnet, int *done, int *iter, double *delta, int *at,
                              unsigned long long *fold_acc, int fold_n, RunParams *rp,
-                             RunParams params) {
+                             RunParams params, int iter0) {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n == 0 && rp) *rp = params;
     if (n >= nnet) return;
     done[n] = 0;
-    iter[n] = 0;
+    iter[n] = iter0;
     delta[n] = INFINITY;
     at[n] = -1;
     if (fold_acc && n < fold_n)  // every rotating buffer of the folded bookkeeping
@@ -410,6 +410,7 @@ struct bp_context {
     // contexts, the FP64 polish of the others); built on first use for the current topology
     PairPlan pair;
     bool pair_tried = false, pair_ok = false;
+    int run_wait_us = 250000;   // option "pair_run": longest wait inside a many-sweep launch, 0: none
 
     // cached sweep graphs (16 sweeps + bookkeeping), one per starting buffer parity; valid
     // while graph_epoch equals the process-wide plan epoch (which moves whenever a captured
@@ -1579,6 +1580,11 @@ int bp_set_option(bp_context *c, const char *name, int value) {
         if (c->have_topo) RETCHK(rebuild_vertex_plan(c));
         return BP_OK;
     }
+    if (strcmp(name, "pair_run") == 0) {
+        if (value < 0) return set_err(BP_ERR_ARG, "pair_run is a wait in us, or 0");
+        c->run_wait_us = value;
+        return BP_OK;
+    }
     if (strcmp(name, "small_bond") == 0) {
         if (value != 0 && value != 1) return set_err(BP_ERR_ARG, "small_bond is 0 or 1");
         c->vx_small = value;
@@ -1596,6 +1602,7 @@ int bp_get_option(bp_context *c, const char *name, int *value) {
     if (strcmp(name, "fold_bookkeeping") == 0) { *value = c->fold_on; return BP_OK; }
     if (strcmp(name, "normalize") == 0) { *value = c->normalize; return BP_OK; }
     if (strcmp(name, "small_bond") == 0) { *value = c->vx_small; return BP_OK; }
+    if (strcmp(name, "pair_run") == 0) { *value = c->run_wait_us; return BP_OK; }
     return set_err(BP_ERR_ARG, "unknown option %s", name);
 }
 
@@ -1633,9 +1640,6 @@ int bp_sweep(bp_context *c) {
     return BP_OK;
 }
 
-// Sweeps per captured chunk of bp_run (between host checks of the done flags with a
-// tolerance); a multiple of FOLD_BUFS, so every chunk starts on accumulator residue 0.
-static constexpr int RUN_CHUNK = 16;
 static_assert(RUN_CHUNK % FOLD_BUFS == 0, "a captured sweep chunk must span whole accumulator cycles");
 
 // Capture and instantiate n sweeps (each with its bookkeeping) starting at the current
@@ -1702,6 +1706,57 @@ int bp_prepare_run(bp_context *c, int maxiter) {
     return BP_OK;
 }
 
+}  // extern "C"
+
+// The run state (delta, done, iter, at: one block) comes back through a pinned buffer.
+static int ensure_h_state(bp_context *c) {
+    const size_t sbytes = run_state_bytes(c->nnet);
+    if (c->h_state_bytes >= sbytes) return BP_OK;
+    if (c->h_state) (void)hipHostFree(c->h_state);
+    c->h_state = nullptr;
+    c->h_state_bytes = 0;
+    HIPCHK(hipHostMalloc((void **)&c->h_state, sbytes, hipHostMallocDefault));
+    c->h_state_bytes = sbytes;
+    return BP_OK;
+}
+
+// A run on the pair kernel's many-sweep launches (pair.hip), when the plan takes the network
+// and no other run of this process uses them on the device.  *over: it ran to its end, the
+// state is in h_state; else it goes on launch by launch after *launched sweeps.
+//
+// us a call, launch by launch / here: see pair.hip.  A network takes it at any size that is
+// resident as a whole: where its sweeps are not latency, they keep the slices in LDS.
+static int pair_run_chunks(bp_context *c, bool sequential, const RunParams &rp, int *launched,
+                           bool *over) {
+    static std::mutex busy[64];
+    *over = false;
+    if (c->run_wait_us == 0 || !pair_run_ready(&c->pair, c->nnet, c->nmsg, c->nports)) return BP_OK;
+    std::unique_lock<std::mutex> lock(busy[(unsigned)c->device % 64], std::try_to_lock);
+    if (!lock.owns_lock()) return BP_OK;
+    RETCHK(ensure_h_state(c));
+    while (!*over) {
+        const int n = std::min(PAIR_RUN_SWEEPS, rp.maxiter - *launched);
+        if (pair_run(&c->pair, c->stream, sequential, c->d_sites, c->d_msg[c->cur],
+                     c->d_msg[c->cur ^ 1], c->d_done, c->d_iter, c->d_at, c->d_delta,
+                     c->d_res_fid, c->d_res_abs, rp, *launched, n, c->run_wait_us) != 0)
+            return set_err(BP_ERR_HIP, "pair run launch failed");
+        HIPCHK(hipEventRecord(c->ev1, c->stream));
+        HIPCHK(hipMemcpyAsync(c->h_state, c->d_delta, run_state_bytes(1), hipMemcpyDeviceToHost,
+                              c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        const int done = *(const int *)(c->h_state + sizeof(double));
+        if (done & PAIR_RUN_BAILED) {
+            pair_run_off(&c->pair);
+            return BP_OK;
+        }
+        c->cur ^= 1;
+        *launched += n;
+        *over = done != 0;
+    }
+    return BP_OK;
+}
+extern "C" {
+
 int bp_run(bp_context *c, int maxiter, double tol, int criterion, int use_graph, int *out_sweeps,
            double *out_delta, int *out_at) {
     RETCHK(ready(c));
@@ -1713,23 +1768,24 @@ int bp_run(bp_context *c, int maxiter, double tol, int criterion, int use_graph,
     c->fp64_active = false;
     RETCHK(prepare_sweep(c));
     const int cap = maxiter > 0 ? maxiter : 100000;  // tol-only runs are capped
-    // The run state (delta, done, iter, at: one block) comes back through a pinned buffer.
     const int nn = c->nnet;
     const size_t sbytes = run_state_bytes(nn);
-    if (c->h_state_bytes < sbytes) {
-        if (c->h_state) (void)hipHostFree(c->h_state);
-        c->h_state = nullptr;
-        c->h_state_bytes = 0;
-        HIPCHK(hipHostMalloc((void **)&c->h_state, sbytes, hipHostMallocDefault));
-        c->h_state_bytes = sbytes;
-    }
+    RETCHK(ensure_h_state(c));
     RunParams rp;
     rp.maxiter = cap;
     rp.crit = criterion;
     rp.tol = tol;
-    hipLaunchKernelGGL(k_reset_nets, dim3((c->nnet + 255) / 256), dim3(256), 0, c->stream,
+    HIPCHK(hipEventRecord(c->ev0, c->stream));
+    int launched = 0;
+    bool over = false;
+    const int path = resolve_path(c);
+    if (cap >= 4 &&
+        (path == BP_PATH_GENERIC ? pair_used(c) : path == BP_PATH_VERTEX && c->v64_kind == 3))
+        RETCHK(pair_run_chunks(c, false, rp, &launched, &over));
+    if (!over)
+        hipLaunchKernelGGL(k_reset_nets, dim3((c->nnet + 255) / 256), dim3(256), 0, c->stream,
                        c->nnet, c->d_done, c->d_iter, c->d_delta, c->d_at, c->d_fold_acc,
-                       c->fold_n, c->d_runp, rp);
+                       c->fold_n, c->d_runp, rp, launched);
     const NetCtl ctl = make_ctl(c, true);
     HIPCHK(hipGetLastError());
     // a captured chunk bakes in the folded accumulator indices k % FOLD_BUFS, so every
@@ -1740,9 +1796,7 @@ int bp_run(bp_context *c, int maxiter, double tol, int criterion, int use_graph,
     // queued at once and the state is read once at the end (no idle gaps between chunks).
     const bool check_chunks = tol >= 0.0;
     if (c->graph_epoch != g_epoch.load()) graphs_release(c);
-    HIPCHK(hipEventRecord(c->ev0, c->stream));
-    int launched = 0;
-    while (launched < cap) {
+    while (!over && launched < cap) {
         const int n = std::min(chunk, cap - launched);
         const bool tail = use_graph && n < chunk && c->gtail[c->cur] && c->gtail_n[c->cur] == n;
         if (use_graph && (n == chunk || tail)) {
@@ -2244,10 +2298,8 @@ struct SeqLevel {
     int begin, pairs, end;
 };
 
-static void seq_levels(const bp_context *c, const int *order, int n, bool pair,
-                       std::vector<int> *items, std::vector<SeqLevel> *levels) {
+static std::vector<int> seq_level_of(const bp_context *c, const int *order, int n) {
     std::vector<int> wrote(c->nports, -1), read(c->nports, -1), level(n);
-    int nl = 0;
     for (int i = 0; i < n; ++i) {
         const int q = order[i], u = c->owner[q];
         int l = std::max(wrote[q], read[q]) + 1;
@@ -2257,8 +2309,52 @@ static void seq_levels(const bp_context *c, const int *order, int n, bool pair,
             if (j != q) read[c->port_rev[j]] = std::max(read[c->port_rev[j]], l);
         wrote[q] = l;
         level[i] = l;
-        nl = std::max(nl, l + 1);
     }
+    return level;
+}
+
+// The same schedule for the pair kernel's many-sweep launches, [record][4]: a vertex's updates
+// of one level are a step, and an incoming message is read in this sweep's version when its
+// update comes earlier in the order (updates of one level agree on that).  Only for orders
+// that hold every message once.
+static bool seq_steps(const bp_context *c, const int *order, int n,
+                      const std::vector<int> &level, std::vector<int> *steps) {
+    std::vector<int> pos(c->nports, -1);
+    for (int i = 0; i < n; ++i) {
+        if (pos[order[i]] >= 0) return false;
+        pos[order[i]] = i;
+    }
+    if (n != c->nports) return false;
+    steps->assign(4 * c->pair.recs.size(), 0);
+    for (size_t r = 0; r < c->pair.recs.size(); ++r) {
+        const PairRec &rec = c->pair.recs[r];
+        int by[4], k = 0;
+        for (int t = 0; t < 4; ++t)
+            if (rec.slot[t] >= 0) by[k++] = t;
+        std::sort(by, by + k, [&](int x, int y) {
+            return std::make_pair(level[pos[rec.slot[x]]], pos[rec.slot[x]]) <
+                   std::make_pair(level[pos[rec.slot[y]]], pos[rec.slot[y]]);
+        });
+        int at = -1, last = -1;
+        for (int i = 0; i < k; ++i) {
+            const int q = rec.slot[by[i]];
+            if (at < 0 || level[pos[q]] != last) ++at;
+            last = level[pos[q]];
+            int &step = (*steps)[4 * r + at];
+            step |= 1 << by[i];
+            for (int t = 0; t < 4; ++t)
+                if (t != by[i] && rec.slot[t] >= 0 && pos[c->port_rev[rec.slot[t]]] < pos[q])
+                    step |= 16 << t;
+        }
+    }
+    return true;
+}
+
+static void seq_levels(const bp_context *c, const int *order, int n, bool pair,
+                       const std::vector<int> &level, std::vector<int> *items,
+                       std::vector<SeqLevel> *levels) {
+    int nl = 0;
+    for (int l : level) nl = std::max(nl, l + 1);
     auto pair_item = [&](int q) {
         if (!pair) return -1;
         const int u = c->owner[q], r = c->pair.rec_of[u];
@@ -2318,17 +2414,41 @@ int bp_run_sequential(bp_context *c, const int *order, int norder, int maxiter, 
     const int cap = maxiter > 0 ? maxiter : 100000;
     const size_t es = c->elt();
     if (c->dtype == BP_F64 || c->is_cplx()) RETCHK(ensure_pair(c));
-    std::vector<int> items;
+    const std::vector<int> level = seq_level_of(c, order, norder);
+    std::vector<int> items, steps;
     std::vector<SeqLevel> levels;
-    seq_levels(c, order, norder, pair_used(c), &items, &levels);
+    int it = 0, at = -1;
+    double delta = INFINITY;
+    if (cap >= 2 && c->run_wait_us != 0 && pair_used(c) &&
+        pair_run_ready(&c->pair, c->nnet, c->nmsg, c->nports) &&
+        seq_steps(c, order, norder, level, &steps)) {
+        RunParams rp;
+        rp.maxiter = cap;
+        rp.crit = criterion == BP_CRIT_FIDELITY ? 0 : 1;
+        rp.tol = tol;
+        bool over = false;
+        HIPCHK(hipEventRecord(c->ev0, c->stream));
+        if (pair_run_steps(&c->pair, c->stream, steps) != 0)
+            return set_err(BP_ERR_HIP, "schedule copy failed");
+        RETCHK(pair_run_chunks(c, true, rp, &it, &over));
+        if (over) {
+            float ms = 0.f;
+            HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
+            c->last_ms = ms;
+            const int *st = (const int *)(c->h_state + sizeof(double));  // done, iter, at
+            if (out_sweeps) *out_sweeps = st[1];
+            if (out_delta) *out_delta = tol >= 0.0 ? *(const double *)c->h_state : INFINITY;
+            if (out_at) *out_at = st[2];
+            return BP_OK;
+        }
+    }
+    seq_levels(c, order, norder, pair_used(c), level, &items, &levels);
     void *prev = nullptr;
     int *d_items = nullptr;
     HIPCHK(hipMalloc(&prev, es * std::max<long long>(c->nmsg, 1)));
     int rc = upload(&d_items, items);
     std::vector<double> res(c->nports);
     const NetCtl off = make_ctl(c, false);
-    int it = 0, at = -1;
-    double delta = INFINITY;
     if (rc == BP_OK && hipEventRecord(c->ev0, c->stream) != hipSuccess)
         rc = set_err(BP_ERR_HIP, "event record failed");
     while (rc == BP_OK && it < cap) {

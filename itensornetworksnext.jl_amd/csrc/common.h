@@ -56,6 +56,11 @@ struct RunParams {
 // read last and sweep k + 1 folds into.
 #define FOLD_SLOTS 32  // accumulators per network (work item u folds into slot u % 32)
 #define FOLD_BUFS 4    // rotating accumulator buffers (a divisor of the captured sweep count)
+
+// Sweeps per captured chunk of bp_run (between host checks of the done flags with a
+// tolerance); a multiple of FOLD_BUFS, so every chunk starts on accumulator residue 0.
+static constexpr int RUN_CHUNK = 16;
+
 struct SweepFold {
     unsigned long long *acc;         // this sweep's: per network, FOLD_SLOTS residual bits
     const RunParams *rp;

@@ -10,6 +10,8 @@
 #define PAIR_MAXD 8        // largest bond dimension
 #define PAIR_SIDE 64       // largest pair dimension (two bonds of PAIR_MAXD)
 #define PAIR_MAXWAVES 8    // waves per workgroup
+#define PAIR_RUN_SWEEPS 256  // sweeps of one pair_run launch
+#define PAIR_RUN_BAILED 2  // bit of the network's done flag: pair_run gave up
 
 enum { PAIR_F64 = 0, PAIR_C128 = 1, PAIR_F32 = 2 };
 
@@ -41,6 +43,15 @@ struct PairPlan {
     int waves = 0;
     int slice_elems = 0, env_elems = 0;  // LDS elements per plane
     size_t lds_bytes = 0;
+
+    // many sweeps a launch (pair_run): allocated on first use for the plan's life, at most
+    // 8 versions of the messages of a network that fits the device at once
+    int run_state = 0;               // 0: not looked at, 1: ready, -1: not for this network
+    long long run_nm = 0;            // doubles of one version
+    int run_nports = 0;
+    int *d_steps[2] = {nullptr, nullptr};  // Jacobi, sequential
+    void *d_ring = nullptr, *d_ctrl = nullptr;
+    double *d_ring_res = nullptr;
 };
 
 void pair_release(PairPlan *p);
@@ -60,3 +71,18 @@ int pair_sweep(const PairPlan *p, hipStream_t st, const void *sites, const void 
 // Vertex scalars of every record at the messages `msgs`: zv[vertex] (complex: interleaved).
 int pair_scalars(const PairPlan *p, hipStream_t st, const void *sites, const void *msgs,
                  double *zv);
+
+// Many sweeps of one network in a launch, its vertices resident together: whether the plan
+// takes it (and its buffers are there).
+bool pair_run_ready(PairPlan *p, int nnet, long long nmsg, int nports);
+void pair_run_off(PairPlan *p);
+// The schedule of sequential runs, [record][4]: positions | versions << 4 (see pair.hip).
+int pair_run_steps(PairPlan *p, hipStream_t st, const std::vector<int> &steps);
+// `sweeps` sweeps from src to dst (src is left as it is), `first` already done; the network's
+// state and residuals as after a folded run.  done & PAIR_RUN_BAILED: nothing is valid, run
+// again launch by launch (a wait in the kernel took longer than wait_us).  One launch at a time per device: two that wait for each other's
+// room would both give up.
+int pair_run(const PairPlan *p, hipStream_t st, bool sequential, const void *sites,
+             const void *src, void *dst, int *done, int *iter, int *at, double *delta,
+             double *res_fid, double *res_abs, const RunParams &rp, int first, int sweeps,
+             int wait_us);
