@@ -9,7 +9,6 @@
 
 #define PAIR_MAXD 8        // largest bond dimension
 #define PAIR_SIDE 64       // largest pair dimension (two bonds of PAIR_MAXD)
-#define PAIR_MAXWAVES 8    // waves per workgroup
 #define PAIR_RUN_SWEEPS 256  // sweeps of one pair_run launch
 #define PAIR_RUN_BAILED 2  // bit of the network's done flag: pair_run gave up
 
@@ -49,6 +48,7 @@ struct PairPlan {
     int run_state = 0;               // 0: not looked at, 1: ready, -1: not for this network
     long long run_nm = 0;            // doubles of one version
     int run_nports = 0;
+    void *d_run = nullptr;                 // what the pointers below point into
     int *d_steps[2] = {nullptr, nullptr};  // Jacobi, sequential
     void *d_ring = nullptr, *d_ctrl = nullptr;
     double *d_ring_res = nullptr;

@@ -43,6 +43,7 @@ struct PairTy<PAIR_F64> {
     }
     // row of the 16x16 result in register r of lane block lk
     static __device__ __forceinline__ int row(int lk, int r) { return lk + 4 * r; }
+    static constexpr int ROW = 4;  // register r holds rows 4 r .. 4 r + 3
 };
 template <>
 struct PairTy<PAIR_C128> : PairTy<PAIR_F64> {
@@ -57,7 +58,11 @@ struct PairTy<PAIR_F32> {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
     static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
+    static constexpr int ROW = 0;  // register r holds rows of the whole tile
 };
+
+// waves of the largest workgroup with NT tile columns
+constexpr int pair_waves(int NT) { return NT == 3 ? 12 : 8; }
 
 __host__ __device__ inline int pair_pad(int n) { return (n + 15) & ~15; }
 
@@ -66,6 +71,11 @@ __host__ __device__ inline int pair_pad(int n) { return (n + 15) & ~15; }
 __host__ __device__ inline int pair_slice_elems(int n0, int n1) {
     // an odd row pitch: both the rows and the columns of a slice are read 16 at a time
     return pair_pad(n0) * (pair_pad(n1) + 1);
+}
+
+// environments have an odd row pitch too: a message is opened over rows, columns or both
+__host__ __device__ inline int pair_env_elems(int N0, int N1) {
+    return N0 * (N0 + 1) + N1 * (N1 + 1);
 }
 
 // floor(i / n) for 0 <= i < 2^22, 1 <= n
@@ -96,7 +106,7 @@ struct PairCore {
         plA = chunk * slice_elems;
         tid = threadIdx.x;
         lane = tid & 63;
-        w = tid >> 6;
+        w = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: what depends on it is, too
         nthr = blockDim.x;
         W = nthr >> 6;
         n0 = rec.n[0];
@@ -237,6 +247,7 @@ struct PairCore {
                     if (j >= nJ) break;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
+                        if (16 * I + P::ROW * r >= nh) break;  // padding
                         const int o = (16 * I + P::row(lk, r)) * sk + 16 * j * sj;
                         const E a = As[o];
                         if constexpr (CX) {
@@ -269,8 +280,8 @@ struct PairCore {
     __device__ __forceinline__ void env_store(const V (&R)[NT], const V (&Ri)[CX ? NT : 1]) {
         if (!work) return;
         const int lk = lane >> 4, li = lane & 15;
-        const int No = h ? N0 : N1;
-        E *Ro = Ml + sg * (N0 * N0 + N1 * N1) + (h ? 0 : N0 * N0);
+        const int No = (h ? N0 : N1) + 1;
+        E *Ro = Ml + sg * pair_env_elems(N0, N1) + (h ? 0 : N0 * (N0 + 1));
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             if (j >= nJ) break;
@@ -283,47 +294,72 @@ struct PairCore {
         }
     }
 
-    // ---- unnormalised message out of position p (one wave): entry `lane` of lanes below D^2
+    // ---- unnormalised message out of position p (one wave): entry `lane` of lanes below D^2.
+    // What a lane reads depends on the vertex only.
+    struct OpenAt {
+        int v, m, b;  // first environment entry, partner entry, partner row (of lanes in use)
+    };
+    __device__ __forceinline__ int open_groups(int p) const {
+        const int DD = rec.dim[p] * rec.dim[p], Dp = rec.dim[p ^ 1];
+        int G = 1;
+        while (2 * G * DD <= 64 && G < Dp) G *= 2;  // lanes per entry, lane = g * DD + entry
+        return G;
+    }
+    __device__ __forceinline__ OpenAt open_at(int p) const {
+        const int D = rec.dim[p], Dp = rec.dim[p ^ 1], DD = D * D;
+        const int sa = (p & 1) ? 1 : Dp, sb = (p & 1) ? D : 1;
+        const int N = ((p >> 1) ? N1 : N0) + 1;
+        const int g = fdiv(lane, 1.0f / (float)DD), e = lane - g * DD;
+        const int a = fdiv(e, 1.0f / (float)D), a2 = e - a * D;
+        OpenAt o;
+        o.v = ((p >> 1) ? N0 * (N0 + 1) : 0) + a2 * sa * N + a * sa + g * sb;
+        o.m = (p ^ 1) * PL * 64 + g * Dp;
+        o.b = g < open_groups(p) ? g : Dp;
+        return o;
+    }
     struct Entry {
         E re, im;
     };
-    __device__ __forceinline__ Entry open(int p) {
-        const int o = p >> 1, D = rec.dim[p], Dp = rec.dim[p ^ 1], DD = D * D;
-        const int sa = (p & 1) ? 1 : Dp, sb = (p & 1) ? D : 1;
-        const int N = o ? N1 : N0, eshare = N0 * N0 + N1 * N1;
-        const E *mp = ml + (p ^ 1) * PL * 64;
-        const E *Ro = Ml + (o ? N0 * N0 : 0);
-        int G = 1;
-        while (2 * G * DD <= 64) G *= 2;  // lanes per entry, lane = g * DD + entry
-        const int g = lane / DD, e = lane - g * DD, a = e / D, a2 = e - a * D;
+    __device__ __forceinline__ Entry open(int p, const OpenAt at) const {
+        const int D = rec.dim[p], Dp = rec.dim[p ^ 1], DD = D * D, G = open_groups(p);
+        const int sb = (p & 1) ? D : 1;
+        const int N = ((p >> 1) ? N1 : N0) + 1;
+        const E *mp = ml + at.m, *Ro = Ml + at.v;
+        // the other share of the slices (without one, the same entry read again and dropped: a
+        // branch here would wait for every load by itself)
+        constexpr bool SHARES = NT < 4;
+        const bool two = split > 1;
+        const int eshare = two ? pair_env_elems(N0, N1) : 0;
         E x = E(0), xi = E(0);
-        if (g < G) {
-            // lane g takes rows b = g, g + G, ... of the partner message; the eight columns
-            // are read at once (clamped, the absent ones dropped)
-            for (int b = g; b < Dp; b += G) {
-                E v[8], m[8], vi[CX ? 8 : 1], mi[CX ? 8 : 1];
+        // lane g takes rows b = g, g + G, ... of the partner message; the eight columns are
+        // read at once (clamped, the absent ones dropped)
+        for (int b = at.b; b < Dp; b += G, mp += G * Dp, Ro += G * sb) {
+            E v[8], m[8], u[8], vi[CX ? 8 : 1], mi[CX ? 8 : 1], ui[CX ? 8 : 1];
 #pragma unroll
-                for (int b2 = 0; b2 < 8; ++b2) {
-                    const int bc = min(b2, Dp - 1);
-                    const int at = (a2 * sa + bc * sb) * N + a * sa + b * sb;
-                    v[b2] = Ro[at];
-                    m[b2] = mp[b * Dp + bc];
-                    if (split > 1) v[b2] += Ro[eshare + at];
-                    if constexpr (CX) {
-                        vi[b2] = Ro[env_elems + at];
-                        mi[b2] = mp[64 + b * Dp + bc];
-                        if (split > 1) vi[b2] += Ro[env_elems + eshare + at];
-                    }
+            for (int b2 = 0; b2 < 8; ++b2) {
+                const int bc = min(b2, Dp - 1), o = bc * sb * N;
+                v[b2] = Ro[o];
+                m[b2] = mp[bc];
+                if constexpr (SHARES) u[b2] = Ro[eshare + o];
+                if constexpr (CX) {
+                    vi[b2] = Ro[env_elems + o];
+                    mi[b2] = mp[64 + bc];
+                    ui[b2] = Ro[env_elems + eshare + o];
                 }
+            }
 #pragma unroll
-                for (int b2 = 0; b2 < 8; ++b2) {
-                    if (b2 >= Dp) break;
-                    if constexpr (CX) {
-                        x += v[b2] * m[b2] - vi[b2] * mi[b2];
-                        xi += v[b2] * mi[b2] + vi[b2] * m[b2];
-                    } else {
-                        x += v[b2] * m[b2];
-                    }
+            for (int b2 = 0; b2 < 8; ++b2) {
+                if constexpr (SHARES) v[b2] = two ? v[b2] + u[b2] : v[b2];
+                if constexpr (CX) vi[b2] = two ? vi[b2] + ui[b2] : vi[b2];
+            }
+#pragma unroll
+            for (int b2 = 0; b2 < 8; ++b2) {
+                if (b2 >= Dp) break;
+                if constexpr (CX) {
+                    x += v[b2] * m[b2] - vi[b2] * mi[b2];
+                    xi += v[b2] * mi[b2] + vi[b2] * m[b2];
+                } else {
+                    x += v[b2] * m[b2];
                 }
             }
         }
@@ -374,7 +410,7 @@ struct PairCore {
 };
 
 template <int TY, int NT>
-__global__ __launch_bounds__(64 * PAIR_MAXWAVES) void k_pair(
+__global__ __launch_bounds__(64 * pair_waves(NT)) void k_pair(
     const PairRec *__restrict__ recs, const int *__restrict__ items,
     const typename PairTy<TY>::E *__restrict__ sites, const typename PairTy<TY>::E *mold,
     typename PairTy<TY>::E *mnew, NetCtl ctl, double *__restrict__ res_fid,
@@ -385,7 +421,7 @@ __global__ __launch_bounds__(64 * PAIR_MAXWAVES) void k_pair(
     constexpr bool CX = Core::CX;
     constexpr int PL = Core::PL;
     extern __shared__ __align__(16) char smem[];
-    __shared__ double fold_m[PAIR_MAXWAVES];
+    __shared__ double fold_m[pair_waves(NT)];
 
     const int item = blockIdx.x;
     const int ri = items ? items[item] >> 2 : item;
@@ -450,7 +486,7 @@ __global__ __launch_bounds__(64 * PAIR_MAXWAVES) void k_pair(
     for (int p = w; p < 4; p += W) {
         const int q = rec.slot[p];
         if (q < 0 || !((mask >> p) & 1)) continue;
-        typename Core::Entry v = K.open(p);
+        typename Core::Entry v = K.open(p, K.open_at(p));
         const bool real = lane < rec.dim[p] * rec.dim[p];
         if (zv) {
             if constexpr (CX) {
@@ -621,7 +657,7 @@ __device__ __forceinline__ double pair_delta(const PairRunArgs &a, int t, int la
 // in registers); larger ones stage them.  Pairs of up to 32 in FP64: four waves a SIMD, two
 // workgroups on a CU.
 template <int TY, int NT>
-__global__ __launch_bounds__(64 * PAIR_MAXWAVES, TY == PAIR_F64 && NT == 2 ? 4 : 1) void k_pair_run(
+__global__ __launch_bounds__(64 * pair_waves(NT), TY == PAIR_F64 && NT == 2 ? 4 : 1) void k_pair_run(
     const PairRec *__restrict__ recs, const int4 *__restrict__ step_list,
     const double *__restrict__ sites, PairRunArgs a) {
     using Core = PairCore<TY, NT>;
@@ -629,7 +665,7 @@ __global__ __launch_bounds__(64 * PAIR_MAXWAVES, TY == PAIR_F64 && NT == 2 ? 4 :
     constexpr int PL = Core::PL;
     constexpr int MB = 4 * PL * 64;  // one set of incoming messages
     extern __shared__ __align__(16) char smem[];
-    __shared__ double fold_m[PAIR_MAXWAVES];
+    __shared__ double fold_m[pair_waves(NT)];
     __shared__ int verdict;  // 0: go on, 1: the sweep of the look-back was the last, 2: give up
     __shared__ int stop_at;
 
@@ -681,6 +717,9 @@ __global__ __launch_bounds__(64 * PAIR_MAXWAVES, TY == PAIR_F64 && NT == 2 ? 4 :
     }
     __syncthreads();
 
+    typename Core::OpenAt where[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) where[i] = K.open_at(min(w + i * W, 3));
     int loaded[2] = {-1, -1};  // version of the incoming message in LDS, per position of the wave
     int stop = 0, s = 1;
     bool leave = false;
@@ -793,11 +832,14 @@ __global__ __launch_bounds__(64 * PAIR_MAXWAVES, TY == PAIR_F64 && NT == 2 ? 4 :
             }
             K.env_store(R, Ri);
             __syncthreads();
-            for (int p = w; p < 4; p += W) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int p = w + i * W;
+                if (p >= 4) break;
                 const int q = rec.slot[p];
                 if (q < 0 || !((mask >> p) & 1)) continue;
                 const bool real = lane < rec.dim[p] * rec.dim[p];
-                const typename Core::Entry y = Core::normalise(real, K.open(p));
+                const typename Core::Entry y = Core::normalise(real, K.open(p, where[i]));
                 const long long o = (rec.out[p] + lane) * PL;
                 pair_settle();  // the poison of version s, stored a sweep ago
                 if (real) {
@@ -906,9 +948,7 @@ static constexpr size_t PAIR_LDS_MAX = 160 * 1024 - 256;  // 256: the static fol
 void pair_release(PairPlan *p) {
     if (p->d_recs) (void)hipFree(p->d_recs);
     if (p->d_lead) (void)hipFree(p->d_lead);
-    for (void *q : {(void *)p->d_steps[0], (void *)p->d_steps[1], p->d_ring, p->d_ctrl,
-                    (void *)p->d_ring_res})
-        if (q) (void)hipFree(q);
+    if (p->d_run) (void)hipFree(p->d_run);
     *p = PairPlan();
 }
 
@@ -973,15 +1013,18 @@ int pair_plan_build(PairPlan *p, int dtype, int plain, int nv, int nnet, const i
     p->all = (int)p->recs.size() == nv;
     for (int n = 0; n < nnet; ++n) p->covers = p->covers && lead[n] >= 0;
     p->nt = (maxn + 15) / 16;
-    // one tile column per half leaves two waves: share the slices between two more
-    p->split = p->nt <= 2 && maxd >= 2 ? 2 : 1;
-    p->waves = 2 * p->nt * p->split;
     const size_t esz = dtype == PAIR_F32 ? 4 : dtype == PAIR_C128 ? 16 : 8;
+    // Few tile columns leave few waves: share the slices between two more each.  Three columns
+    // a half are six waves, which four SIMDs take in two turns; twelve are even, but take the
+    // LDS of two workgroups, so only where the vertices are at most one to a CU (us a sweep at
+    // 16x16 D = 6: 19 against 14).
+    p->split = maxd >= 2 && (p->nt <= 2 || (p->nt == 3 && p->recs.size() <= 256)) ? 2 : 1;
+    p->waves = 2 * p->nt * p->split;
     int slice = 0, env = 0;
     for (const PairRec &r : p->recs) {
         const int N0 = pair_pad(r.n[0]), N1 = pair_pad(r.n[1]);
         slice = std::max(slice, pair_slice_elems(r.n[0], r.n[1]));
-        env = std::max(env, p->split * (N0 * N0 + N1 * N1));
+        env = std::max(env, p->split * pair_env_elems(N0, N1));
     }
     const size_t fixed = esz * ((size_t)env + 4 * 64);
     // as many slices at a time as fit the LDS
@@ -1112,14 +1155,25 @@ bool pair_run_ready(PairPlan *p, int nnet, long long nmsg, int nports) {
     const size_t pl = p->dtype == PAIR_C128 ? 2 : 1, sb = sizeof(int) * steps.size();
     p->run_nm = (long long)pl * nmsg;
     p->run_nports = nports;
-    if (hipMalloc((void **)&p->d_steps[0], sb) != hipSuccess ||
-        hipMalloc((void **)&p->d_steps[1], sb) != hipSuccess ||
-        hipMalloc(&p->d_ring, sizeof(double) * PAIR_RING * p->run_nm) != hipSuccess ||
-        hipMalloc(&p->d_ctrl, sizeof(PairCtrl) * PAIR_CTRL_LINES * PAIR_RUN_SWEEPS) != hipSuccess ||
-        hipMalloc((void **)&p->d_ring_res, sizeof(double) * 2 * PAIR_RING * nports) != hipSuccess ||
-        hipMemcpy(p->d_steps[0], steps.data(), sb, hipMemcpyHostToDevice) != hipSuccess) {
+    // one allocation: ring, residuals, counters, schedules
+    const size_t ring = sizeof(double) * PAIR_RING * (size_t)p->run_nm;
+    const size_t res = sizeof(double) * 2 * PAIR_RING * (size_t)nports;
+    const size_t ctrl = sizeof(PairCtrl) * PAIR_CTRL_LINES * PAIR_RUN_SWEEPS;
+    const size_t at_ctrl = (ring + res + 63) / 64 * 64;
+    char *base = nullptr;
+    if (hipMalloc((void **)&base, at_ctrl + ctrl + 2 * sb) != hipSuccess) {
         (void)hipGetLastError();
-        return false;  // pair_release frees what there is
+        return false;
+    }
+    p->d_run = base;
+    p->d_ring = base;
+    p->d_ring_res = (double *)(base + ring);
+    p->d_ctrl = base + at_ctrl;
+    p->d_steps[0] = (int *)(base + at_ctrl + ctrl);
+    p->d_steps[1] = (int *)(base + at_ctrl + ctrl + sb);
+    if (hipMemcpy(p->d_steps[0], steps.data(), sb, hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
     }
     p->run_state = 1;
     return true;
