@@ -18,6 +18,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/bp_mi355x.h"
@@ -431,6 +432,12 @@ struct bp_context {
     // adjoint scratch
     AdjointScratch adj;
 
+    // kept between calls, freed with the context (or at the end of a call that needed more
+    // than KEEP_BYTES): device workspace and pinned host staging
+    void *d_scratch = nullptr, *h_scratch = nullptr;
+    size_t scratch_bytes = 0, h_scratch_bytes = 0;
+    hipEvent_t ev_chunk[2] = {nullptr, nullptr};  // chunked copies to the host
+
     size_t elt() const {
         return dtype == BP_C128 ? sizeof(cplx) : dtype == BP_F64 ? sizeof(double) : sizeof(float);
     }
@@ -487,6 +494,128 @@ static int vx_variant_of(const bp_context *c) {
 }
 
 static size_t run_state_bytes(int nnet) { return (sizeof(double) + 3 * sizeof(int)) * nnet; }
+
+static constexpr size_t KEEP_BYTES = (size_t)1 << 30;
+
+// The kept device workspace and pinned staging, at least this large.
+static int keep_scratch(bp_context *c, size_t dev, size_t host) {
+    if (c->scratch_bytes < dev) {
+        if (c->d_scratch) (void)hipFree(c->d_scratch);
+        c->d_scratch = nullptr;
+        c->scratch_bytes = 0;
+        if (hipMalloc(&c->d_scratch, dev) != hipSuccess) {
+            c->d_scratch = nullptr;
+            (void)hipGetLastError();
+            return set_err(BP_ERR_NOMEM, "workspace (%zu bytes) does not fit", dev);
+        }
+        c->scratch_bytes = dev;
+    }
+    if (c->h_scratch_bytes < host) {
+        if (c->h_scratch) (void)hipHostFree(c->h_scratch);
+        c->h_scratch = nullptr;
+        c->h_scratch_bytes = 0;
+        if (hipHostMalloc(&c->h_scratch, host, hipHostMallocDefault) != hipSuccess) {
+            c->h_scratch = nullptr;
+            (void)hipGetLastError();
+            return set_err(BP_ERR_NOMEM, "pinned staging (%zu bytes) does not fit", host);
+        }
+        c->h_scratch_bytes = host;
+    }
+    return BP_OK;
+}
+
+static void scratch_release(bp_context *c, size_t keep) {
+    if (c->scratch_bytes > keep) {
+        (void)hipFree(c->d_scratch);
+        c->d_scratch = nullptr;
+        c->scratch_bytes = 0;
+    }
+    if (c->h_scratch_bytes > keep) {
+        (void)hipHostFree(c->h_scratch);
+        c->h_scratch = nullptr;
+        c->h_scratch_bytes = 0;
+    }
+}
+
+// n FP32 or FP64 values from the device to doubles, `stream` drained.  Large arrays go through
+// two pinned chunks, one in flight while up to four threads unpack the other: the copy of a
+// pageable buffer, the page faults of its zeroed memory and of `out`, and the conversion came
+// one after the other (9.4 MB of FP32 messages: 2.2 ms, now 0.7).
+static int download_doubles(bp_context *c, const void *dev, bool f32, long long n, double *out) {
+    constexpr size_t CHUNK = (size_t)2 << 20;  // bytes
+    const size_t es = f32 ? sizeof(float) : sizeof(double);
+    if (es * n <= CHUNK / 8 || (!f32 && es * n <= CHUNK)) {
+        std::vector<float> tmp(f32 ? n : 0);
+        HIPCHK(hipMemcpyAsync(f32 ? (void *)tmp.data() : (void *)out, dev, es * n,
+                              hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        for (size_t i = 0; i < tmp.size(); ++i) out[i] = tmp[i];
+        return BP_OK;
+    }
+    const long long per = (long long)(CHUNK / es), chunks = (n + per - 1) / per;
+    RETCHK(keep_scratch(c, 0, std::min<size_t>(es * n, 2 * CHUNK)));
+    for (auto &e : c->ev_chunk)
+        if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    auto fetch = [&](long long k) {
+        const long long m = std::min(per, n - k * per);
+        hipError_t e = hipMemcpyAsync((char *)c->h_scratch + (k & 1) * CHUNK,
+                                      (const char *)dev + es * k * per, es * m,
+                                      hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipEventRecord(c->ev_chunk[k & 1], c->stream);
+        return e;
+    };
+    auto unpack = [&](long long k, long long i0, long long i1) {
+        const char *h = (const char *)c->h_scratch + (k & 1) * CHUNK;
+        double *o = out + k * per;
+        if (f32)
+            for (long long i = i0; i < i1; ++i) o[i] = (double)((const float *)h)[i];
+        else
+            std::memcpy(o + i0, (const double *)h + i0, sizeof(double) * (i1 - i0));
+    };
+    if (chunks > 0) HIPCHK(fetch(0));
+    hipError_t err = hipSuccess;
+    // helper threads hold chunks' shares back until main has seen the chunk arrive
+    const int T = n >= (1 << 19) ? 4 : 1;
+    std::atomic<long long> ready{-1};
+    std::vector<std::atomic<long long>> done(T);
+    for (auto &d : done) d.store(-1);
+    std::vector<std::thread> pool;
+    pool.reserve(T);
+    auto share = [&](int t, long long k) {
+        const long long m = std::min(per, n - k * per);
+        unpack(k, m * t / T, m * (t + 1) / T);
+    };
+    auto helper = [&](int t) {
+        for (long long k = 0; k < chunks; ++k) {
+            long long r;
+            while ((r = ready.load(std::memory_order_acquire)) < k) std::this_thread::yield();
+            if (r > chunks) return;  // given up
+            share(t, k);
+            done[t].store(k, std::memory_order_release);
+        }
+    };
+    int started = 1;
+    try {
+        for (; started < T; ++started) pool.emplace_back(helper, started);
+    } catch (...) {  // no more threads: their shares are unpacked here
+    }
+    for (long long k = 0; k < chunks && err == hipSuccess; ++k) {
+        // chunk k + 1 goes where chunk k - 1 was
+        if (k + 1 < chunks) err = fetch(k + 1);
+        if (err == hipSuccess) err = hipEventSynchronize(c->ev_chunk[k & 1]);
+        if (err != hipSuccess) break;
+        ready.store(k, std::memory_order_release);
+        share(0, k);
+        for (int t = started; t < T; ++t) share(t, k);
+        for (int t = 1; t < started; ++t)
+            while (done[t].load(std::memory_order_acquire) < k) std::this_thread::yield();
+    }
+    if (err != hipSuccess) ready.store(chunks + 1, std::memory_order_release);
+    for (auto &t : pool) t.join();
+    HIPCHK(err);
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return BP_OK;
+}
 
 static void graphs_release(bp_context *c) {
     for (auto &g : c->gexec) {
@@ -1200,6 +1329,9 @@ int bp_destroy(bp_context *c) {
     (void)hipStreamSynchronize(c->stream);
     free_all(c);
     if (c->h_state) (void)hipHostFree(c->h_state);
+    scratch_release(c, 0);
+    for (auto &e : c->ev_chunk)
+        if (e) (void)hipEventDestroy(e);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
@@ -1448,21 +1580,9 @@ int bp_download_messages(bp_context *c, double *out) {
     if (!c || !out) return set_err(BP_ERR_ARG, "NULL argument");
     if (!c->have_msgs) return set_err(BP_ERR_STATE, "no messages");
     HIPCHK(hipSetDevice(c->device));
-    if (c->fp64_active) {
-        HIPCHK(hipMemcpyAsync(out, c->d_msg64[c->cur64], sizeof(double) * c->nmsg,
-                              hipMemcpyDeviceToHost, c->stream));
-    } else if (c->dtype == BP_F64 || c->is_cplx()) {
-        HIPCHK(hipMemcpyAsync(out, c->d_msg[c->cur], sizeof(double) * c->hw() * c->nmsg,
-                              hipMemcpyDeviceToHost, c->stream));
-    } else {
-        std::vector<float> tmp(c->nmsg);
-        HIPCHK(hipMemcpyAsync(tmp.data(), c->d_msg[c->cur], sizeof(float) * c->nmsg,
-                              hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        for (long long i = 0; i < c->nmsg; ++i) out[i] = tmp[i];
-    }
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return BP_OK;
+    if (c->fp64_active) return download_doubles(c, c->d_msg64[c->cur64], false, c->nmsg, out);
+    return download_doubles(c, c->d_msg[c->cur], c->dtype != BP_F64 && !c->is_cplx(),
+                            c->hw() * c->nmsg, out);
 }
 
 // Slot ranges of the message buffer: checks the slots and sizes a host buffer.
@@ -3232,39 +3352,40 @@ int bp_apply_gates_resident(bp_context *c, int ngates, const int *kind, const in
     HIPCHK(hipSetDevice(c->device));
     bool is64 = false;
     const void *msgs = current_msgs(c, &is64);
-    int *d_desc = nullptr, *d_chi = nullptr;
-    long long *d_offs = nullptr, *d_seg = nullptr, *d_rec = nullptr;
-    double *d_gates = nullptr, *d_in = nullptr, *d_out = nullptr, *d_ws = nullptr, *d_s = nullptr;
-    auto release = [&]() {
-        for (void *ptr : {(void *)d_desc, (void *)d_chi, (void *)d_offs, (void *)d_seg,
-                          (void *)d_rec, (void *)d_gates, (void *)d_in, (void *)d_out,
-                          (void *)d_ws, (void *)d_s})
-            if (ptr) (void)hipFree(ptr);
+    // one kept workspace: [desc | offs | seg | rec | gates | chi | s] with one copy in and one
+    // of its tail out, then the packed inputs, outputs and scratch of the kernel
+    const int sv = out_s ? s_stride : 0;
+    size_t at = 0;
+    auto place = [&](size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) / 256 * 256;
+        return o;
     };
-    const size_t sbytes = out_s ? sizeof(double) * (size_t)ngates * s_stride : 0;
-    if (hipMalloc((void **)&d_desc, sizeof(int) * desc.size()) != hipSuccess ||
-        hipMalloc((void **)&d_chi, sizeof(int) * (size_t)ngates) != hipSuccess ||
-        hipMalloc((void **)&d_offs, sizeof(long long) * offs.size()) != hipSuccess ||
-        hipMalloc((void **)&d_seg, sizeof(long long) * std::max<size_t>(seg.size(), 1)) != hipSuccess ||
-        hipMalloc((void **)&d_rec, sizeof(long long) * rec.size()) != hipSuccess ||
-        hipMalloc((void **)&d_gates, sizeof(double) * std::max(gsum, 1LL)) != hipSuccess ||
-        hipMalloc((void **)&d_in, sizeof(double) * std::max(tin, 1LL)) != hipSuccess ||
-        hipMalloc((void **)&d_out, sizeof(double) * std::max(tout, 1LL)) != hipSuccess ||
-        hipMalloc((void **)&d_ws, sizeof(double) * std::max(tws, 1LL)) != hipSuccess ||
-        (out_s && hipMalloc((void **)&d_s, sbytes) != hipSuccess)) {
-        release();
-        return set_err(BP_ERR_NOMEM, "gate workspace (%lld doubles) does not fit", tws);
-    }
-    hipError_t e = hipSuccess;
-    auto up = [&](void *dst, const void *src, size_t n) {
-        if (e == hipSuccess) e = hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, c->stream);
-    };
-    up(d_desc, desc.data(), sizeof(int) * desc.size());
-    up(d_offs, offs.data(), sizeof(long long) * offs.size());
-    up(d_seg, seg.data(), sizeof(long long) * seg.size());
-    up(d_rec, rec.data(), sizeof(long long) * rec.size());
-    up(d_gates, gates, sizeof(double) * gsum);
-    if (e == hipSuccess && d_s) e = hipMemsetAsync(d_s, 0, sbytes, c->stream);
+    const size_t o_desc = place(sizeof(int) * desc.size());
+    const size_t o_offs = place(sizeof(long long) * offs.size());
+    const size_t o_seg = place(sizeof(long long) * seg.size());
+    const size_t o_rec = place(sizeof(long long) * rec.size());
+    const size_t o_gates = place(sizeof(double) * gsum);
+    const size_t o_chi = place(sizeof(int) * (size_t)ngates);
+    const size_t o_s = place(sizeof(double) * (size_t)ngates * sv);
+    const size_t up_bytes = at;
+    const size_t o_in = place(sizeof(double) * tin), o_out = place(sizeof(double) * tout);
+    const size_t o_ws = place(sizeof(double) * tws);
+    RETCHK(keep_scratch(c, at, up_bytes));
+    char *dev = (char *)c->d_scratch, *host = (char *)c->h_scratch;
+    std::memcpy(host + o_desc, desc.data(), sizeof(int) * desc.size());
+    std::memcpy(host + o_offs, offs.data(), sizeof(long long) * offs.size());
+    std::memcpy(host + o_seg, seg.data(), sizeof(long long) * seg.size());
+    std::memcpy(host + o_rec, rec.data(), sizeof(long long) * rec.size());
+    std::memcpy(host + o_gates, gates, sizeof(double) * gsum);
+    std::memset(host + o_chi, 0, up_bytes - o_chi);
+    int *d_desc = (int *)(dev + o_desc), *d_chi = (int *)(dev + o_chi);
+    long long *d_offs = (long long *)(dev + o_offs), *d_seg = (long long *)(dev + o_seg),
+              *d_rec = (long long *)(dev + o_rec);
+    double *d_gates = (double *)(dev + o_gates), *d_in = (double *)(dev + o_in),
+           *d_out = (double *)(dev + o_out), *d_ws = (double *)(dev + o_ws),
+           *d_s = out_s ? (double *)(dev + o_s) : nullptr;
+    hipError_t e = hipMemcpyAsync(dev, host, up_bytes, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess)
         e = hipFuncSetAttribute((const void *)k_gate,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
@@ -3310,15 +3431,17 @@ int bp_apply_gates_resident(bp_context *c, int ngates, const int *kind, const in
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipEventRecord(c->ev1, c->stream);
-    if (e == hipSuccess && out_chi)
-        e = hipMemcpyAsync(out_chi, d_chi, sizeof(int) * (size_t)ngates, hipMemcpyDeviceToHost,
+    if (e == hipSuccess && (out_chi || out_s))
+        e = hipMemcpyAsync(host + o_chi, dev + o_chi, up_bytes - o_chi, hipMemcpyDeviceToHost,
                            c->stream);
-    if (e == hipSuccess && out_s)
-        e = hipMemcpyAsync(out_s, d_s, sbytes, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess && out_chi)
+        std::memcpy(out_chi, host + o_chi, sizeof(int) * (size_t)ngates);
+    if (e == hipSuccess && out_s)
+        std::memcpy(out_s, host + o_s, sizeof(double) * (size_t)ngates * sv);
     float ms = 0.f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, c->ev0, c->ev1);
-    release();
+    scratch_release(c, KEEP_BYTES);
     if (e != hipSuccess) return set_err(BP_ERR_HIP, "resident gates: %s", hipGetErrorString(e));
     c->last_ms = ms;
     RETCHK(refresh_sites(c));
