@@ -268,11 +268,108 @@ __global__ __launch_bounds__(256) void k_cn_cols(
     }
 }
 
+// Two streaming products in one pass: X[m, v, (s, o)] = sum_u A[m, v, u] B1[u, (s, o)], then
+// C[m, o, n] = sum_{v, s} X[m, v, (s, o)] B2[(v, s), n], with X in LDS for 16 rows m at a time.
+//
+// Both steps are bound by memory: absorbing a site tensor and its conjugate into the boundary
+// of a PEPS norm writes and reads the intermediate X, d times the boundary, between them (6 x 6
+// at D = 3: 38 MB in, 77 MB out and in, 38 MB out, 64 us a site).  Here the boundary is read
+// and written once.  The products are on 16x16x4 FP64 MFMA: a tile is 16 rows m of one v (then
+// of one o), and a wave keeps its fragments of B1 and B2 in registers for the whole launch.  On
+// the vector units the same pass is bound by its LDS reads of B1 and B2, one for two FMAs
+// (1296 us a call; two rows a thread 1858).
+#define CN_PAIR_NT 256
+#define CN_PAIR_P 17  // row pitch of X: its columns are written, its rows read, 16 at a time
+struct CnPairArgs {
+    const double *A, *B1, *B2;
+    const long long *ahi, *alo, *au, *av;    // A: rows (high, low), u, v
+    const long long *b1r, *b1c, *b2r, *b2c;  // B1: u, (s, o); B2: (v, s), n
+    double *C;
+    unsigned M, mlo;
+    int U, V, S, O, N;
+};
+
+// KU, KS: 16x16x4 steps over u and over (v, s); NS: 16-wide tiles of (s, o)
+template <int KU, int NS, int KS>
+__global__ __launch_bounds__(CN_PAIR_NT) void k_cn_pair(CnPairArgs a) {
+    typedef double v4 __attribute__((ext_vector_type(4)));
+    extern __shared__ double cn_lds[];  // X [(v, s, o)][CN_PAIR_P]
+    const int SO = a.S * a.O, VS = a.V * a.S;
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    double b1[KU][NS], b2[KS];
+    long long ou[KU];
+#pragma unroll
+    for (int t = 0; t < KU; ++t) {
+        const int u = min(4 * t + lk, a.U - 1);
+        const bool in = 4 * t + lk < a.U;
+        ou[t] = a.au[u];
+#pragma unroll
+        for (int c = 0; c < NS; ++c) {
+            const double x = a.B1[a.b1r[u] + a.b1c[min(16 * c + li, SO - 1)]];
+            b1[t][c] = in && 16 * c + li < SO ? x : 0.0;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < KS; ++t) {
+        const double x = a.B2[a.b2r[min(4 * t + lk, VS - 1)] + a.b2c[min(li, a.N - 1)]];
+        b2[t] = 4 * t + lk < VS && li < a.N ? x : 0.0;
+    }
+    for (unsigned m0 = blockIdx.x * 16u; m0 < a.M; m0 += gridDim.x * 16u) {
+        const unsigned m = min(m0 + li, a.M - 1), hi = m / a.mlo;
+        const double *row = a.A + a.ahi[hi] + a.alo[m - hi * a.mlo];
+        for (int v = w; v < a.V; v += CN_PAIR_NT / 64) {
+            const double *x = row + a.av[v];
+            double e[KU];
+#pragma unroll
+            for (int t = 0; t < KU; ++t) e[t] = x[ou[t]];
+            v4 acc[NS];
+#pragma unroll
+            for (int c = 0; c < NS; ++c) acc[c] = v4{0, 0, 0, 0};
+#pragma unroll
+            for (int t = 0; t < KU; ++t) {
+                const double y = 4 * t + lk < a.U ? e[t] : 0.0;
+#pragma unroll
+                for (int c = 0; c < NS; ++c)
+                    acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(y, b1[t][c], acc[c], 0, 0, 0);
+            }
+            // lane: column 16 c + li, rows lk + 4 q
+#pragma unroll
+            for (int c = 0; c < NS; ++c)
+                if (16 * c + li < SO) {
+                    double *X = cn_lds + (v * SO + 16 * c + li) * CN_PAIR_P + lk;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) X[4 * q] = acc[c][q];
+                }
+        }
+        __syncthreads();
+        for (int o = w; o < a.O; o += CN_PAIR_NT / 64) {
+            double e[KS];
+#pragma unroll
+            for (int t = 0; t < KS; ++t)
+                e[t] = cn_lds[(min(4 * t + lk, VS - 1) * a.O + o) * CN_PAIR_P + li];
+            v4 acc = v4{0, 0, 0, 0};
+#pragma unroll
+            for (int t = 0; t < KS; ++t)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(4 * t + lk < VS ? e[t] : 0.0, b2[t], acc,
+                                                           0, 0, 0);
+            if (li < a.N) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const unsigned r = m0 + lk + 4 * q;
+                    if (r < a.M) a.C[((long long)r * a.O + o) * a.N + li] = acc[q];
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
 // ------------------------------------------------------------------ host plan
 
 enum { CN_ORDER_LEFT = 0, CN_ORDER_GREEDY = 1, CN_ORDER_CHEAPEST = 2 };
 
-enum { CN_KIND_MFMA = 0, CN_KIND_ROWS = 1, CN_KIND_COLS = 2 };
+enum { CN_KIND_MFMA = 0, CN_KIND_ROWS = 1, CN_KIND_COLS = 2, CN_KIND_NONE = 3, CN_KIND_PAIR = 4 };
 
 struct CnStep {
     int a = 0, b = 0;             // operand ids (< nt: input tensors, else nt + step)
@@ -289,6 +386,11 @@ struct CnStep {
     long long c = 0;              // arena offset of the result
     int splits = 1;
     long long kchunk = 0, part = -1;  // split K: chunk and arena offset of the partials
+    // CN_KIND_PAIR (the step before it is CN_KIND_NONE): its second small operand, tables in
+    // the order of CnPairArgs, extents
+    int b2 = 0;
+    long long t2[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    int U = 1, V = 1, S = 1, O = 1;
 };
 
 struct bp_cn_plan {
@@ -557,6 +659,124 @@ static int cn_plan_step(const CnOperand &A, const CnOperand &B, const int *label
     return 0;
 }
 
+// Plans the contraction of A with B1 and of the result with B2 as one fused step when both are
+// streaming products over A's rows (the shapes of cn_plan_step's rule) and the small operands
+// fit a wave's fragments; false leaves everything as it was.  The result's labels are in the order of the
+// two steps: A's open ones, B1's, B2's (those that the consumer contracts first).
+static bool cn_plan_pair(const CnOperand &A, const CnOperand &B1, const CnOperand &B2,
+                         const int *label_dim, long long max_elems, CnArena &ar,
+                         std::vector<long long> &offs, CnStep &st, CnOperand &R,
+                         const std::vector<int> &next_shared) {
+    auto in = [](const std::vector<int> &l, int x) {
+        return std::find(l.begin(), l.end(), x) != l.end();
+    };
+    auto dims = [&](const CnOperand &T, std::vector<int> &d, std::vector<long long> &str) {
+        const int r = (int)T.lab.size();
+        d.resize(r);
+        str.resize(r);
+        long long s = 1;
+        for (int i = r - 1; i >= 0; --i) {
+            d[i] = label_dim[T.lab[i]];
+            str[i] = s;
+            s *= d[i];
+        }
+    };
+    auto where = [](const CnOperand &T, int l) {
+        return (int)(std::find(T.lab.begin(), T.lab.end(), l) - T.lab.begin());
+    };
+    std::vector<int> da, d1, d2;
+    std::vector<long long> sa, s1, s2;
+    dims(A, da, sa);
+    dims(B1, d1, s1);
+    dims(B2, d2, s2);
+    std::vector<int> f, ua, va, u1, v2, sh1, sh2, o1, o2;  // positions
+    for (int i = 0; i < (int)A.lab.size(); ++i) {
+        if (in(B1.lab, A.lab[i])) {
+            ua.push_back(i);
+            u1.push_back(where(B1, A.lab[i]));
+        } else if (in(B2.lab, A.lab[i])) {
+            va.push_back(i);
+            v2.push_back(where(B2, A.lab[i]));
+        } else {
+            f.push_back(i);
+        }
+    }
+    for (int j = 0; j < (int)B1.lab.size(); ++j) {
+        if (in(A.lab, B1.lab[j])) continue;
+        if (in(B2.lab, B1.lab[j])) {
+            sh1.push_back(j);
+            sh2.push_back(where(B2, B1.lab[j]));
+        } else {
+            o1.push_back(j);
+        }
+    }
+    for (int j = 0; j < (int)B2.lab.size(); ++j)
+        if (!in(A.lab, B2.lab[j]) && !in(B1.lab, B2.lab[j])) o2.push_back(j);
+    std::stable_partition(o2.begin(), o2.end(), [&](int j) { return in(next_shared, B2.lab[j]); });
+    // b1's open labels that the consumer of the pair contracts stay where the second step, which
+    // keeps them, leaves them
+    double M = 1, U = 1, V = 1, S = 1, O = 1, N = 1;
+    for (int i : f) M *= da[i];
+    for (int i : ua) U *= da[i];
+    for (int i : va) V *= da[i];
+    for (int j : sh1) S *= d1[j];
+    for (int j : o1) O *= d1[j];
+    for (int j : o2) N *= d2[j];
+    if (f.size() + va.size() + sh1.size() + o1.size() > 64 || f.size() + o1.size() + o2.size() > 64)
+        return false;
+    // both steps stream A's side (so neither is refused or runs on another kernel alone)
+    auto rows = [](double m, double n, double k) {
+        return m >= n && m < (double)(1LL << 31) && k * (std::ceil(n / 16) * 16 + 1) <= CN_LDS_ELEMS;
+    };
+    if (!rows(M * V, S * O, U) || !rows(M * O, N, V * S)) return false;
+    if (M * V * S * O > (double)max_elems || M * O * N > (double)max_elems) return false;
+    // the fragments that k_cn_pair's instances hold, and X: every pair of a PEPS norm up to
+    // D = 4 at d = 2
+    if (U > 16 || S * O > 32 || V * S > 32 || N > 16 ||
+        V * S * O * CN_PAIR_P > (double)CN_LDS_ELEMS * 2)
+        return false;
+    size_t cut = f.size();
+    long long lo_n = 1;
+    while (cut > 0 && lo_n < 256) lo_n *= da[f[--cut]];
+    const std::vector<int> hi(f.begin(), f.begin() + cut), lo(f.begin() + cut, f.end());
+    std::vector<int> so(sh1), vs(v2);
+    so.insert(so.end(), o1.begin(), o1.end());
+    vs.insert(vs.end(), sh2.begin(), sh2.end());
+    int n = 0;
+    auto table = [&](const std::vector<int> &pos, const std::vector<long long> &str,
+                     const std::vector<int> &dim) {
+        st.t2[n++] = (long long)offs.size();
+        cn_offsets(pos, str, dim, offs);
+    };
+    table(hi, sa, da);
+    table(lo, sa, da);
+    table(ua, sa, da);
+    table(va, sa, da);
+    table(u1, s1, d1);
+    table(so, s1, d1);
+    table(vs, s2, d2);
+    table(o2, s2, d2);
+    st.kind = CN_KIND_PAIR;
+    st.M = (long long)(M * O);
+    st.N = (long long)N;
+    st.K = (long long)(V * S);
+    st.lo_n = lo_n;
+    st.U = (int)U;
+    st.V = (int)V;
+    st.S = (int)S;
+    st.O = (int)O;
+    st.kchunk = st.K;
+    st.c = ar.alloc((long long)(M * O * N));
+    R.lab.clear();
+    for (int i : f) R.lab.push_back(A.lab[i]);
+    for (int j : o1) R.lab.push_back(B1.lab[j]);
+    for (int j : o2) R.lab.push_back(B2.lab[j]);
+    R.size = (long long)(M * O * N);
+    R.arena = st.c;
+    R.live = true;
+    return true;
+}
+
 // ---- contraction orders (host only: labels and dimensions, no data)
 
 // the pairwise result's labels (a's open ones, then b's), its size and the shared size
@@ -800,6 +1020,36 @@ static int cn_build_plan(int nt, const int *ranks, const int *labels, int n_labe
         st.a = a;
         st.b = b;
         CnOperand R;
+        // this step and the next one on its result as one pass
+        if (s + 1 < nt - 1 && pairs[s + 1].first == nt + s) {
+            const int b2 = pairs[s + 1].second;
+            st.b2 = b2;
+            if (cn_plan_pair(ops[a], ops[b], ops[b2], label_dim, max_elems, ar, offs, st, R,
+                             next_shared[s + 1])) {
+                for (int t : {a, b, b2}) {
+                    if (ops[t].arena >= 0) ar.release(ops[t].arena);
+                    ops[t].live = false;
+                }
+                const double m = (double)st.M / st.O;  // rows of the block form
+                p.flops += 2.0 * m * st.V * st.U * st.S * st.O + 2.0 * (double)st.M * st.N * st.K;
+                // the plan's figures are those of the two pairwise steps
+                const long long x = (long long)m * st.V * st.S * st.O;
+                p.bytes += 8.0 * ((double)ops[a].size + (double)ops[b].size + 2.0 * (double)x +
+                                  (double)ops[b2].size + (double)R.size);
+                p.max_interm = std::max(p.max_interm, std::max(x, R.size));
+                CnStep none;
+                none.a = a;
+                none.b = b;
+                none.kind = CN_KIND_NONE;
+                CnOperand gone;
+                ops.push_back(gone);
+                p.steps.push_back(none);
+                ops.push_back(R);
+                p.steps.push_back(st);
+                ++s;
+                continue;
+            }
+        }
         const int rc = cn_plan_step(ops[a], ops[b], label_dim, max_elems, ar, offs, st, R, msg,
                                     next_shared[s]);
         if (rc == 3 || rc == 5) return 4;
@@ -886,7 +1136,48 @@ static const double *cn_result(const bp_cn_plan &p, const double *in) {
 static hipError_t cn_enqueue(const bp_cn_plan &p, const double *in, hipStream_t st,
                              const double **res) {
     for (const CnStep &s : p.steps) {
+        if (s.kind == CN_KIND_NONE) continue;
         const double *A = cn_operand(p, in, s.a), *B = cn_operand(p, in, s.b);
+        if (s.kind == CN_KIND_PAIR) {
+            CnPairArgs x;
+            x.A = A;
+            x.B1 = B;
+            x.B2 = cn_operand(p, in, s.b2);
+            x.ahi = p.offs + s.t2[0];
+            x.alo = p.offs + s.t2[1];
+            x.au = p.offs + s.t2[2];
+            x.av = p.offs + s.t2[3];
+            x.b1r = p.offs + s.t2[4];
+            x.b1c = p.offs + s.t2[5];
+            x.b2r = p.offs + s.t2[6];
+            x.b2c = p.offs + s.t2[7];
+            x.C = p.arena + s.c;
+            x.M = (unsigned)(s.M / s.O);
+            x.mlo = (unsigned)s.lo_n;
+            x.U = s.U;
+            x.V = s.V;
+            x.S = s.S;
+            x.O = s.O;
+            x.N = (int)s.N;
+            const size_t lds = sizeof(double) * (size_t)(s.V * s.S * s.O * CN_PAIR_P);
+            const unsigned grid = (x.M + 15) / 16;
+            const int ku = s.U <= 4 ? 1 : s.U <= 12 ? 3 : 4, ns = s.S * s.O <= 16 ? 1 : 2;
+            const int ks = s.V * s.S <= 8 ? 2 : s.V * s.S <= 20 ? 5 : 8;
+#define CN_PAIR_GO(KU, NS, KS)                                                                   \
+    if (ku == KU && ns == NS && ks == KS) {                                                      \
+        const hipError_t e = hipFuncSetAttribute((const void *)k_cn_pair<KU, NS, KS>,            \
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize,     \
+                                                 CN_LDS_ELEMS * 2 * (int)sizeof(double));        \
+        if (e != hipSuccess) return e;                                                           \
+        hipLaunchKernelGGL((k_cn_pair<KU, NS, KS>), dim3(grid), dim3(CN_PAIR_NT), lds, st, x);   \
+    }
+#define CN_PAIR_GO3(KU, NS) CN_PAIR_GO(KU, NS, 2) CN_PAIR_GO(KU, NS, 5) CN_PAIR_GO(KU, NS, 8)
+            CN_PAIR_GO3(1, 1) CN_PAIR_GO3(1, 2) CN_PAIR_GO3(3, 1) CN_PAIR_GO3(3, 2)
+            CN_PAIR_GO3(4, 1) CN_PAIR_GO3(4, 2)
+#undef CN_PAIR_GO3
+#undef CN_PAIR_GO
+            continue;
+        }
         if (s.kind == CN_KIND_ROWS) {
             const long long N16 = (s.N + 15) / 16 * 16;
             const long long base = s.K * (N16 + 1);
