@@ -1160,7 +1160,13 @@ static hipError_t cn_enqueue(const bp_cn_plan &p, const double *in, hipStream_t 
             x.O = s.O;
             x.N = (int)s.N;
             const size_t lds = sizeof(double) * (size_t)(s.V * s.S * s.O * CN_PAIR_P);
-            const unsigned grid = (x.M + 15) / 16;
+            // whole rounds of what is resident at once: the fragments are read once a workgroup
+            // (6 x 6 at D = 3: 896 us with a workgroup a tile, 725)
+            const long long tiles = (x.M + 15) / 16;
+            const long long room = 256 * std::max<long long>(
+                                             1, std::min<long long>(8, (160 << 10) / (long long)lds));
+            const long long per = (tiles + room - 1) / room;
+            const unsigned grid = (unsigned)((tiles + per - 1) / per);
             const int ku = s.U <= 4 ? 1 : s.U <= 12 ? 3 : 4, ns = s.S * s.O <= 16 ? 1 : 2;
             const int ks = s.V * s.S <= 8 ? 2 : s.V * s.S <= 20 ? 5 : 8;
 #define CN_PAIR_GO(KU, NS, KS)                                                                   \
