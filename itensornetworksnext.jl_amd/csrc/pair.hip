@@ -557,7 +557,10 @@ __global__ __launch_bounds__(64 * pair_waves(NT)) void k_pair(
 //
 // Bounded run-ahead: a workgroup starts sweep s when all have finished sweep s - 4 and the
 // stopping rule says that sweep s - 5 was not the last, so the versions in use, s - 5 to
-// s + 2, are distinct entries of the ring; all workgroups leave at the same sweep.
+// s + 2, are distinct entries of the ring; all workgroups leave at the same sweep.  A sequential
+// sweep is long: it waits for all to have finished sweep s - 2 and reads that one's residual
+// then (the sweeps after the last one are work for nothing: 10x10 D = 4, eight sweeps, 1136 us
+// a call with the longer look back).
 //
 // Every poll ends after the caller's limit (0.25 s by default), when the network turns out not to be resident as a
 // whole (another process on the device, say): the run's state is then marked PAIR_RUN_BAILED
@@ -679,7 +682,8 @@ __global__ __launch_bounds__(64 * pair_waves(NT), TY == PAIR_F64 && NT == 2 ? 4 
     constexpr int SET = MB + 128;
     double *own = ml0 + 2 * SET;
     const int4 steps = step_list[ri];
-    const bool turns = steps.y == 0;  // one step a sweep, which reads every message anew
+    const bool turns = a.every > 0;  // Jacobi: one step a sweep, which reads every message anew
+    const int lag = turns ? 4 : 2, back = turns ? 5 : 2;
 
     if (tid == 0) verdict = 0;
     if (tid < 128) zero[tid] = zero[SET + tid] = 0.0;
@@ -723,14 +727,14 @@ __global__ __launch_bounds__(64 * pair_waves(NT), TY == PAIR_F64 && NT == 2 ? 4 
     int loaded[2] = {-1, -1};  // version of the incoming message in LDS, per position of the wave
     int stop = 0, s = 1;
     bool leave = false;
-    // sweep s - 1 is counted and the maximum of sweep s goes out (thread 0): a maximum is
-    // stored a sweep before its count, and this wave has settled in between (position 0 is
-    // always there and is updated once a sweep)
+    // the maximum of sweep s goes out (thread 0), and in a Jacobi run sweep s - 1 is counted: a
+    // maximum is stored a sweep before its count, and this wave has settled in between
+    // (position 0 is always there and is updated once a sweep)
     auto report = [&](int s) {
         PairCtrl *c = a.ctrl + (long long)(s - 1) * PAIR_CTRL_LINES + ri % PAIR_CTRL_LINES;
         double m = 0.0;
         for (int k = 0; k < W; ++k) m = fold_max(m, fold_m[k]);
-        if (s > 1)
+        if (turns && s > 1)
             __hip_atomic_fetch_add(&c[-PAIR_CTRL_LINES].cnt, 1u, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_fetch_max(&c->acc, (unsigned long long)__double_as_longlong(m),
@@ -749,20 +753,23 @@ __global__ __launch_bounds__(64 * pair_waves(NT), TY == PAIR_F64 && NT == 2 ? 4 
             if constexpr (!DIRECT) asm volatile("" : "+v"(K.lane), "+v"(K.tid));
             // ---- once a sweep, the last wave: has the run ended, may this sweep's versions be
             // written.  Its loads go ahead of the first poll's, its waits come after.
-            bool look = k == 0 && w == W - 1 && s > 4;
+            bool look = k == 0 && w == W - 1 && s > lag;
             unsigned long long acc = 0ull;
             unsigned int cnt = 0u;
             if (look && lane < PAIR_CTRL_LINES) {
-                const PairCtrl *c = a.ctrl + (long long)(s - 5) * PAIR_CTRL_LINES + lane;
+                const PairCtrl *c = a.ctrl + (long long)(s - lag - 1) * PAIR_CTRL_LINES + lane;
                 cnt = pair_get(&c->cnt);
-                if (s > 5) acc = pair_get(&c[-PAIR_CTRL_LINES].acc);
+                if (turns && s > back) acc = pair_get(&c[-PAIR_CTRL_LINES].acc);
             }
             auto look_back = [&]() {
                 look = false;
-                if (s > 5 && a.tol >= 0.0 && wave_max_v(__longlong_as_double((long long)acc)) < a.tol)
+                if (turns && s > back && a.tol >= 0.0 &&
+                    wave_max_v(__longlong_as_double((long long)acc)) < a.tol)
                     verdict = 1;
-                else if (!pair_finished(a, s - 4, lane, cnt))
+                else if (!pair_finished(a, s - lag, lane, cnt))
                     verdict = 2;
+                else if (!turns && a.tol >= 0.0 && pair_delta(a, s - back, lane) < a.tol)
+                    verdict = 1;
             };
             // ---- the messages this step reads, polled until they are there; a run that has
             // ended writes no more of them
@@ -879,7 +886,13 @@ __global__ __launch_bounds__(64 * pair_waves(NT), TY == PAIR_F64 && NT == 2 ? 4 
             if (!turns) __syncthreads();
         }
         if (leave) break;
-        if (!turns && tid == 0) report(s);
+        if (!turns && tid == 0) {
+            report(s);
+            pair_settle();
+            __hip_atomic_fetch_add(&a.ctrl[(long long)(s - 1) * PAIR_CTRL_LINES +
+                                           ri % PAIR_CTRL_LINES].cnt,
+                                   1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
     __syncthreads();
     if (turns && !verdict && tid == 0) report(a.sweeps);
@@ -888,10 +901,10 @@ __global__ __launch_bounds__(64 * pair_waves(NT), TY == PAIR_F64 && NT == 2 ? 4 
         bool bail = verdict == 2;
         double m = 0.0;
         if (!bail && verdict == 1) {
-            stop = s - 5;
+            stop = s - back;
             m = pair_delta(a, stop, lane);
         } else if (!bail) {
-            if (lane == 0) {
+            if (turns && lane == 0) {
                 pair_settle();
                 __hip_atomic_fetch_add(&a.ctrl[(long long)(a.sweeps - 1) * PAIR_CTRL_LINES +
                                                ri % PAIR_CTRL_LINES].cnt,
@@ -900,7 +913,7 @@ __global__ __launch_bounds__(64 * pair_waves(NT), TY == PAIR_F64 && NT == 2 ? 4 
             // the sweeps the loop has not looked at (sweep t is finished before sweep t + 1)
             if (lead || a.tol >= 0.0) {
                 bail = !pair_finished(a, a.sweeps, lane, 0u);
-                for (int t = max(1, a.sweeps - 4); t <= a.sweeps && !bail && !stop; ++t) {
+                for (int t = max(1, a.sweeps - back + 1); t <= a.sweeps && !bail && !stop; ++t) {
                     m = pair_delta(a, t, lane);
                     if (a.tol >= 0.0 && m < a.tol) stop = t;
                 }
