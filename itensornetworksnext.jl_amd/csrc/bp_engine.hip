@@ -438,6 +438,10 @@ struct bp_context {
     size_t scratch_bytes = 0, h_scratch_bytes = 0;
     hipEvent_t ev_chunk[2] = {nullptr, nullptr};  // chunked copies to the host
 
+    // the small-bond buckets of a sweep beside its large-bond one (made by prepare_sweep)
+    hipStream_t side = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+
     size_t elt() const {
         return dtype == BP_C128 ? sizeof(cplx) : dtype == BP_F64 ? sizeof(double) : sizeof(float);
     }
@@ -1053,7 +1057,23 @@ static int resolve_path(bp_context *c) {
 
 // Allocate whatever workspace the next sweeps need, before any graph capture (no
 // allocation may happen inside a captured region).
+static bool sweep_forks(const bp_context *c) {
+    return c->side && c->vplan_ok && c->dtype == BP_F32 && c->vplan.nv16 >= 256 &&
+           c->vplan.nv >= 256;
+}
+
 static int prepare_sweep(bp_context *c) {
+    // FP32 networks of bond dimensions 9..12 beside ones of up to 8, a chip's worth of vertices
+    // each: the former read their sites from HBM with one workgroup on a CU, the latter are
+    // products and fit beside them (16 networks of D = 4..12: 14.30 ms a call one after the
+    // other, 13.54 like this).  Smaller buckets leave
+    // room anyway and keep one stream (not measured).
+    if (!c->side && c->vplan_ok && c->dtype == BP_F32 && c->vplan.nv16 >= 256 &&
+        c->vplan.nv >= 256) {
+        HIPCHK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+        HIPCHK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
+        HIPCHK(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
+    }
     if (c->dtype == BP_F64) RETCHK(ensure_v64(c));
     const int path = resolve_path(c);
     if (path < 0) return BP_OK;  // reported by sweep_once
@@ -1193,15 +1213,29 @@ static int sweep_once(bp_context *c, const NetCtl &done, bool *folded = nullptr,
     if (path == BP_PATH_VERTEX && c->dtype == BP_F64) {
         RETCHK(v64_sweep(c, (const double *)src, (double *)dst, done, fold));
     } else if (path == BP_PATH_VERTEX || path == BP_PATH_MIXED) {
-        RETCHK(vertex_sweep(&c->vplan, c->stream, c->topo(), c->d_vsites, src, dst, done,
-                            c->d_res_fid, c->d_res_abs, fold));
-        RETCHK(vertex_k3_sweep(&c->vplan, c->stream, c->topo(), src, dst, done,
-                               c->d_res_fid, c->d_res_abs));
-        RETCHK(vertex16_sweep(&c->vplan, c->stream, c->topo(), src, dst, done, c->d_res_fid,
-                              c->d_res_abs));
-        if (vertex_s_sweep(&c->vplan, c->stream, c->topo(), src, dst, done, c->d_res_fid,
-                           c->d_res_abs, fold) != 0)
-            return set_err(BP_ERR_HIP, "small-bond sweep launch failed");
+        const bool fork = sweep_forks(c);
+        const hipStream_t st = fork ? c->side : c->stream;
+        if (fork) {
+            HIPCHK(hipEventRecord(c->ev_fork, c->stream));
+            HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork, 0));
+        }
+        // the large-bond launches go first: theirs are the long ones
+        int rc = vertex16_sweep(&c->vplan, c->stream, c->topo(), src, dst, done, c->d_res_fid,
+                                c->d_res_abs);
+        if (rc == 0)
+            rc = vertex_sweep(&c->vplan, st, c->topo(), c->d_vsites, src, dst, done,
+                              c->d_res_fid, c->d_res_abs, fold);
+        if (rc == 0)
+            rc = vertex_k3_sweep(&c->vplan, st, c->topo(), src, dst, done, c->d_res_fid,
+                                 c->d_res_abs);
+        if (rc == 0)
+            rc = vertex_s_sweep(&c->vplan, st, c->topo(), src, dst, done, c->d_res_fid,
+                                c->d_res_abs, fold);
+        if (fork) {  // joined whatever happened: nothing outlives the sweep on the side stream
+            HIPCHK(hipEventRecord(c->ev_join, c->side));
+            HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
+        }
+        if (rc != 0) return set_err(BP_ERR_HIP, "vertex sweep launch failed");
         HIPCHK(hipGetLastError());
     }
     if (pair && pair_sweep(&c->pair, c->stream, c->d_sites, src, dst, done, c->d_res_fid,
@@ -1333,6 +1367,9 @@ int bp_destroy(bp_context *c) {
     scratch_release(c, 0);
     for (auto &e : c->ev_chunk)
         if (e) (void)hipEventDestroy(e);
+    if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
+    if (c->ev_join) (void)hipEventDestroy(c->ev_join);
+    if (c->side) (void)hipStreamDestroy(c->side);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);

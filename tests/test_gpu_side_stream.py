@@ -1,0 +1,32 @@
+"""FP32 engines whose large-bond bucket (9..12) and small-bond buckets hold 256 vertices or more
+each sweep them on two streams (a fork and a join in every sweep, captured or not).  Every
+network runs the same kernels as in an engine of its own, which has one bucket and one stream:
+the messages, sweeps and deltas agree bit for bit, run after run."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_two_buckets_match_each_alone(pkg, use_graph):
+    print(f"case side stream graph={use_graph}", flush=True)
+    nets = [(pkg.named_grid((16, 17)), 10), (pkg.named_grid((18, 16)), 6),
+            (pkg.heavy_hex_lattice(5, 12), 12), (pkg.heavy_hex_lattice(4, 8), 8)]
+    tops = [pkg.build_topology(g, D, 2) for g, D in nets]
+    sites = [pkg.peps.random_sites(t, 3 + i, scale=pkg.peps.peps_scale(2, D))
+             for i, (t, (_, D)) in enumerate(zip(tops, nets))]
+    kw = {"maxiter": 37, "tol": 1e-5, "use_graph": use_graph}
+    alone = []
+    for t, s in zip(tops, sites):
+        with pkg.Engine(t, s, dtype="f32") as e:
+            e.init_messages("identity")
+            r = e.run(**kw)
+            alone.append((e.messages(), r.sweeps[0], r.delta[0]))
+    with pkg.Engine(pkg.concat_topologies(tops), np.concatenate(sites), dtype="f32") as e:
+        for _ in range(3):
+            e.init_messages("identity")
+            r = e.run(**kw)
+            np.testing.assert_array_equal(e.messages(), np.concatenate([a[0] for a in alone]))
+            np.testing.assert_array_equal(r.sweeps, [a[1] for a in alone])
+            np.testing.assert_array_equal(r.delta, [a[2] for a in alone])
