@@ -1029,8 +1029,8 @@ int pair_plan_build(PairPlan *p, int dtype, int plain, int nv, int nnet, const i
     const size_t esz = dtype == PAIR_F32 ? 4 : dtype == PAIR_C128 ? 16 : 8;
     // Few tile columns leave few waves: share the slices between two more each.  Three columns
     // a half are six waves, which four SIMDs take in two turns; twelve are even, but take the
-    // LDS of two workgroups, so only where the vertices are at most one to a CU (us a sweep at
-    // 16x16 D = 6: 19 against 14).
+    // LDS of two workgroups, so only where the vertices are at most one to a CU (us a sweep of
+    // a run at 16x16 D = 6: 18.4 against 14.9).
     p->split = maxd >= 2 && (p->nt <= 2 || (p->nt == 3 && p->recs.size() <= 256)) ? 2 : 1;
     p->waves = 2 * p->nt * p->split;
     int slice = 0, env = 0;
