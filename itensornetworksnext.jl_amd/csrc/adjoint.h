@@ -264,8 +264,8 @@ __global__ void k_expect_ratio(const double *num, const double *den, int n, doub
 }
 
 // ---- cotangent through the sum normalisation f = g / S:  gg = (lam - <lam, f>) / S
-template <typename T>
-__global__ void k_adj_gg(DevTopo tp, const T *lam, const T *G, const double *S, T *gg) {
+template <typename T, typename TO = T>
+__global__ void k_adj_gg(DevTopo tp, const T *lam, const T *G, const double *S, TO *gg) {
     const int q = blockIdx.x;
     if (q >= tp.nports) return;
     const long long mo = tp.msg_off[q];
@@ -277,7 +277,7 @@ __global__ void k_adj_gg(DevTopo tp, const T *lam, const T *G, const double *S, 
     dot = wave_sum(dot);  // one wave per slot
     for (int i = threadIdx.x; i < len; i += blockDim.x) {
         const double l = (double)lam[mo + i];
-        gg[mo + i] = (T)(s != 0.0 ? (l - dot / s) / s : l);
+        gg[mo + i] = (TO)(s != 0.0 ? (l - dot / s) / s : l);
     }
 }
 

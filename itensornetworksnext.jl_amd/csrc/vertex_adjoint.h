@@ -131,20 +131,36 @@ __device__ __forceinline__ VdSlots vd_slots(const int4 *vin, const int4 *vout, c
 // the scalar O[s'][s] on each, so a launch of shift c pairs slice w of wave w with slice
 // ks = (w + c) % NS and puts the scalars on the overrides and on the value term; NS launches
 // cover the operator.  The terms without an operator ride in the launch of shift 0.
+//
+// Operators, coefficients and sums over slices stay in FP64, rounded once to the products'
+// FP32 operand, so that what an operator shares with the identity cancels in them.  Rounded to
+// FP32 each (same time, 1.34 ms a call at 16 x 16, D = 6): the energy of 1000 + h on every
+// vertex of 11 x 13, D = 7 was off by 1.5e-9 of it and its gradient by 1.6e-4, now 5e-13 and
+// 1.4e-7 (the generic kernels, FP64 sums over an FP32 op.A: 3e-10 and 2.3e-4).
 struct VdOps {
     const double *ov = nullptr;   // per vertex, ld x ld (null: no vertex operators)
     const double *oq = nullptr;   // per out-slot, ld x ld (null: none)
     int ld = -1, shift = 0;
-    const float *wo = nullptr;    // overrides of the operator-inserted edge terms
+    const double *w = nullptr;    // overrides of the terms without an operator,
+    const double *wo = nullptr;   // and of the operator-inserted edge terms
     const double *cv1 = nullptr;  // value coefficients of the vertex operators
-    float *out = nullptr;         // forward opens: operator-inserted messages,
-    double *z = nullptr;          // and vertex scalars (shift > 0 adds to both)
+    double *g = nullptr;          // forward opens: messages (shift 0) and operator-inserted
+    double *out = nullptr;        // ones, and the
+    double *z = nullptr;          // operator-inserted scalars (shift > 0 adds to these)
 };
 
 // O[s'][s] of matrix `i`, with bra and ket exchanged for the ket-side derivative
-__device__ __forceinline__ float vd_op(const double *o, int ld, long long i, int sp, int s,
-                                       int trans) {
-    return (float)o[i * ld * ld + (trans ? s * ld + sp : sp * ld + s)];
+__device__ __forceinline__ double vd_op(const double *o, int ld, long long i, int sp, int s,
+                                        int trans) {
+    return o[i * ld * ld + (trans ? s * ld + sp : sp * ld + s)];
+}
+
+// value coefficient of vertex vid in the slice pair (sp, s) of this launch
+__device__ __forceinline__ float vd_op_cv(const VdOps &ops, const double *cv0, int vid, int sp,
+                                          int s, int trans) {
+    double c = ops.shift == 0 && cv0 ? cv0[vid] : 0.0;
+    if (ops.ov) c += ops.cv1[vid] * vd_op(ops.ov, ops.ld, vid, sp, s, trans);
+    return (float)c;
 }
 
 // With Gn != nullptr, W holds lambda and the override is its cotangent through the sum
@@ -163,7 +179,7 @@ __device__ __forceinline__ void vd_load_mats(const float *msgs, const float *W, 
                                              const VdOps *ops = nullptr) {
     const int w = threadIdx.x >> 6, e = threadIdx.x & 63;
     const int a = trans ? (e & 7) : (e >> 3), b = trans ? (e >> 3) : (e & 7);
-    if (ops && W) {  // this wave's overrides
+    if (ops && ops->w) {  // this wave's overrides
         const int ks = (w + ops->shift) % NS;
         float *ws = wsm + w * 256;
 #pragma unroll
@@ -171,10 +187,10 @@ __device__ __forceinline__ void vd_load_mats(const float *msgs, const float *W, 
             const int D = sl.dims[j];
             const bool have = sl.outs[j] >= 0 && a < D && b < D;
             const long long off = sl.outo[j] + a * D + b;
-            float x = have && ops->shift == 0 ? W[off] : 0.f;
+            double x = have && ops->shift == 0 ? ops->w[off] : 0.0;
             if (have && ops->oq)
                 x += vd_op(ops->oq, ops->ld, sl.outs[j], w, ks, trans) * ops->wo[off];
-            ws[j * 64 + e] = x;
+            ws[j * 64 + e] = (float)x;
         }
     }
     if (W && W2) {
@@ -293,12 +309,9 @@ void k_vd_msg(const float *__restrict__ vsites, const float *__restrict__ msgs,
     float *part = wsm0 + NS * 4 * 64;
     const VdSlots sl = vd_slots(vin, vout, vdim, msg_off, u);
     const int vid = vlist[u];
-    float cv = (float)(cv_vertex ? cv_vertex[vid] : cv_const);
-    if constexpr (OPM && HASW) {
-        if (ops.shift != 0) cv = 0.f;
-        if (ops.ov)
-            cv += (float)ops.cv1[vid] * vd_op(ops.ov, ops.ld, vid, w, (w + ops.shift) % NS, 0);
-    }
+    float cv;
+    if constexpr (OPM && HASW) cv = vd_op_cv(ops, cv_vertex, vid, w, (w + ops.shift) % NS, 0);
+    else cv = (float)(cv_vertex ? cv_vertex[vid] : cv_const);
     vd_load_mats<NS>(msgs, HASW ? W : nullptr, sl, 0, msm, wsm0, Gn, Sn, HASW ? W2 : nullptr,
                      OPM ? &ops : nullptr);
     const float *wsm = wsm0 + (W2 || OPM ? w * 256 : 0);
@@ -403,28 +416,34 @@ void k_vd_msg(const float *__restrict__ vsites, const float *__restrict__ msgs,
             x += v;
             xz += s == 1 ? -v : v;
         }
-        if (j == 0 && z_out) {
+        if (j == 0 && z_out && !OPM) {
             const double z = wave_sum_v((double)x * (double)msm[lane]);
             if (lane == 0) z_out[vid] = z;
         }
-        if constexpr (OPM && !HASW) {  // operator-inserted messages and vertex scalars
-            float xo = 0.f, xv = 0.f;
+        if constexpr (OPM && !HASW) {  // messages and vertex scalars with and without operator
+            double xi = 0.0, xo = 0.0, xv = 0.0;
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                const float v = part[(s * 4 + j) * 64 + lane];
+                const double v = (double)part[(s * 4 + j) * 64 + lane];
                 const int kt = (s + ops.shift) % NS;
+                xi += v;
                 if (ops.oq && sl.outs[j] >= 0)
                     xo += vd_op(ops.oq, ops.ld, sl.outs[j], s, kt, 0) * v;
                 if (ops.ov && j == 0) xv += vd_op(ops.ov, ops.ld, vid, s, kt, 0) * v;
             }
             if (j == 0 && ops.ov) {
-                const double z = wave_sum_v((double)xv * (double)msm[lane]);
+                const double z = wave_sum_v(xv * (double)msm[lane]);
                 if (lane == 0) ops.z[vid] = z + (ops.shift ? ops.z[vid] : 0.0);
+            }
+            if (j == 0 && z_out) {
+                const double z = wave_sum_v(xi * (double)msm[lane]);
+                if (lane == 0) z_out[vid] = z;
             }
             const int Dj = sl.dims[j];
             if (ops.oq && sl.outs[j] >= 0 && (lane >> 3) < Dj && (lane & 7) < Dj) {
-                float *p = ops.out + sl.outo[j] + (lane >> 3) * Dj + (lane & 7);
-                *p = xo + (ops.shift ? *p : 0.f);
+                const long long at = sl.outo[j] + (lane >> 3) * Dj + (lane & 7);
+                if (ops.shift == 0) ops.g[at] = xi;
+                ops.out[at] = xo + (ops.shift ? ops.out[at] : 0.0);
             }
         }
         // lane = entry (a, a') of the padded 8 x 8 block; real below the bond dimension
@@ -490,12 +509,10 @@ void k_vd_site(const float *__restrict__ vsites, const float *__restrict__ msgs,
     float *wsm0 = msm + 4 * 64;
     const VdSlots sl = vd_slots(vin, vout, vdim, msg_off, u);
     const int vid = vlist[u];
-    float cv = (float)(cv_vertex ? cv_vertex[vid] : cv_const);
     const int ks = OPM ? (w + ops.shift) % NS : op == OP_X ? (w ^ 1) : w;
-    if constexpr (OPM) {
-        if (ops.shift != 0) cv = 0.f;
-        if (ops.ov) cv += (float)ops.cv1[vid] * vd_op(ops.ov, ops.ld, vid, w, ks, trans);
-    }
+    float cv;
+    if constexpr (OPM) cv = vd_op_cv(ops, cv_vertex, vid, w, ks, trans);
+    else cv = (float)(cv_vertex ? cv_vertex[vid] : cv_const);
     vd_load_mats<NS>(msgs, HASW ? W : nullptr, sl, trans, msm, wsm0, nullptr, nullptr,
                      HASW ? W2 : nullptr, OPM ? &ops : nullptr);
     const float *wsm = wsm0 + (W2 || OPM ? w * 256 : 0);
@@ -605,18 +622,19 @@ __global__ void k_vd_vertex_terms(DevTopo tp, const float *G, const float *GX, c
 }
 
 // dst[q] = coef[q] * src[rev q]  (+ dst[q] when acc)
-__global__ void k_vd_scale_rev(DevTopo tp, const double *coef, const float *src, float *dst,
-                               int acc) {
+template <typename T>
+__global__ void k_vd_scale_rev(DevTopo tp, const double *coef, const T *src, T *dst, int acc) {
     const int q = blockIdx.x;
     if (q >= tp.nports) return;
     const long long mo = tp.msg_off[q], ro = tp.msg_off[tp.port_rev[q]];
     const int len = (int)(tp.msg_off[q + 1] - mo);
-    const float c = (float)coef[q];
+    const T c = (T)coef[q];
     for (int i = threadIdx.x; i < len; i += blockDim.x)
-        dst[mo + i] = c * src[ro + i] + (acc ? dst[mo + i] : 0.f);
+        dst[mo + i] = c * src[ro + i] + (acc ? dst[mo + i] : T(0));
 }
 
-__global__ void k_vd_axpy(const float *a, float *b, long long n) {
+template <typename T>
+__global__ void k_vd_axpy(const T *a, T *b, long long n) {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
          i += (long long)gridDim.x * blockDim.x)
         b[i] += a[i];
@@ -674,7 +692,7 @@ static int vd_msg(const VdCtx &c, const float *msgs, const float *W, int op, dou
     const VertexPlan &p = *c.vp;
     const dim3 grid(p.nv), block(64 * p.d);
     const size_t lds = vd_msg_lds(p.d);
-    const bool hw = W != nullptr;
+    const bool hw = W || (ops && ops->w);
     if (op != OP_I && p.d != 2) return 4;  // X and Z pair the two slices of a qubit
     if (W2 && (p.d != 2 || op != OP_I || !W || Gn)) return 4;
     if (out_z && (p.d != 2 || op != OP_I || W || to_in)) return 4;
@@ -713,7 +731,7 @@ static int vd_site(const VdCtx &c, const float *msgs, const float *W, int trans,
     const VertexPlan &p = *c.vp;
     const dim3 grid(p.nv), block(64 * p.d);
     const size_t lds = vd_site_lds(p.d, cv_swap != nullptr);
-    const bool hw = W != nullptr;
+    const bool hw = W || (ops && ops->w);
     if (op != OP_I && p.d != 2) return 4;
     if ((W2 || cv_swap) && (p.d != 2 || op != OP_I)) return 4;
     if (W2 && !W) return 4;
@@ -881,9 +899,9 @@ static int vadj_tfim(AdjointScratch *s, const VdCtx &c, int ne, const float *msg
     if (np > 0) {
         hipLaunchKernelGGL(k_vd_vertex_terms, dim3(np), dim3(64), 0, c.st, tp, (const float *)G,
                            (const float *)GX, (const double *)cv0, (const double *)cv1, dm);
-        hipLaunchKernelGGL(k_vd_scale_rev, dim3(np), dim3(64), 0, c.st, tp, (const double *)cq0,
+        hipLaunchKernelGGL(k_vd_scale_rev<float>, dim3(np), dim3(64), 0, c.st, tp, (const double *)cq0,
                            (const float *)G, WI, 0);
-        hipLaunchKernelGGL(k_vd_scale_rev, dim3(np), dim3(64), 0, c.st, tp, (const double *)cq1,
+        hipLaunchKernelGGL(k_vd_scale_rev<float>, dim3(np), dim3(64), 0, c.st, tp, (const double *)cq1,
                            (const float *)GZ, WZ, 0);
         // the I- and Z-inserted edge terms in one launch (overrides WI + sigma WZ per slice)
         VD_RET(vd_msg(c, msgs, WI, OP_I, 0.0, nullptr, 1, dm, dm, nullptr, nullptr, nullptr,
@@ -904,7 +922,7 @@ static int vadj_tfim(AdjointScratch *s, const VdCtx &c, int ne, const float *msg
     if (np > 0) {
         hipLaunchKernelGGL(k_adj_gg<float>, dim3(np), dim3(64), 0, c.st, tp, (const float *)lam,
                            (const float *)G, (const double *)S, gg);
-        hipLaunchKernelGGL(k_vd_axpy, dim3(cblocks), dim3(256), 0, c.st, (const float *)gg, WI,
+        hipLaunchKernelGGL(k_vd_axpy<float>, dim3(cblocks), dim3(256), 0, c.st, (const float *)gg, WI,
                            nmsg);
     }
     const float *wi = np > 0 ? WI : nullptr, *wz = np > 0 ? WZ : nullptr;
@@ -944,7 +962,8 @@ static int vadj_local(AdjointScratch *s, const VdCtx &c, int ne, const float *ms
     double *z = (double *)s->alloc(sizeof(double) * nv);
     double *zo = (double *)s->alloc(sizeof(double) * nv);
     float *G = (float *)s->alloc(sizeof(float) * nmsg);
-    float *GO = (float *)s->alloc(sizeof(float) * nmsg);
+    double *G64 = (double *)s->alloc(sizeof(double) * nmsg);
+    double *GO = (double *)s->alloc(sizeof(double) * nmsg);
     double *S = (double *)s->alloc(sizeof(double) * std::max(np, 1));
     double *nz = (double *)s->alloc(sizeof(double) * std::max(ne, 1));
     double *dd = (double *)s->alloc(sizeof(double) * std::max(ne, 1));
@@ -955,8 +974,8 @@ static int vadj_local(AdjointScratch *s, const VdCtx &c, int ne, const float *ms
     double *ev = (double *)s->alloc(sizeof(double) * nv);
     double *eq = (double *)s->alloc(sizeof(double) * std::max(np, 1));
     double *esum = (double *)s->alloc(sizeof(double));
-    if (!dopv || !dopa || !dopb || !dopq || !z || !zo || !G || !GO || !S || !nz || !dd || !cv1 ||
-        !cv0 || !cq1 || !cq0 || !ev || !eq || !esum)
+    if (!dopv || !dopa || !dopb || !dopq || !z || !zo || !G || !G64 || !GO || !S || !nz || !dd ||
+        !cv1 || !cv0 || !cq1 || !cq0 || !ev || !eq || !esum)
         VD_RET(5);
     if ((hv && hipMemcpyAsync(dopv, ops_v, blk * nv, hipMemcpyHostToDevice, c.st) != hipSuccess) ||
         (he && (hipMemcpyAsync(dopa, ops_first, blk * ne, hipMemcpyHostToDevice, c.st) !=
@@ -971,6 +990,7 @@ static int vadj_local(AdjointScratch *s, const VdCtx &c, int ne, const float *ms
     om.ov = hv ? dopv : nullptr;
     om.oq = he ? dopq : nullptr;
     om.ld = ld;
+    om.g = G64;
     om.out = GO;
     om.z = zo;
     // forward opens: G, its sums and Z_u beside the operator-inserted ones
@@ -981,8 +1001,8 @@ static int vadj_local(AdjointScratch *s, const VdCtx &c, int ne, const float *ms
                       nullptr, 0, nullptr, 0.0, -1, nullptr, nullptr, &om));
     }
     if (he)
-        hipLaunchKernelGGL(k_adj_edge_dots<float>, dim3((np + 255) / 256), dim3(256), 0, c.st, tp,
-                           (const float *)G, (const float *)GO, nz, dd);
+        hipLaunchKernelGGL(k_adj_edge_dots<double>, dim3((np + 255) / 256), dim3(256), 0, c.st, tp,
+                           (const double *)G64, (const double *)GO, nz, dd);
     const int nmax = std::max(nv, np);
     hipLaunchKernelGGL(k_local_coefs, dim3((nmax + 255) / 256), dim3(256), 0, c.st, tp, hv ? 1 : 0,
                        he ? 1 : 0, (const double *)z, (const double *)zo, (const double *)nz,
@@ -999,11 +1019,11 @@ static int vadj_local(AdjointScratch *s, const VdCtx &c, int ne, const float *ms
     }
     const bool direct = go.dev && !go.dev_f64;
     float *dm = (float *)s->alloc(sizeof(float) * nmsg);
-    float *WI = (float *)s->alloc(sizeof(float) * nmsg);
-    float *WO = (float *)s->alloc(sizeof(float) * nmsg);
+    double *WI = (double *)s->alloc(sizeof(double) * nmsg);
+    double *WO = (double *)s->alloc(sizeof(double) * nmsg);
     float *lbuf[2] = {(float *)s->alloc(sizeof(float) * nmsg),
                       (float *)s->alloc(sizeof(float) * nmsg)};
-    float *gg = (float *)s->alloc(sizeof(float) * nmsg);
+    double *gg = (double *)s->alloc(sizeof(double) * nmsg);
     float *da = direct ? (float *)go.dev : (float *)s->alloc(sizeof(float) * nsite);
     unsigned long long *acc = (unsigned long long *)s->alloc(sizeof(unsigned long long) * 384 +
                                                              sizeof(VdLoopState));
@@ -1013,21 +1033,22 @@ static int vadj_local(AdjointScratch *s, const VdCtx &c, int ne, const float *ms
         VD_RET(5);
     if (hipMemsetAsync(da, 0, sizeof(float) * nsite, c.st) != hipSuccess ||
         hipMemsetAsync(dm, 0, sizeof(float) * nmsg, c.st) != hipSuccess ||
-        hipMemsetAsync(WI, 0, sizeof(float) * nmsg, c.st) != hipSuccess)
+        hipMemsetAsync(WI, 0, sizeof(double) * nmsg, c.st) != hipSuccess)
         VD_RET(2);
     // explicit dE/dm: vertex terms (value coefficients cv0 and cv1 O_v), edge terms (overrides
     // cq0 G and cq1 O_q GO of the other side)
     if (he) {
-        hipLaunchKernelGGL(k_vd_scale_rev, dim3(np), dim3(64), 0, c.st, tp, (const double *)cq0,
-                           (const float *)G, WI, 0);
-        hipLaunchKernelGGL(k_vd_scale_rev, dim3(np), dim3(64), 0, c.st, tp, (const double *)cq1,
-                           (const float *)GO, WO, 0);
+        hipLaunchKernelGGL(k_vd_scale_rev<double>, dim3(np), dim3(64), 0, c.st, tp,
+                           (const double *)cq0, (const double *)G64, WI, 0);
+        hipLaunchKernelGGL(k_vd_scale_rev<double>, dim3(np), dim3(64), 0, c.st, tp,
+                           (const double *)cq1, (const double *)GO, WO, 0);
     }
+    om.w = np > 0 ? WI : nullptr;
     om.wo = WO;
     om.cv1 = cv1;
     if (np > 0)
         for (om.shift = 0; om.shift < ns; ++om.shift)
-            VD_RET(vd_msg(c, msgs, WI, OP_I, 0.0, cv0, 1, dm, dm, nullptr, nullptr, nullptr,
+            VD_RET(vd_msg(c, msgs, nullptr, OP_I, 0.0, cv0, 1, dm, dm, nullptr, nullptr, nullptr,
                           nullptr, nullptr, nullptr, 0, nullptr, 0.0, -1, nullptr, nullptr, &om));
     const int cblocks = (int)std::max<long long>(1, std::min<long long>((nmsg + 255) / 256, 4096));
     hipLaunchKernelGGL(k_adj_axpy_copy<float>, dim3(cblocks), dim3(256), 0, c.st,
@@ -1036,16 +1057,15 @@ static int vadj_local(AdjointScratch *s, const VdCtx &c, int ne, const float *ms
     VD_RET(vadj_sweeps(c, msgs, G, S, dm, lbuf, acc, lst, adj_tol, adj_maxiter, &hst));
     // grad = dE/dA + J_A^T lambda: the overrides without an operator take the cotangent too
     if (np > 0) {
-        hipLaunchKernelGGL(k_adj_gg<float>, dim3(np), dim3(64), 0, c.st, tp,
+        hipLaunchKernelGGL((k_adj_gg<float, double>), dim3(np), dim3(64), 0, c.st, tp,
                            (const float *)lbuf[hst.it & 1], (const float *)G, (const double *)S,
                            gg);
-        hipLaunchKernelGGL(k_vd_axpy, dim3(cblocks), dim3(256), 0, c.st, (const float *)gg, WI,
-                           nmsg);
+        hipLaunchKernelGGL(k_vd_axpy<double>, dim3(cblocks), dim3(256), 0, c.st,
+                           (const double *)gg, WI, nmsg);
     }
     for (int tr = 0; tr < 2; ++tr)
         for (om.shift = 0; om.shift < ns; ++om.shift)
-            VD_RET(vd_site(c, msgs, np > 0 ? WI : nullptr, tr, OP_I, 0.0, cv0, da, nullptr,
-                           nullptr, &om));
+            VD_RET(vd_site(c, msgs, nullptr, tr, OP_I, 0.0, cv0, da, nullptr, nullptr, &om));
     if (!direct) VD_RET(adj_emit_grad(c.st, (const float *)da, g64, nsite, go));
     double hE = 0.0;
     if (hipMemcpyAsync(&hE, esum, sizeof(double), hipMemcpyDeviceToHost, c.st) != hipSuccess)

@@ -46,3 +46,29 @@ def test_against_fp64(pkg, orc, shape, D, d, terms, ld):
     assert np.max(np.abs(g - gw)) < 1e-4 * scale
     np.testing.assert_array_equal(dev, g.astype(np.float32))
     assert abs(E - Ew) < 1e-4 * max(abs(Ew), 1.0)
+
+
+@pytest.mark.parametrize("shape,D,d", [((4, 4), 5, 2), ((3, 4), 6, 3), ((3, 3), 8, 2), ((1, 4), 6, 2)])
+def test_multiples_of_the_identity(pkg, shape, D, d):
+    """O_v = c, A_e B_e = c: the energy is c per term and its gradient zero whatever the tensors
+    are, so what is left is the rounding of operators, coefficients and sums over slices.  In
+    FP64 that is some 1e-15 of c (sums of at most 64 d terms of the same FP32 products above and
+    below the fraction; 1e-12 is asserted), with c rounded to FP32 1e-8 of it."""
+    print(f"case local identity {shape} D={D} d={d}", flush=True)
+    t = pkg.build_topology(pkg.named_grid(shape), D, d)
+    s = pkg.peps.random_sites(t, 33, scale=pkg.peps.peps_scale(d, D))
+    c = 1000.1
+    one = lambda n, x: np.broadcast_to(x * np.eye(d), (n, d, d)).copy()  # noqa: E731
+    with pkg.Engine(t, s, dtype="f32") as e:
+        e.init_messages("identity")
+        e.run(maxiter=300, tol=1e-13)
+        assert e.path() == "vertex"
+        kw = {"grad": True, "adj_tol": 1e-6, "adj_maxiter": 50}
+        Ev, gv, _, _ = e.local_energy(one(t.nv, c), **kw)
+        Ee, ge, _, _ = e.local_energy(None, one(t.ne, c), one(t.ne, 1.0), **kw)
+        h = np.random.default_rng(34).standard_normal((t.nv, d, d))
+        size = np.max(np.abs(e.local_energy(h, **kw)[1])) if d > 1 else 1.0
+    assert abs(Ev - c * t.nv) <= 1e-12 * c * t.nv
+    assert abs(Ee - c * t.ne) <= 1e-12 * c * t.ne
+    assert np.max(np.abs(gv)) <= 1e-10 * c * size
+    assert np.max(np.abs(ge)) <= 1e-10 * c * size
