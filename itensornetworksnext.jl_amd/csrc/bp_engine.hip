@@ -2690,29 +2690,24 @@ static int pair_zv(bp_context *c, const void *sites, const void *m, bool *done) 
 }
 
 // Vertex scalars of FP32 contexts whose vertices are all on the vertex kernels, each bucket by
-// its own kernel: Z_u = <G_{u, port 0}, m_in,0> from the unnormalised message out of port 0.
-// 65 536 vertices at D = 3: 937 us on the generic kernel.
+// a kernel of its own: ports absorbed in FP32, the last contraction in FP64, as in the generic
+// kernel (65 536 vertices at D = 3: 937 us there).
 static int vertex_zv(bp_context *c, const float *m, bool *done) {
     *done = false;
     const VertexPlan &p = c->vplan;
     if (c->dtype != BP_F32 || !c->vplan_ok || !p.all || c->path == BP_PATH_GENERIC ||
         (p.nv > 0 && !c->d_vsites))
         return BP_OK;
-    if (p.nv16 > 0)  // the large-bond finisher leaves out padded ports, port 0 included
-        for (int u = 0; u < c->nv; ++u)
-            if (c->port_off[u] == c->port_off[u + 1]) return BP_OK;
     if (p.nv > 0) {
         if (vd_set_limits(p.d) != 0) return BP_OK;
         const VdCtx vc{&c->vplan, c->stream, c->topo(), (const float *)c->d_vsites};
-        if (vd_msg(vc, m, nullptr, OP_I, 1.0, nullptr, 0, nullptr, nullptr, nullptr, nullptr,
-                   c->d_zv) != 0)
+        if (vd_scalars(vc, m, c->d_zv) != 0)
             return set_err(BP_ERR_HIP, "vertex scalar launch failed");
     }
     const NetCtl off = make_ctl(c, false);
     if (vertex_s_sweep(&c->vplan, c->stream, c->topo(), m, nullptr, off, nullptr, nullptr,
                        SweepFold{}, c->d_zv) != 0 ||
-        vertex16_sweep(&c->vplan, c->stream, c->topo(), m, nullptr, off, nullptr, nullptr,
-                       c->d_zv) != BP_OK)
+        vertex16_scalars(&c->vplan, c->stream, c->topo(), m, c->d_zv) != 0)
         return set_err(BP_ERR_HIP, "vertex scalar launch failed");
     *done = true;
     return BP_OK;

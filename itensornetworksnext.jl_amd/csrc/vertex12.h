@@ -252,6 +252,23 @@ __device__ __forceinline__ void v12_pair(float *S, float *red, const float *src,
     }
 }
 
+// Incoming messages as MFMA A operands: lane l holds m[4 kc + l/16][l%16] (zero beyond the bond
+// dimension; padded ports are never absorbed).
+__device__ __forceinline__ void v12_load_am(const float *mold, const long long *msg_off,
+                                            const int (&ins)[4], const int (&dims)[4],
+                                            float (&Am)[4][3]) {
+    const int lane = threadIdx.x & 63, n = lane & 15, kk = lane >> 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int kc = 0; kc < 3; ++kc) {
+            const int k = 4 * kc + kk, D = dims[j];
+            Am[j][kc] = (ins[j] >= 0 && k < D && n < D) ? mold[msg_off[ins[j]] + k * D + n]
+                                                         : 0.f;
+        }
+    }
+}
+
 // grid: items x d (one workgroup per slice of items i0 .. i0 + grid / d - 1), 64 DP threads.
 // vsites_n / vsites_w hold those items' padded slices from item i0 on.  part[((item * d + s)
 // * 4 + j) * 256 + a * 16 + a'] receives slice s's unnormalised out_j (the layout
@@ -267,31 +284,76 @@ __global__ __launch_bounds__(64 * DP) void k_vertex_d12(
     float *S = v12sm;
     float *red = v12sm + C::LDS_ELEMS;
     const int il = blockIdx.x / d, s = blockIdx.x - il * d, item = i0 + il;
-    const int lane = threadIdx.x & 63;
-    const int n = lane & 15, kk = lane >> 4;
     if (ctl.enabled && ctl.done[vnet[item]]) return;  // k_v16_finish carries the messages
     const int4 vi = vin[item], vo = vout[item], vd = vdim[item];
     const int ins[4] = {vi.x, vi.y, vi.z, vi.w};
     const int outs[4] = {vo.x, vo.y, vo.z, vo.w};
     const int dims[4] = {vd.x, vd.y, vd.z, vd.w};
-    // incoming messages as MFMA A operands: lane l holds m[4 kc + l/16][l%16] (zero beyond
-    // the bond dimension; padded ports are never absorbed)
     float Am[4][3];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-        for (int kc = 0; kc < 3; ++kc) {
-            const int k = 4 * kc + kk, D = dims[j];
-            Am[j][kc] = (ins[j] >= 0 && k < D && n < D) ? mold[msg_off[ins[j]] + k * D + n]
-                                                         : 0.f;
-        }
-    }
+    v12_load_am(mold, msg_off, ins, dims, Am);
     const long long so = ((long long)il * d + s) * C::ELEMS;
     const float *src = vsites_n + so, *src_w = vsites_w + so;
     float *dst = part + ((long long)item * d + s) * 4 * 256;
     // E23 serves outgoing ports 0 (absorb 1) and 1 (absorb 0); E01 serves 2 and 3
     v12_pair<DP, 0, 1, 2, 3, 1, 0>(S, red, src, src_w, dst, ins, outs, Am);
     v12_pair<DP, 2, 3, 0, 1, 3, 2>(S, red, src, src_w, dst, ins, outs, Am);
+}
+
+// Vertex scalars, slice by slice (grid and items as k_vertex_d12): every port absorbed in LDS,
+// then <E, A> in FP64, part[item * d + s], with the generic kernel's roundings.  4 mode products
+// and no open, bound as the sweep by the slices' way through LDS; from the sweep kernels' own
+// message out of port 0 (8 products, 4 opens, the last contraction in FP32) a call on 16
+// networks of D = 4..12 took 13.65 ms against 12.94.
+template <int DP>
+__global__ __launch_bounds__(64 * DP) void k_v12_scalar(
+    const float *__restrict__ vsites_n, const float *__restrict__ msgs,
+    const int4 *__restrict__ vin, const int4 *__restrict__ vdim,
+    const long long *__restrict__ msg_off, int d, int i0, double *__restrict__ part) {
+    using C = VQ<DP>;
+    extern __shared__ __align__(16) float v12sm[];
+    float *S = v12sm;
+    static_assert(C::LDS_ELEMS % 2 == 0, "doubles follow the slice");
+    double *red = reinterpret_cast<double *>(v12sm + C::LDS_ELEMS);
+    const int il = blockIdx.x / d, s = blockIdx.x - il * d, item = i0 + il;
+    const int4 vi = vin[item], vd = vdim[item];
+    const int ins[4] = {vi.x, vi.y, vi.z, vi.w};
+    const int dims[4] = {vd.x, vd.y, vd.z, vd.w};
+    float Am[4][3];
+    v12_load_am(msgs, msg_off, ins, dims, Am);
+    const float *src = vsites_n + ((long long)il * d + s) * C::ELEMS;
+    v12_load_slice<DP>(S, src);
+    __syncthreads();
+    v12_mode_if<DP, 0>(S, ins, Am);
+    v12_mode_if<DP, 1>(S, ins, Am);
+    v12_mode_if<DP, 2>(S, ins, Am);
+    v12_mode_if<DP, 3>(S, ins, Am);
+    double z = 0.0;
+    const float4 *g = reinterpret_cast<const float4 *>(src);
+    for (int c = threadIdx.x; c < C::ELEMS / 4; c += 64 * C::NW) {
+        const float4 v = g[c];
+        const int e = 4 * c;
+        const int row = e / (DP * DP), col = e - DP * DP * row;  // row = DP p0 + p1
+        const int p0 = row / DP, p1 = row - DP * p0;
+        const float *x = S + p0 * C::S0 + p1 * C::S1 + col;
+        z += (double)x[0] * (double)v.x + (double)x[1] * (double)v.y +
+             (double)x[2] * (double)v.z + (double)x[3] * (double)v.w;
+    }
+    z = wave_sum_v(z);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = z;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < C::NW; ++w) z += red[w];
+        part[(long long)item * d + s] = z;
+    }
+}
+
+__global__ void k_v16_scalar_sum(const double *__restrict__ part, const int *__restrict__ vlist,
+                                 int nitems, int d, double *__restrict__ zv) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nitems) return;
+    double z = 0.0;
+    for (int s = 0; s < d; ++s) z += part[(long long)i * d + s];
+    zv[vlist[i]] = z;
 }
 
 // Padded FP32 site entries of DP-side items: vsites_n[item][s][p0][p1][p2][p3] (DP each)
@@ -531,6 +593,39 @@ __global__ __launch_bounds__(64 * V3_WAVES) void k_vertex_k3(
         v3_mode_if<DP, 1>(S, ins, Am);
         v3_open_store<DP, 2>(S, pre, dst);
     }
+}
+
+// Vertex scalars of degree <= 3 items (grid as k_vertex_k3): part[(item0 + i) * d + s].
+template <int DP>
+__global__ __launch_bounds__(64 * V3_WAVES) void k_v3_scalar(
+    const float *__restrict__ vs3, const float *__restrict__ msgs, const int4 *__restrict__ vin,
+    const int4 *__restrict__ vdim, const long long *__restrict__ msg_off, int d, int item0,
+    int nitems, double *__restrict__ part) {
+    using C = V3<DP>;
+    __shared__ float v3sm[V3_WAVES * C::LDS];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int slice = blockIdx.x * V3_WAVES + w;
+    if (slice >= nitems * d) return;  // uniform over the wave; no workgroup barriers below
+    const int i = slice / d, s = slice - i * d;
+    const int item = item0 + i;
+    float *S = v3sm + w * C::LDS;
+    const int4 vi = vin[item], vd = vdim[item];
+    const int ins[4] = {vi.x, vi.y, vi.z, -1};
+    const int dims[4] = {vd.x, vd.y, vd.z, 1};
+    float Am[4][3];
+    v12_load_am(msgs, msg_off, ins, dims, Am);
+    const float *src = vs3 + ((long long)i * d + s) * 3 * C::ELEMS;  // port 0 first: natural
+    v3_load_slice<DP>(S, src);
+    v3_mode_if<DP, 0>(S, ins, Am);
+    v3_mode_if<DP, 1>(S, ins, Am);
+    v3_mode_if<DP, 2>(S, ins, Am);
+    double z = 0.0;
+    for (int e = lane; e < C::ELEMS; e += 64) {
+        const int p0 = e / (DP * DP), rem = e - DP * DP * p0;
+        z += (double)S[p0 * C::S0 + rem] * (double)src[e];
+    }
+    z = wave_sum_v(z);
+    if (lane == 0) part[(long long)item * d + s] = z;
 }
 
 // Site copies of degree <= 3 items: vs3[(i * d + s) * 3 + O][a'][x][y], port O first, then

@@ -367,8 +367,7 @@ __global__ __launch_bounds__(256) void k_v16_finish(
     const float *__restrict__ part, const float *__restrict__ mold, float *__restrict__ mnew,
     const int4 *__restrict__ vout, const int4 *__restrict__ vdim, const int *__restrict__ vnet,
     const long long *__restrict__ msg_off, NetCtl ctl, int d, double *__restrict__ res_fid,
-    double *__restrict__ res_abs, const int4 *__restrict__ vin = nullptr,
-    const int *__restrict__ vlist = nullptr, double *__restrict__ zv = nullptr) {
+    double *__restrict__ res_abs) {
     const int item = blockIdx.x;
     const int j = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int4 vo = vout[item], vd = vdim[item];
@@ -391,19 +390,6 @@ __global__ __launch_bounds__(256) void k_v16_finish(
         for (int s = 0; s < d; ++s) v += part[(((long long)item * d + s) * 4 + j) * 256 + e];
         x[k] = v;
         ls += (double)v;
-    }
-    if (zv) {  // the vertex scalar: the unnormalised message out of port 0 meets the one into it
-        if (j != 0) return;
-        const long long mi = msg_off[vin[item].x];
-        double z = 0.0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int e = lane + 64 * k, a = e >> 4, b = e & 15;
-            if (a < D && b < D) z += (double)x[k] * (double)mold[mi + a * D + b];
-        }
-        z = wave_sum_v(z);
-        if (lane == 0) zv[vlist[item]] = z;
-        return;
     }
     const double S = wave_sum_v(ls);
     double dn = 0.0, nn = 0.0, oo = 0.0, mx = 0.0;
@@ -525,17 +511,21 @@ static int vertex16_set_lds_limit() {
                             (int)VQ<12>::lds()) != hipSuccess ||
         hipFuncSetAttribute((const void *)k_vertex_d12<10>,
                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)VQ<10>::lds()) != hipSuccess ||
+        hipFuncSetAttribute((const void *)k_v12_scalar<12>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)VQ<12>::lds()) != hipSuccess ||
+        hipFuncSetAttribute((const void *)k_v12_scalar<10>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)VQ<10>::lds()) != hipSuccess)
         return 2;
     done = 1;
     return 0;
 }
 
-// The large-bond bucket's part of a sweep: slices, then the per-message finish (with zv, the
-// vertex scalars at the messages src instead; dst and the residuals are not written).
+// The large-bond bucket's part of a sweep: slices, then the per-message finish.
 static int vertex16_sweep(VertexPlan *p, hipStream_t st, DevTopo tp, const void *src, void *dst,
-                          const NetCtl &ctl, double *res_fid, double *res_abs,
-                          double *zv = nullptr) {
+                          const NetCtl &ctl, double *res_fid, double *res_abs) {
     if (p->nv16 == 0) return 0;
     if (!p->bf16) {
         const int n10 = p->nv16_k10, n12 = p->nv16_k4 - p->nv16_k10;
@@ -569,7 +559,7 @@ static int vertex16_sweep(VertexPlan *p, hipStream_t st, DevTopo tp, const void 
         hipLaunchKernelGGL(k_v16_finish, dim3(p->nv16), dim3(256), 0, st,
                            (const float *)p->d_v16part, (const float *)src, (float *)dst,
                            p->d_v16out, p->d_v16dim, p->d_v16net, tp.msg_off, ctl, p->d,
-                           res_fid, res_abs, p->d_v16in, p->d_v16list, zv);
+                           res_fid, res_abs);
         return hipGetLastError() == hipSuccess ? 0 : 2;
     }
     const size_t half = (size_t)p->nv16 * p->d * V16_ELEMS;
@@ -586,7 +576,7 @@ static int vertex16_sweep(VertexPlan *p, hipStream_t st, DevTopo tp, const void 
 #undef V16_LAUNCH
     hipLaunchKernelGGL(k_v16_finish, dim3(p->nv16), dim3(256), 0, st, (const float *)p->d_v16part,
                        (const float *)src, (float *)dst, p->d_v16out, p->d_v16dim, p->d_v16net,
-                       tp.msg_off, ctl, p->d, res_fid, res_abs, p->d_v16in, p->d_v16list, zv);
+                       tp.msg_off, ctl, p->d, res_fid, res_abs);
     return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
@@ -621,5 +611,31 @@ static int vertex_k3_sweep(VertexPlan *p, hipStream_t st, DevTopo tp, const void
                        (const float *)p->d_vk3part, (const float *)src, (float *)dst,
                        p->d_vout + i0, p->d_vdim + i0, p->d_vnet + i0, tp.msg_off, ctl, p->d,
                        res_fid, res_abs);
+    return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+
+// Vertex scalars of the large-bond bucket (FP32) at the messages src: zv[vertex].  The slices'
+// shares take the space of the sweep's partial results.
+static int vertex16_scalars(const VertexPlan *p, hipStream_t st, DevTopo tp, const void *src,
+                            double *zv) {
+    if (p->nv16 == 0) return 0;
+    const int n10 = p->nv16_k10, n12 = p->nv16_k4 - p->nv16_k10;
+    const int n4 = p->nv16_k4, n3 = p->nv16 - p->nv16_k4;
+    double *part = (double *)p->d_v16part;
+    if (n10 > 0)
+        hipLaunchKernelGGL((k_v12_scalar<10>), dim3(n10 * p->d), dim3(64 * VQ<10>::NW),
+                           (VQ<10>::lds()), st, (const float *)p->d_v10sites, (const float *)src,
+                           p->d_v16in, p->d_v16dim, tp.msg_off, p->d, 0, part);
+    if (n12 > 0)
+        hipLaunchKernelGGL((k_v12_scalar<12>), dim3(n12 * p->d), dim3(64 * VQ<12>::NW),
+                           (VQ<12>::lds()), st, (const float *)p->d_v12sites, (const float *)src,
+                           p->d_v16in, p->d_v16dim, tp.msg_off, p->d, n10, part);
+    if (n3 > 0)
+        hipLaunchKernelGGL(k_v3_scalar<12>, dim3((n3 * p->d + V3_WAVES - 1) / V3_WAVES),
+                           dim3(64 * V3_WAVES), 0, st, (const float *)p->d_v3sites,
+                           (const float *)src, p->d_v16in, p->d_v16dim, tp.msg_off, p->d, n4, n3,
+                           part);
+    hipLaunchKernelGGL(k_v16_scalar_sum, dim3((p->nv16 + 255) / 256), dim3(256), 0, st,
+                       (const double *)part, p->d_v16list, p->nv16, p->d, zv);
     return hipGetLastError() == hipSuccess ? 0 : 2;
 }

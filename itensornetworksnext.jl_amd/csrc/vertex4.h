@@ -80,8 +80,9 @@ __device__ __forceinline__ void vs_mode_0(float (&X)[VsShape<DP>::RP], const flo
     }
 }
 
-// ZV: the vertex scalars zv[vlist[item]] at the messages mold instead of a sweep: the
-// unnormalised message out of port 0 meets the one into it (a padded port 0: e0 e0^T).
+// ZV: the vertex scalars zv[vlist[item]] at the messages mold instead of a sweep: every port
+// absorbed, then <E, A> in FP64 (the message out of port 0, opened in FP32, against the one
+// into it was 1.7 to 6 times further from FP64: 3.9e-8 relative at D = 3 against 1.2e-8).
 //
 // fold: the stopping rule of a run on one network whose vertices are all in one bucket, folded
 // as in the D <= 8 kernels (work item: the wave's group).  With one 1024-thread workgroup
@@ -104,6 +105,7 @@ __global__ __launch_bounds__(64) void k_vertex_s(
     constexpr int R = Shp::R, RP = Shp::RP, M2 = Shp::M2;
     __shared__ float msm[16 * 4 * M2];   // [vi][port][p * DP + b], padded incoming messages
     __shared__ float part[16 * 4 * M2];  // [quad][port][a * DP + a'], per-slice results
+    __shared__ double zq[ZV ? 16 : 1];   // the slices' shares of the vertex scalars
     const int g = blockIdx.x, lane = threadIdx.x;
     const int quad = lane >> 2, j = lane & 3;
     const int W = 16 / d;
@@ -162,8 +164,10 @@ __global__ __launch_bounds__(64) void k_vertex_s(
         for (int e = 0; e < M2; ++e) pq[prt * M2 + e] = quad_sum(o[e]);
     };
     if (!live) {  // uniform over the quad; an idle or stopped slice contributes zeros
+        if constexpr (!ZV) {
 #pragma unroll
-        for (int e = 0; e < 4 * M2; ++e) pq[e] = 0.f;
+            for (int e = 0; e < 4 * M2; ++e) pq[e] = 0.f;
+        }
     } else {
         const float *m0 = msm + (vi * 4 + 0) * M2, *m1 = msm + (vi * 4 + 1) * M2;
         const float *m2 = msm + (vi * 4 + 2) * M2, *m3 = msm + (vi * 4 + 3) * M2;
@@ -175,95 +179,106 @@ __global__ __launch_bounds__(64) void k_vertex_s(
             c2[p] = j < DP ? m2[p * DP + j] : 0.f;
             c3[p] = j < DP ? m3[p * DP + j] : 0.f;
         }
-        float E[RP], o[M2];
-
-        // ---- phase A: E = A x0 m0 x1 m1
-        if constexpr (!ZV) {
+        float E[RP];
+        if constexpr (ZV) {
 #pragma unroll
-        for (int r = 0; r < RP; ++r) E[r] = A[r];
-        vs_mode_0<DP>(E, c0);
-        vs_mode_in<DP, 1>(E, c1);
-        // out2[a][a'] = sum_{p1,b3} G[p1,a,b3] A[p1,a',b3], G = E x3 m3 block by block (p1)
+            for (int r = 0; r < RP; ++r) E[r] = A[r];
+            vs_mode_0<DP>(E, c0);
+            vs_mode_in<DP, 1>(E, c1);
+            vs_mode_in<DP, 2>(E, c2);
+            vs_mode_in<DP, 3>(E, c3);
+            double z = 0.0;
 #pragma unroll
-        for (int e = 0; e < M2; ++e) o[e] = 0.f;
+            for (int r = 0; r < R; ++r) z += (double)E[r] * (double)A[r];
+            z = group_sum<4>(j < DP ? z : 0.0);
+            if (j == 0) zq[quad] = z;
+        } else {
+            float o[M2];
+            // ---- phase A: E = A x0 m0 x1 m1
 #pragma unroll
-        for (int p1 = 0; p1 < DP; ++p1) {
-            float G[M2];  // [a = p2][b3]
+            for (int r = 0; r < RP; ++r) E[r] = A[r];
+            vs_mode_0<DP>(E, c0);
+            vs_mode_in<DP, 1>(E, c1);
+            // out2[a][a'] = sum_{p1,b3} G[p1,a,b3] A[p1,a',b3], G = E x3 m3 block by block (p1)
 #pragma unroll
-            for (int x = 0; x < DP; ++x) {
-                v4f acc = {0.f, 0.f, 0.f, 0.f};
+            for (int e = 0; e < M2; ++e) o[e] = 0.f;
 #pragma unroll
-                for (int p = 0; p < DP; ++p)
-                    acc = __builtin_amdgcn_mfma_f32_4x4x1f32(c3[p], E[(p1 * DP + x) * DP + p], acc, 0, 0, 0);
+            for (int p1 = 0; p1 < DP; ++p1) {
+                float G[M2];  // [a = p2][b3]
 #pragma unroll
-                for (int y = 0; y < DP; ++y) G[x * DP + y] = acc[y];
+                for (int x = 0; x < DP; ++x) {
+                    v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int p = 0; p < DP; ++p)
+                        acc = __builtin_amdgcn_mfma_f32_4x4x1f32(c3[p], E[(p1 * DP + x) * DP + p], acc, 0, 0, 0);
+#pragma unroll
+                    for (int y = 0; y < DP; ++y) G[x * DP + y] = acc[y];
+                }
+#pragma unroll
+                for (int a = 0; a < DP; ++a)
+#pragma unroll
+                    for (int ap = 0; ap < DP; ++ap)
+#pragma unroll
+                        for (int t = 0; t < DP; ++t)
+                            o[a * DP + ap] = fmaf(G[a * DP + t], A[(p1 * DP + ap) * DP + t], o[a * DP + ap]);
             }
+            store(o, 2);
+            // out3[a][a'] = sum_{p1,b2} G[p1,b2,a] A[p1,b2,a'], G = E x2 m2 block by block (p1)
+#pragma unroll
+            for (int e = 0; e < M2; ++e) o[e] = 0.f;
+#pragma unroll
+            for (int p1 = 0; p1 < DP; ++p1) {
+                float G[M2];  // [b2][a = p3]
+#pragma unroll
+                for (int y = 0; y < DP; ++y) {
+                    v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int p = 0; p < DP; ++p)
+                        acc = __builtin_amdgcn_mfma_f32_4x4x1f32(c2[p], E[(p1 * DP + p) * DP + y], acc, 0, 0, 0);
+#pragma unroll
+                    for (int x = 0; x < DP; ++x) G[x * DP + y] = acc[x];
+                }
+#pragma unroll
+                for (int a = 0; a < DP; ++a)
+#pragma unroll
+                    for (int ap = 0; ap < DP; ++ap)
+#pragma unroll
+                        for (int t = 0; t < DP; ++t)
+                            o[a * DP + ap] = fmaf(G[t * DP + a], A[(p1 * DP + t) * DP + ap], o[a * DP + ap]);
+            }
+            store(o, 3);
+
+            // ---- phase B: E = A x2 m2 x3 m3
+#pragma unroll
+            for (int r = 0; r < RP; ++r) E[r] = A[r];
+            vs_mode_in<DP, 2>(E, c2);
+            vs_mode_in<DP, 3>(E, c3);
+            // out1 = open_1(E x0 m0, A), the port-0 product fused entry by entry
+#pragma unroll
+            for (int e = 0; e < M2; ++e) o[e] = 0.f;
 #pragma unroll
             for (int a = 0; a < DP; ++a)
 #pragma unroll
-                for (int ap = 0; ap < DP; ++ap)
+                for (int t = 0; t < DP * DP; ++t) {
+                    const v4f gx = quad_gather(E[a * DP * DP + t]);
+                    float gv = 0.f;
 #pragma unroll
-                    for (int t = 0; t < DP; ++t)
-                        o[a * DP + ap] = fmaf(G[a * DP + t], A[(p1 * DP + ap) * DP + t], o[a * DP + ap]);
-        }
-        store(o, 2);
-        // out3[a][a'] = sum_{p1,b2} G[p1,b2,a] A[p1,b2,a'], G = E x2 m2 block by block (p1)
+                    for (int p = 0; p < DP; ++p) gv = fmaf(gx[p], c0[p], gv);
 #pragma unroll
-        for (int e = 0; e < M2; ++e) o[e] = 0.f;
+                    for (int ap = 0; ap < DP; ++ap) o[a * DP + ap] = fmaf(gv, A[ap * DP * DP + t], o[a * DP + ap]);
+                }
+            store(o, 1);
+            // out0 = open_0(E x1 m1, A) on the matrix cores: with a = G (row a = lane i) and
+            // b = A (column a' = lane j), register i of lane j collects out0[i][j]
+            vs_mode_in<DP, 1>(E, c1);
+            v4f o0 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int p1 = 0; p1 < DP; ++p1) {
-            float G[M2];  // [b2][a = p3]
+            for (int r = 0; r < R; ++r)
+                o0 = __builtin_amdgcn_mfma_f32_4x4x1f32(E[r], A[r], o0, 0, 0, 0);
+            if (j < DP) {
 #pragma unroll
-            for (int y = 0; y < DP; ++y) {
-                v4f acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int p = 0; p < DP; ++p)
-                    acc = __builtin_amdgcn_mfma_f32_4x4x1f32(c2[p], E[(p1 * DP + p) * DP + y], acc, 0, 0, 0);
-#pragma unroll
-                for (int x = 0; x < DP; ++x) G[x * DP + y] = acc[x];
+                for (int i = 0; i < DP; ++i) pq[i * DP + j] = o0[i];
             }
-#pragma unroll
-            for (int a = 0; a < DP; ++a)
-#pragma unroll
-                for (int ap = 0; ap < DP; ++ap)
-#pragma unroll
-                    for (int t = 0; t < DP; ++t)
-                        o[a * DP + ap] = fmaf(G[t * DP + a], A[(p1 * DP + t) * DP + ap], o[a * DP + ap]);
-        }
-        store(o, 3);
-        }
-
-        // ---- phase B: E = A x2 m2 x3 m3
-#pragma unroll
-        for (int r = 0; r < RP; ++r) E[r] = A[r];
-        vs_mode_in<DP, 2>(E, c2);
-        vs_mode_in<DP, 3>(E, c3);
-        // out1 = open_1(E x0 m0, A), the port-0 product fused entry by entry
-        if constexpr (!ZV) {
-#pragma unroll
-        for (int e = 0; e < M2; ++e) o[e] = 0.f;
-#pragma unroll
-        for (int a = 0; a < DP; ++a)
-#pragma unroll
-            for (int t = 0; t < DP * DP; ++t) {
-                const v4f gx = quad_gather(E[a * DP * DP + t]);
-                float gv = 0.f;
-#pragma unroll
-                for (int p = 0; p < DP; ++p) gv = fmaf(gx[p], c0[p], gv);
-#pragma unroll
-                for (int ap = 0; ap < DP; ++ap) o[a * DP + ap] = fmaf(gv, A[ap * DP * DP + t], o[a * DP + ap]);
-            }
-        store(o, 1);
-        }
-        // out0 = open_0(E x1 m1, A) on the matrix cores: with a = G (row a = lane i) and
-        // b = A (column a' = lane j), register i of lane j collects out0[i][j]
-        vs_mode_in<DP, 1>(E, c1);
-        v4f o0 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int r = 0; r < R; ++r) o0 = __builtin_amdgcn_mfma_f32_4x4x1f32(E[r], A[r], o0, 0, 0, 0);
-        if (j < DP) {
-#pragma unroll
-            for (int i = 0; i < DP; ++i) pq[i * DP + j] = o0[i];
         }
     }
     __syncthreads();
@@ -271,12 +286,7 @@ __global__ __launch_bounds__(64) void k_vertex_s(
     if constexpr (ZV) {  // one lane per vertex
         if (!mine || port != 0) return;
         double z = 0.0;
-#pragma unroll
-        for (int e = 0; e < M2; ++e) {
-            float v = 0.f;
-            for (int t = 0; t < d; ++t) v += part[((vi2 * d + t) * 4) * M2 + e];
-            z += (double)v * (double)msm[(vi2 * 4) * M2 + e];
-        }
+        for (int t = 0; t < d; ++t) z += zq[vi2 * d + t];
         zv[vlist[b2]] = z;
         return;
     }
@@ -331,16 +341,17 @@ __device__ __forceinline__ int t2_idx(int p0, int p1, int p2, int p3) {
     return p0 * 8 + p1 * 4 + p2 * 2 + p3;
 }
 
-// X[.., b at port P, ..] = sum_p X[.., p, ..] m[p][b], in place (m: 2 x 2, [p][b])
-template <int P>
+// X[.., b at port P, ..] = sum_p X[.., p, ..] m[p][b], in place (m: 2 x 2, [p][b]).  UP: summed
+// over p upwards, as the generic kernel does (the vertex scalars; the same roundings as there).
+template <int P, bool UP = false>
 __device__ __forceinline__ void t2_mode(float (&X)[16], const float (&m)[4]) {
     constexpr int st = 8 >> P;  // register stride of port P
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         if (r & st) continue;  // r has digit 0 at port P
         const float x0 = X[r], x1 = X[r + st];
-        X[r] = fmaf(x0, m[0], x1 * m[2]);
-        X[r + st] = fmaf(x0, m[1], x1 * m[3]);
+        X[r] = UP ? fmaf(x1, m[2], x0 * m[0]) : fmaf(x0, m[0], x1 * m[2]);
+        X[r + st] = UP ? fmaf(x1, m[3], x0 * m[1]) : fmaf(x0, m[1], x1 * m[3]);
     }
 }
 
@@ -424,39 +435,41 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         part[lane * 4 + j] = make_float4(o[0], o[1], o[2], o[3]);
     };
     if (live) {
-        float E[16], G[16], o[4];
-        // phase A: E = A x0 m0 x1 m1; out2 = open_2(E x3 m3, A), out3 = open_3(E x2 m2, A)
-        if constexpr (!ZV) {
+        float E[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) E[r] = A[r];
-        t2_mode<0>(E, m[0]);
-        t2_mode<1>(E, m[1]);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) G[r] = E[r];
-        t2_mode<3>(G, m[3]);
-        t2_open<2>(G, A, o);
-        put(2, o);
-        t2_mode<2>(E, m[2]);
-        t2_open<3>(E, A, o);
-        put(3, o);
-        }
-        // phase B: E = A x2 m2 x3 m3; out0 = open_0(E x1 m1, A), out1 = open_1(E x0 m0, A)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) E[r] = A[r];
-        t2_mode<2>(E, m[2]);
-        t2_mode<3>(E, m[3]);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) G[r] = E[r];
-        t2_mode<1>(G, m[1]);
-        t2_open<0>(G, A, o);
         if constexpr (ZV) {  // this slice's share of the vertex scalar
-            o[0] = o[0] * m[0][0];
-            o[1] = o[1] * m[0][1];
-            o[2] = o[2] * m[0][2];
-            o[3] = o[3] * m[0][3];
-        }
-        put(0, o);
-        if constexpr (!ZV) {
+            t2_mode<0, true>(E, m[0]);
+            t2_mode<1, true>(E, m[1]);
+            t2_mode<2, true>(E, m[2]);
+            t2_mode<3, true>(E, m[3]);
+            double z = 0.0;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z += (double)E[r] * (double)A[r];
+            reinterpret_cast<double *>(part)[lane] = z;
+        } else {
+            float G[16], o[4];
+            // phase A: E = A x0 m0 x1 m1; out2 = open_2(E x3 m3, A), out3 = open_3(E x2 m2, A)
+            t2_mode<0>(E, m[0]);
+            t2_mode<1>(E, m[1]);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) G[r] = E[r];
+            t2_mode<3>(G, m[3]);
+            t2_open<2>(G, A, o);
+            put(2, o);
+            t2_mode<2>(E, m[2]);
+            t2_open<3>(E, A, o);
+            put(3, o);
+            // phase B: E = A x2 m2 x3 m3; out0 = open_0(E x1 m1, A), out1 = open_1(E x0 m0, A)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) E[r] = A[r];
+            t2_mode<2>(E, m[2]);
+            t2_mode<3>(E, m[3]);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) G[r] = E[r];
+            t2_mode<1>(G, m[1]);
+            t2_open<0>(G, A, o);
+            put(0, o);
             t2_mode<0>(E, m[0]);
             t2_open<1>(E, A, o);
             put(1, o);
@@ -470,10 +483,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
     if constexpr (ZV) {
         if (!inr || s != 0) return;
         double z = 0.0;
-        for (int t = 0; t < d; ++t) {
-            const float4 pv = part[(vi * d + t) * 4];
-            z += ((double)pv.x + (double)pv.y) + ((double)pv.z + (double)pv.w);
-        }
+        for (int t = 0; t < d; ++t) z += reinterpret_cast<const double *>(part)[vi * d + t];
         zv[vlist[b]] = z;
         return;
     }

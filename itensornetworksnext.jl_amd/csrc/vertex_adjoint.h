@@ -608,6 +608,50 @@ void k_vd_site(const float *__restrict__ vsites, const float *__restrict__ msgs,
     }
 }
 
+// ---- vertex scalars: every port absorbed (the chain of the site form), then <E, A> in FP64.
+template <int NS>
+__global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void k_vd_scalar(const float *__restrict__ vsites, const float *__restrict__ msgs,
+                 const int4 *__restrict__ vin, const int4 *__restrict__ vout,
+                 const int4 *__restrict__ vdim, const int *__restrict__ vlist,
+                 const long long *__restrict__ msg_off, double *__restrict__ zv) {
+    extern __shared__ __align__(16) float vsm[];
+    __shared__ double zs[NS];
+    const int u = blockIdx.x;
+    const int w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    float *bufB = vsm + w * VX_BUF;
+    float *msm = vsm + NS * VX_BUF;
+    const VdSlots sl = vd_slots(vin, vout, vdim, msg_off, u);
+    vd_load_mats<NS>(msgs, nullptr, sl, 0, msm, nullptr);
+    const float *src = vsites + ((long long)u * NS + w) * 4096;
+    float R1[64], R2[64];
+#pragma unroll
+    for (int r = 0; r < 64; ++r) R1[r] = src[r * 64 + lane];
+    __syncthreads();
+    float M[16];
+    vx_load_m(msm + 0 * 64, M);
+    vd_mp1<true>(R1, M, R2);
+    vx_load_m(msm + 1 * 64, M);
+    vd_mp1<false>(R2, M, R2);
+    vd_x_to_y(R2, bufB, lane);
+    vx_load_m(msm + 2 * 64, M);
+    vd_mp1<true>(R2, M, R2);
+    vx_load_m(msm + 3 * 64, M);
+    vd_mp1<false>(R2, M, R2);
+    vd_y_to_x(R2, bufB, lane);
+    double z = 0.0;
+#pragma unroll
+    for (int r = 0; r < 64; ++r) z += (double)R2[r] * (double)R1[r];
+    z = wave_sum_v(z);
+    if (lane == 0) zs[w] = z;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int s = 1; s < NS; ++s) z += zs[s];
+        zv[vlist[u]] = z;
+    }
+}
+
 // ---- small kernels of the orchestration
 // dm[rev q] = cv1[owner q] * GX[q] + cv0[owner q] * G[q]   (vertex terms of the energy)
 __global__ void k_vd_vertex_terms(DevTopo tp, const float *G, const float *GX, const double *cv0,
@@ -671,10 +715,11 @@ static int vd_set_limits(int ns) {
     {(const void *)k_vd_msg<NS, false, false>, (const void *)k_vd_msg<NS, true, false>,        \
      (const void *)k_vd_msg<NS, false, true>, (const void *)k_vd_msg<NS, true, true>,          \
      (const void *)k_vd_site<NS, false, false>, (const void *)k_vd_site<NS, true, false>,      \
-     (const void *)k_vd_site<NS, false, true>, (const void *)k_vd_site<NS, true, true>}
-    const void *fns[4][8] = {VD_FNS(1), VD_FNS(2), VD_FNS(3), VD_FNS(4)};
+     (const void *)k_vd_site<NS, false, true>, (const void *)k_vd_site<NS, true, true>,        \
+     (const void *)k_vd_scalar<NS>}
+    const void *fns[4][9] = {VD_FNS(1), VD_FNS(2), VD_FNS(3), VD_FNS(4)};
 #undef VD_FNS
-    for (int h = 0; h < 8; ++h)
+    for (int h = 0; h < 9; ++h)
         if (hipFuncSetAttribute(fns[ns - 1][h], hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)(h < 4 ? vd_msg_lds(ns) : vd_site_lds(ns))) != hipSuccess)
             return 2;
@@ -768,6 +813,24 @@ static int vd_site(const VdCtx &c, const float *msgs, const float *W, int trans,
             return rc_;            \
         }                          \
     } while (0)
+
+// Vertex scalars of the bucket at the messages msgs: zv[vertex].
+static int vd_scalars(const VdCtx &c, const float *msgs, double *zv) {
+    const VertexPlan &p = *c.vp;
+    const size_t lds = sizeof(float) * ((size_t)p.d * VX_BUF + 256);
+#define VD_SCALAR(NS)                                                                          \
+    hipLaunchKernelGGL(k_vd_scalar<NS>, dim3(p.nv), dim3(64 * NS), lds, c.st, c.vsites, msgs,  \
+                       p.d_vin, p.d_vout, p.d_vdim, p.d_vlist, c.tp.msg_off, zv)
+    switch (p.d) {
+        case 1: VD_SCALAR(1); break;
+        case 2: VD_SCALAR(2); break;
+        case 3: VD_SCALAR(3); break;
+        case 4: VD_SCALAR(4); break;
+        default: return 4;
+    }
+#undef VD_SCALAR
+    return hipGetLastError() == hipSuccess ? 0 : 2;
+}
 
 // Gradient of log Z_BP: dlogZ/dA_u = (bra + ket derivative of Z_u) / Z_u at the fixed point.
 static int vadj_grad_lognorm(AdjointScratch *s, const VdCtx &c, const float *msgs, long long nsite,
