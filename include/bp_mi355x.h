@@ -285,7 +285,8 @@ int bp_get_option(bp_context *ctx, const char *name, int *value);
 /* Autotuner.  Times, on the context's own sites and messages, (a) for every largest bond
  * dimension D present that the vertex kernels take (<= 12 FP32, <= 16 BF16 and FP64; norm networks,
  * automatic path) whether its networks sweep faster on the vertex kernels (bonds padded to
- * 8, 12 or 16) or on the generic kernel, and
+ * 8, 12 or 16) or on the generic kernel (FP64 up to D = 8: the D <= 8 kernel or the pair
+ * kernel, a choice of its own for every largest degree), and
  * (b) the D <= 8 vertex sweep kernel variant ("vertex_variant" of bp_set_option) and the
  * waves per workgroup of the bond-dimension-16 kernel ("vertex16_waves"), and
  * (c) for every bucket of generic-kernel slots (owner's physical dimension and largest

@@ -389,6 +389,7 @@ struct bp_context {
     VertexPlan vplan;
     bool vplan_ok = false;
     unsigned vx_mask = 0x1FFFEu;  // bit D: networks of largest bond dimension D may use it
+    unsigned vx_timed = 0u;       // FP64, bit D: the autotuner timed it against the pair kernel
     int vx_variant = -1;        // D <= 8 vertex sweep kernel (0: two LDS buffers per wave,
                                 // 1: one buffer per wave, two waves per SIMD; -1: the faster
                                 // one at 32x32 D=8: 1 in FP32 with d >= 2, else 0)
@@ -961,6 +962,18 @@ static int launch_edge_scalars(bp_context *c, const T *msgs) {
 
 static constexpr double PAIR_MFMA_MAX = 400.0;
 
+// Bits of the networks' largest bond dimensions (up to 31).
+static unsigned net_dim_mask(const bp_context *c) {
+    unsigned mask = 0u;
+    for (int n = 0; n < c->nnet; ++n) {
+        int dm = 0;
+        for (int q = c->pbeg[n]; q < c->pbeg[n + 1]; ++q)
+            dm = std::max(dm, c->edge_dim[c->port_edge[q]]);
+        if (dm < 32) mask |= 1u << dm;
+    }
+    return mask;
+}
+
 // The FP64 vertex plan for this context's networks (bond dimensions enabled: the context's
 // vertex mask in FP64 contexts; 6..8 and 9..16 for the polish of FP32/BF16 contexts): the
 // D <= 8 kernel (vertex64.h) when every network's largest bond dimension is 6..8, else the
@@ -989,8 +1002,11 @@ static int ensure_v64(bp_context *c) {
         // products it pads to 16 x 16, the other's is that of bond dimension 8.  us per sweep,
         // d = 2, pair / other: D = 6 (324 products per slice) 23 / 36 at 16x16 and 71 / 82 at
         // 32x32; D = 7 (832) 33 / 36 and 118 / 83; D = 8 of degree 3 (152) 21 / 41 at 8x16 hex
+        // (bond dimensions that the autotuner has timed stay with what it chose)
         RETCHK(ensure_pair(c));
-        if (c->v64_kind == 1 && c->pair_ok && c->pair.covers && pair_mfma_per_slice(&c->pair) <= PAIR_MFMA_MAX) {
+        const unsigned timed = c->dtype == BP_F64 ? c->vx_timed & net_dim_mask(c) : 0u;
+        if (c->v64_kind == 1 && c->pair_ok && c->pair.covers && timed == 0u &&
+            pair_mfma_per_slice(&c->pair) <= PAIR_MFMA_MAX) {
             vertex64_release(&c->v64);
             c->v64_kind = 3;
         }
@@ -1735,6 +1751,7 @@ int bp_set_option(bp_context *c, const char *name, int value) {
     }
     if (strcmp(name, "vertex_bond_mask") == 0) {
         c->vx_mask = (unsigned)value & 0x1FFFEu;
+        c->vx_timed = 0u;
         if (c->have_topo) RETCHK(rebuild_vertex_plan(c));
         return BP_OK;
     }
@@ -2005,8 +2022,10 @@ int bp_run(bp_context *c, int maxiter, double tol, int criterion, int use_graph,
 // a warm-up) and kept in a JSON cache, one entry per line:
 //   "vx|<dtype>|d<d>|D<D>": {"vertex": 0|1, "us": t_chosen, "us_alt": t_other}
 //       networks whose largest bond dimension is D run on the vertex kernels (padded to 8,
-//       12 or 16; FP64: the FP64 vertex kernel, D <= 8) or on the generic kernel,
-//       whichever sweeps faster;
+//       12 or 16) or on the generic kernel, whichever sweeps faster;
+//   "vx|f64|d<d>|D<D>|k<degree>", D <= 8: the same for the FP64 D <= 8 kernel against the
+//       pair kernel (generic kernel where that declines a vertex), at the largest degree of
+//       those networks;
 //   "vxk|<f32|bf16>|d<d>": {"variant": 0..5, "us": t_chosen, "us_alt": t_next}
 //       the D <= 8 vertex sweep kernel: 0 two LDS buffers per wave, 1 one buffer per wave
 //       with two waves per SIMD, 2 and 3 (FP32 only) open contractions on MFMA with the
@@ -2146,7 +2165,8 @@ int bp_autotune(bp_context *c, const char *cache_path, int mode, int *out_tuned)
     int rc = BP_OK;
     // 1. vertex kernels or generic kernel, per largest bond dimension (<= 12 FP32, <= 16 BF16)
     if (!c->plain && !c->is_cplx() && c->path == BP_PATH_AUTO) {
-        std::map<int, int> dmax_d;  // largest bond dimension -> physical dimension
+        std::map<int, int> dmax_d;    // largest bond dimension -> physical dimension
+        std::map<int, int> dmax_deg;  // and largest degree
         for (int n = 0; n < c->nnet && rc == BP_OK; ++n) {
             int dm = 0, deg = 0, d = c->phys_dim[c->vbeg[n]];
             for (int u = c->vbeg[n]; u < c->vbeg[n + 1]; ++u) {
@@ -2155,19 +2175,35 @@ int bp_autotune(bp_context *c, const char *cache_path, int mode, int *out_tuned)
                     dm = std::max(dm, c->edge_dim[c->port_edge[q]]);
             }
             const int dlim = c->dtype == BP_BF16 ? 16 : c->dtype == BP_F32 ? 12 : 16;
-            if (dm >= 1 && dm <= dlim && deg <= 4 && d <= 4) dmax_d[dm] = d;
+            if (dm >= 1 && dm <= dlim && deg <= 4 && d <= 4) {
+                dmax_d[dm] = d;
+                dmax_deg[dm] = std::max(dmax_deg[dm], deg);
+            }
         }
         for (const auto &kv : dmax_d) {
             const int D = kv.first;
             std::ostringstream o;
             o << "vx|" << dtype_name(c->dtype) << "|d" << kv.second << "|D" << D;
+            // FP64 up to the pair kernel's bond dimensions: the D <= 8 kernel against that one,
+            // whose time grows with the degree
+            const bool against_pair = c->dtype == BP_F64 && D <= PAIR_MAXD;
+            if (against_pair) o << "|k" << dmax_deg[D];
             const std::string key = o.str();
+            const unsigned bit = 1u << D, mask0 = c->vx_mask, timed0 = c->vx_timed;
             auto it = c->tune.find(key);
             if (it == c->tune.end() && mode >= 1) {
-                c->vx_mask |= 1u << D;
+                c->vx_mask |= bit;
+                if (against_pair) c->vx_timed |= bit;  // the kernel itself, not its stand-in
                 rc = rebuild_vertex_plan(c);
                 const double t_on = rc == BP_OK ? tune_time_sweep(c, 3) : -1.0;
-                c->vx_mask &= ~(1u << D);
+                if (rc == BP_OK && t_on >= 0.0 && c->dtype == BP_F64 &&
+                    resolve_path(c) != BP_PATH_VERTEX) {
+                    // another network keeps every one off the vertex kernel: nothing to choose
+                    c->vx_mask = mask0;
+                    c->vx_timed = timed0;
+                    continue;
+                }
+                c->vx_mask &= ~bit;
                 if (rc == BP_OK) rc = rebuild_vertex_plan(c);
                 const double t_off = rc == BP_OK ? tune_time_sweep(c, 3) : -1.0;
                 if (rc != BP_OK || t_on < 0.0 || t_off < 0.0) {
@@ -2182,8 +2218,9 @@ int bp_autotune(bp_context *c, const char *cache_path, int mode, int *out_tuned)
                 ++tuned;
             }
             if (it != c->tune.end()) {
-                if (it->second.vertex) c->vx_mask |= 1u << D;
-                else c->vx_mask &= ~(1u << D);
+                if (it->second.vertex) c->vx_mask |= bit;
+                else c->vx_mask &= ~bit;
+                if (against_pair) c->vx_timed |= bit;
             }
         }
         if (rc == BP_OK) rc = rebuild_vertex_plan(c);

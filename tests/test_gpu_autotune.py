@@ -80,3 +80,55 @@ def test_autotune_fp64_generic_buckets(pkg, orc):
     want, _, _, at = orc.bp(t, s, m0, maxiter=400, tol=1e-13, criterion="maxabs")
     assert at > 0
     assert np.max(np.abs(got - want)) < 1e-10
+
+
+def _fp64(pkg, g, D, cache, mode):
+    t = pkg.build_topology(g, D, 2)
+    s = pkg.peps.random_sites(t, 9, scale=pkg.peps.peps_scale(2, D))
+    with pkg.Engine(t, s, dtype="f64") as e:
+        e.init_messages("identity")
+        n = e.autotune(cache=cache, mode=mode)
+        return n, e.path()
+
+
+def test_autotune_fp64_times_two_kernels(pkg, tmp_path):
+    """The FP64 choice is between the D <= 8 kernel and the pair kernel: at D = 8 on a heavy-hex
+    lattice the latter takes about half the time, so the times tell which kernels were timed."""
+    _say("case autotune fp64 two kernels")
+    cache = str(tmp_path / "tune.json")
+    n, path = _fp64(pkg, pkg.heavy_hex_lattice(8, 16), 8, cache, "missing")
+    table = json.load(open(cache))
+    _say(f"tuned {table}, path {path}")
+    assert n == 1 and list(table) == ["vx|f64|d2|D8|k3"]
+    v = table["vx|f64|d2|D8|k3"]
+    assert v["vertex"] == 0 and v["us_alt"] > 1.2 * v["us"]
+    # a lattice of another degree has a choice of its own
+    assert _fp64(pkg, pkg.named_grid((3, 3)), 8, cache, "cached") == (0, "vertex")
+
+
+def test_autotune_fp64_other_caches(pkg, tmp_path):
+    """Entries without a degree, whose alternative was the generic kernel, decide nothing; an
+    entry for the D <= 8 kernel keeps it where the pair kernel would stand in."""
+    _say("case autotune fp64 other caches")
+    cache = str(tmp_path / "tune.json")
+    with open(cache, "w") as f:
+        f.write('{\n  "vx|f64|d2|D8": {"vertex": 0, "us": 1, "us_alt": 2}\n}\n')
+    assert _fp64(pkg, pkg.named_grid((3, 3)), 8, cache, "cached") == (0, "vertex")
+    with open(cache, "w") as f:
+        f.write('{\n  "vx|f64|d2|D4|k3": {"vertex": 1, "us": 1, "us_alt": 2}\n}\n')
+    assert _fp64(pkg, pkg.named_grid((2, 4)), 4, cache, "cached") == (0, "vertex")
+    assert _fp64(pkg, pkg.named_grid((3, 3)), 4, cache, "cached") == (0, "generic")
+
+
+def test_autotune_fp64_nothing_to_choose(pkg, tmp_path):
+    """Networks of bond dimensions 3 and 9 keep each other off the vertex kernels."""
+    _say("case autotune fp64 nothing to choose")
+    cache = str(tmp_path / "tune.json")
+    tops = [pkg.build_topology(pkg.named_grid((3, 3)), D, 2) for D in (3, 9)]
+    sites = [pkg.peps.random_sites(t, 9, scale=pkg.peps.peps_scale(2, D)) for t, D in zip(tops, (3, 9))]
+    with pkg.Engine(pkg.concat_topologies(tops), np.concatenate(sites), dtype="f64") as e:
+        e.init_messages("identity")
+        mask = e.get_option("vertex_bond_mask")
+        e.autotune(cache=cache, mode="missing")
+        assert e.get_option("vertex_bond_mask") == mask
+    assert not any(k.startswith("vx|") for k in json.load(open(cache)))
