@@ -82,6 +82,23 @@ def test_autotune_fp64_generic_buckets(pkg, orc):
     assert np.max(np.abs(got - want)) < 1e-10
 
 
+def test_autotune_fp64_bucket_the_pair_kernel_declines(pkg, orc):
+    """A degree-5 vertex keeps its messages on the generic kernel, whose bucket is timed."""
+    _say("case autotune fp64 generic bucket")
+    g = pkg.NamedGraph(vertices=[], edges=[("c", i) for i in range(5)] + [(0, 1), (1, 2)])
+    t = pkg.build_topology(g, 3, 2)
+    s = pkg.peps.random_sites(t, 9, scale=pkg.peps.peps_scale(2, 3))
+    m0 = pkg.peps.identity_messages(t)
+    with pkg.Engine(t, s, dtype="f64") as e:
+        e.set_messages(m0)
+        assert e.autotune(mode="all") > 0
+        e.run(maxiter=400, tol=1e-13, criterion="maxabs")
+        got = e.messages()
+    want, _, _, at = orc.bp(t, s, m0, maxiter=400, tol=1e-13, criterion="maxabs")
+    assert at > 0
+    assert np.max(np.abs(got - want)) < 1e-10
+
+
 def _fp64(pkg, g, D, cache, mode):
     t = pkg.build_topology(g, D, 2)
     s = pkg.peps.random_sites(t, 9, scale=pkg.peps.peps_scale(2, D))
