@@ -270,6 +270,11 @@ int bp_local_energy_device(bp_context *ctx, const double *ops_v, const double *o
  *   "pair_run"         longest wait in us (default 250000) inside the launches that run many
  *                      sweeps of a small FP64 or complex network at once, after which the run
  *                      is repeated launch by launch; 0: launch by launch (same messages);
+ *   "keep_workspace"   MiB of device workspace that the context keeps between gate layers
+ *                      (default 512; a layer at 32x32, D = 8 takes 368), and up to 32 MiB of
+ *                      pinned staging for gates and message downloads; setting it gives back
+ *                      what is above, 0: nothing is kept and no memory pinned.  Freed with
+ *                      the context in any case;
  *   "normalize"        1 (default): every update divides the new message by its sum when
  *                      the sum is nonzero; 0: messages are kept unnormalised, as
  *                      SimpleMessageUpdate(; normalize = false) (beliefpropagation.jl:237-253);

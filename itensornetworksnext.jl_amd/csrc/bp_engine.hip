@@ -433,8 +433,9 @@ struct bp_context {
     // adjoint scratch
     AdjointScratch adj;
 
-    // kept between calls, freed with the context (or at the end of a call that needed more
-    // than KEEP_BYTES): device workspace and pinned host staging
+    // kept between calls, freed with the context (or at the end of a call that needed more than
+    // keep_mib MiB, pinned: KEEP_PINNED bytes): device workspace and pinned host staging
+    int keep_mib = 512;         // option "keep_workspace"; 0: nothing kept, nothing pinned
     void *d_scratch = nullptr, *h_scratch = nullptr;
     size_t scratch_bytes = 0, h_scratch_bytes = 0;
     hipEvent_t ev_chunk[2] = {nullptr, nullptr};  // chunked copies to the host
@@ -500,42 +501,51 @@ static int vx_variant_of(const bp_context *c) {
 
 static size_t run_state_bytes(int nnet) { return (sizeof(double) + 3 * sizeof(int)) * nnet; }
 
-static constexpr size_t KEEP_BYTES = (size_t)1 << 30;
+// A layer of two-site gates on every second bond takes 30 MiB of workspace at 16x16 D = 6, 368
+// at 32x32 D = 8 and 1.5 GiB at 64x64 D = 8, where allocating is a small part of the call.  Its
+// staging is a few MiB.
+static constexpr size_t KEEP_PINNED = (size_t)32 << 20;
 
-// The kept device workspace and pinned staging, at least this large.
-static int keep_scratch(bp_context *c, size_t dev, size_t host) {
-    if (c->scratch_bytes < dev) {
-        if (c->d_scratch) (void)hipFree(c->d_scratch);
+// The kept device workspace, at least this large.
+static int keep_device(bp_context *c, size_t bytes) {
+    if (c->scratch_bytes >= bytes) return BP_OK;
+    if (c->d_scratch) (void)hipFree(c->d_scratch);
+    c->d_scratch = nullptr;
+    c->scratch_bytes = 0;
+    if (hipMalloc(&c->d_scratch, bytes) != hipSuccess) {
         c->d_scratch = nullptr;
-        c->scratch_bytes = 0;
-        if (hipMalloc(&c->d_scratch, dev) != hipSuccess) {
-            c->d_scratch = nullptr;
-            (void)hipGetLastError();
-            return set_err(BP_ERR_NOMEM, "workspace (%zu bytes) does not fit", dev);
-        }
-        c->scratch_bytes = dev;
+        (void)hipGetLastError();
+        return set_err(BP_ERR_NOMEM, "workspace (%zu bytes) does not fit", bytes);
     }
-    if (c->h_scratch_bytes < host) {
-        if (c->h_scratch) (void)hipHostFree(c->h_scratch);
-        c->h_scratch = nullptr;
-        c->h_scratch_bytes = 0;
-        if (hipHostMalloc(&c->h_scratch, host, hipHostMallocDefault) != hipSuccess) {
-            c->h_scratch = nullptr;
-            (void)hipGetLastError();
-            return set_err(BP_ERR_NOMEM, "pinned staging (%zu bytes) does not fit", host);
-        }
-        c->h_scratch_bytes = host;
-    }
+    c->scratch_bytes = bytes;
     return BP_OK;
 }
 
-static void scratch_release(bp_context *c, size_t keep) {
-    if (c->scratch_bytes > keep) {
+// Pinned staging of at least this size; null when there is none to be had (the caller copies
+// from or to pageable memory then).
+static char *keep_pinned(bp_context *c, size_t bytes) {
+    if (c->keep_mib == 0) return nullptr;
+    if (c->h_scratch_bytes >= bytes) return (char *)c->h_scratch;
+    if (c->h_scratch) (void)hipHostFree(c->h_scratch);
+    c->h_scratch = nullptr;
+    c->h_scratch_bytes = 0;
+    if (hipHostMalloc(&c->h_scratch, bytes, hipHostMallocDefault) != hipSuccess) {
+        c->h_scratch = nullptr;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    c->h_scratch_bytes = bytes;
+    return (char *)c->h_scratch;
+}
+
+// Gives back what is larger than the caller lets the context keep (`all`: everything).
+static void scratch_release(bp_context *c, bool all = false) {
+    if (c->scratch_bytes > (all ? 0 : (size_t)c->keep_mib << 20)) {
         (void)hipFree(c->d_scratch);
         c->d_scratch = nullptr;
         c->scratch_bytes = 0;
     }
-    if (c->h_scratch_bytes > keep) {
+    if (c->h_scratch_bytes > (all || c->keep_mib == 0 ? 0 : KEEP_PINNED)) {
         (void)hipHostFree(c->h_scratch);
         c->h_scratch = nullptr;
         c->h_scratch_bytes = 0;
@@ -550,7 +560,10 @@ static void scratch_release(bp_context *c, size_t keep) {
 static int download_doubles(bp_context *c, const void *dev, bool f32, long long n, double *out) {
     constexpr size_t CHUNK = (size_t)2 << 20;  // bytes
     const size_t es = f32 ? sizeof(float) : sizeof(double);
-    if (es * n <= CHUNK / 8 || (!f32 && es * n <= CHUNK)) {
+    char *pinned = nullptr;
+    if (es * n > CHUNK / 8 && (f32 || es * n > CHUNK))
+        pinned = keep_pinned(c, std::min<size_t>(es * n, 2 * CHUNK));
+    if (!pinned) {
         std::vector<float> tmp(f32 ? n : 0);
         HIPCHK(hipMemcpyAsync(f32 ? (void *)tmp.data() : (void *)out, dev, es * n,
                               hipMemcpyDeviceToHost, c->stream));
@@ -559,19 +572,18 @@ static int download_doubles(bp_context *c, const void *dev, bool f32, long long 
         return BP_OK;
     }
     const long long per = (long long)(CHUNK / es), chunks = (n + per - 1) / per;
-    RETCHK(keep_scratch(c, 0, std::min<size_t>(es * n, 2 * CHUNK)));
     for (auto &e : c->ev_chunk)
         if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     auto fetch = [&](long long k) {
         const long long m = std::min(per, n - k * per);
-        hipError_t e = hipMemcpyAsync((char *)c->h_scratch + (k & 1) * CHUNK,
+        hipError_t e = hipMemcpyAsync(pinned + (k & 1) * CHUNK,
                                       (const char *)dev + es * k * per, es * m,
                                       hipMemcpyDeviceToHost, c->stream);
         if (e == hipSuccess) e = hipEventRecord(c->ev_chunk[k & 1], c->stream);
         return e;
     };
     auto unpack = [&](long long k, long long i0, long long i1) {
-        const char *h = (const char *)c->h_scratch + (k & 1) * CHUNK;
+        const char *h = pinned + (k & 1) * CHUNK;
         double *o = out + k * per;
         if (f32)
             for (long long i = i0; i < i1; ++i) o[i] = (double)((const float *)h)[i];
@@ -1380,7 +1392,7 @@ int bp_destroy(bp_context *c) {
     (void)hipStreamSynchronize(c->stream);
     free_all(c);
     if (c->h_state) (void)hipHostFree(c->h_state);
-    scratch_release(c, 0);
+    scratch_release(c, true);
     for (auto &e : c->ev_chunk)
         if (e) (void)hipEventDestroy(e);
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
@@ -1760,6 +1772,13 @@ int bp_set_option(bp_context *c, const char *name, int value) {
         c->run_wait_us = value;
         return BP_OK;
     }
+    if (strcmp(name, "keep_workspace") == 0) {
+        if (value < 0) return set_err(BP_ERR_ARG, "keep_workspace is a size in MiB, or 0");
+        c->keep_mib = value;
+        HIPCHK(hipSetDevice(c->device));
+        scratch_release(c);
+        return BP_OK;
+    }
     if (strcmp(name, "small_bond") == 0) {
         if (value != 0 && value != 1) return set_err(BP_ERR_ARG, "small_bond is 0 or 1");
         c->vx_small = value;
@@ -1778,6 +1797,7 @@ int bp_get_option(bp_context *c, const char *name, int *value) {
     if (strcmp(name, "normalize") == 0) { *value = c->normalize; return BP_OK; }
     if (strcmp(name, "small_bond") == 0) { *value = c->vx_small; return BP_OK; }
     if (strcmp(name, "pair_run") == 0) { *value = c->run_wait_us; return BP_OK; }
+    if (strcmp(name, "keep_workspace") == 0) { *value = c->keep_mib; return BP_OK; }
     return set_err(BP_ERR_ARG, "unknown option %s", name);
 }
 
@@ -3442,8 +3462,13 @@ int bp_apply_gates_resident(bp_context *c, int ngates, const int *kind, const in
     const size_t up_bytes = at;
     const size_t o_in = place(sizeof(double) * tin), o_out = place(sizeof(double) * tout);
     const size_t o_ws = place(sizeof(double) * tws);
-    RETCHK(keep_scratch(c, at, up_bytes));
-    char *dev = (char *)c->d_scratch, *host = (char *)c->h_scratch;
+    RETCHK(keep_device(c, at));
+    char *dev = (char *)c->d_scratch, *host = keep_pinned(c, up_bytes);
+    std::vector<char> pageable;
+    if (!host) {
+        pageable.resize(up_bytes);
+        host = pageable.data();
+    }
     std::memcpy(host + o_desc, desc.data(), sizeof(int) * desc.size());
     std::memcpy(host + o_offs, offs.data(), sizeof(long long) * offs.size());
     std::memcpy(host + o_seg, seg.data(), sizeof(long long) * seg.size());
@@ -3505,14 +3530,15 @@ int bp_apply_gates_resident(bp_context *c, int ngates, const int *kind, const in
     if (e == hipSuccess && (out_chi || out_s))
         e = hipMemcpyAsync(host + o_chi, dev + o_chi, up_bytes - o_chi, hipMemcpyDeviceToHost,
                            c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    const hipError_t drained = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = drained;
     if (e == hipSuccess && out_chi)
         std::memcpy(out_chi, host + o_chi, sizeof(int) * (size_t)ngates);
     if (e == hipSuccess && out_s)
         std::memcpy(out_s, host + o_s, sizeof(double) * (size_t)ngates * sv);
     float ms = 0.f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, c->ev0, c->ev1);
-    scratch_release(c, KEEP_BYTES);
+    scratch_release(c);
     if (e != hipSuccess) return set_err(BP_ERR_HIP, "resident gates: %s", hipGetErrorString(e));
     c->last_ms = ms;
     RETCHK(refresh_sites(c));
