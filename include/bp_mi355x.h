@@ -269,7 +269,11 @@ int bp_local_energy_device(bp_context *ctx, const double *ops_v, const double *o
  *                      0: a separate bookkeeping kernel after every sweep (same results);
  *   "pair_run"         longest wait in us (default 250000) inside the launches that run many
  *                      sweeps of a small FP64 or complex network at once, after which the run
- *                      is repeated launch by launch; 0: launch by launch (same messages);
+ *                      is repeated launch by launch, as are the next 1, 2, 4, .. runs while
+ *                      it happens again; 0: launch by launch (same messages);
+ *   "pair_run_give_up" reads how many of these launches have given up a wait; set to n > 0, the
+ *                      n-th launch of every run waits for nothing and so gives up (tests of
+ *                      the way back), 0 (default): none does;
  *   "keep_workspace"   MiB of device workspace that the context keeps between gate layers
  *                      (default 512; a layer at 32x32, D = 8 takes 368), and up to 32 MiB of
  *                      pinned staging for gates and message downloads; setting it gives back

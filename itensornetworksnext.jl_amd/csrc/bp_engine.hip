@@ -413,6 +413,8 @@ struct bp_context {
     PairPlan pair;
     bool pair_tried = false, pair_ok = false;
     int run_wait_us = 250000;   // option "pair_run": longest wait inside a many-sweep launch, 0: none
+    int run_give_up = 0;        // option "pair_run_give_up": the launch of a run that waits for nothing
+    int run_gave_up = 0;        // many-sweep launches that have given up
 
     // cached sweep graphs (16 sweeps + bookkeeping), one per starting buffer parity; valid
     // while graph_epoch equals the process-wide plan epoch (which moves whenever a captured
@@ -1772,6 +1774,11 @@ int bp_set_option(bp_context *c, const char *name, int value) {
         c->run_wait_us = value;
         return BP_OK;
     }
+    if (strcmp(name, "pair_run_give_up") == 0) {
+        if (value < 0) return set_err(BP_ERR_ARG, "pair_run_give_up counts launches from 1");
+        c->run_give_up = value;
+        return BP_OK;
+    }
     if (strcmp(name, "keep_workspace") == 0) {
         if (value < 0) return set_err(BP_ERR_ARG, "keep_workspace is a size in MiB, or 0");
         c->keep_mib = value;
@@ -1797,6 +1804,7 @@ int bp_get_option(bp_context *c, const char *name, int *value) {
     if (strcmp(name, "normalize") == 0) { *value = c->normalize; return BP_OK; }
     if (strcmp(name, "small_bond") == 0) { *value = c->vx_small; return BP_OK; }
     if (strcmp(name, "pair_run") == 0) { *value = c->run_wait_us; return BP_OK; }
+    if (strcmp(name, "pair_run_give_up") == 0) { *value = c->run_gave_up; return BP_OK; }
     if (strcmp(name, "keep_workspace") == 0) { *value = c->keep_mib; return BP_OK; }
     return set_err(BP_ERR_ARG, "unknown option %s", name);
 }
@@ -1926,15 +1934,18 @@ static int pair_run_chunks(bp_context *c, bool sequential, const RunParams &rp, 
                            bool *over) {
     static std::mutex busy[64];
     *over = false;
-    if (c->run_wait_us == 0 || !pair_run_ready(&c->pair, c->nnet, c->nmsg, c->nports)) return BP_OK;
+    if (c->run_wait_us == 0 || !pair_run_ready(&c->pair, c->nnet, c->nmsg, c->nports) ||
+        pair_run_paused(&c->pair))
+        return BP_OK;
     std::unique_lock<std::mutex> lock(busy[(unsigned)c->device % 64], std::try_to_lock);
     if (!lock.owns_lock()) return BP_OK;
     RETCHK(ensure_h_state(c));
-    while (!*over) {
+    for (int k = 1; !*over; ++k) {
         const int n = std::min(PAIR_RUN_SWEEPS, rp.maxiter - *launched);
         if (pair_run(&c->pair, c->stream, sequential, c->d_sites, c->d_msg[c->cur],
                      c->d_msg[c->cur ^ 1], c->d_done, c->d_iter, c->d_at, c->d_delta,
-                     c->d_res_fid, c->d_res_abs, rp, *launched, n, c->run_wait_us) != 0)
+                     c->d_res_fid, c->d_res_abs, rp, *launched, n,
+                     k == c->run_give_up ? 0 : c->run_wait_us) != 0)
             return set_err(BP_ERR_HIP, "pair run launch failed");
         HIPCHK(hipEventRecord(c->ev1, c->stream));
         HIPCHK(hipMemcpyAsync(c->h_state, c->d_delta, run_state_bytes(1), hipMemcpyDeviceToHost,
@@ -1942,13 +1953,15 @@ static int pair_run_chunks(bp_context *c, bool sequential, const RunParams &rp, 
         HIPCHK(hipStreamSynchronize(c->stream));
         const int done = *(const int *)(c->h_state + sizeof(double));
         if (done & PAIR_RUN_BAILED) {
-            pair_run_off(&c->pair);
+            ++c->run_gave_up;
+            pair_run_ended(&c->pair, true);
             return BP_OK;
         }
         c->cur ^= 1;
         *launched += n;
         *over = done != 0;
     }
+    pair_run_ended(&c->pair, false);
     return BP_OK;
 }
 extern "C" {

@@ -46,6 +46,7 @@ struct PairPlan {
     // many sweeps a launch (pair_run): allocated on first use for the plan's life, at most
     // 8 versions of the messages of a network that fits the device at once
     int run_state = 0;               // 0: not looked at, 1: ready, -1: not for this network
+    int run_pause = 0, run_next = 0; // runs to leave out, twice the next pause
     long long run_nm = 0;            // doubles of one version
     int run_nports = 0;
     void *d_run = nullptr;                 // what the pointers below point into
@@ -75,13 +76,16 @@ int pair_scalars(const PairPlan *p, hipStream_t st, const void *sites, const voi
 // Many sweeps of one network in a launch, its vertices resident together: whether the plan
 // takes it (and its buffers are there).
 bool pair_run_ready(PairPlan *p, int nnet, long long nmsg, int nports);
-void pair_run_off(PairPlan *p);
+// After a run that gave up, the next 1, 2, 4, .. runs are left out (the count starts again after
+// one that did not): whether this one is, and how one that was not has ended.
+bool pair_run_paused(PairPlan *p);
+void pair_run_ended(PairPlan *p, bool gave_up);
 // The schedule of sequential runs, [record][4]: positions | versions << 4 (see pair.hip).
 int pair_run_steps(PairPlan *p, hipStream_t st, const std::vector<int> &steps);
 // `sweeps` sweeps from src to dst (src is left as it is), `first` already done; the network's
 // state and residuals as after a folded run.  done & PAIR_RUN_BAILED: nothing is valid, run
-// again launch by launch (a wait in the kernel took longer than wait_us).  One launch at a time per device: two that wait for each other's
-// room would both give up.
+// again launch by launch (a wait in the kernel took longer than wait_us).  One launch at a time
+// per device: two that wait for each other's room would both give up.
 int pair_run(const PairPlan *p, hipStream_t st, bool sequential, const void *sites,
              const void *src, void *dst, int *done, int *iter, int *at, double *delta,
              double *res_fid, double *res_abs, const RunParams &rp, int first, int sweeps,

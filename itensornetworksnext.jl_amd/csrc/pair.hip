@@ -564,7 +564,9 @@ __global__ __launch_bounds__(64 * pair_waves(NT)) void k_pair(
 //
 // Every poll ends after the caller's limit (0.25 s by default), when the network turns out not to be resident as a
 // whole (another process on the device, say): the run's state is then marked PAIR_RUN_BAILED
-// and the caller runs it again launch by launch from the untouched source messages.
+// and the caller runs it again launch by launch from the untouched source messages.  The next
+// 1, 2, 4, .. runs of the plan go launch by launch too, so what was there for a moment costs one
+// wait, and what stays costs a wait in ever more runs.
 static constexpr int PAIR_RING = 8;
 static constexpr unsigned long long PAIR_POISON = 0x7FF4DEADBEEF0001ull;
 static constexpr unsigned long long PAIR_QUIET = 1ull << 51;
@@ -590,6 +592,7 @@ struct PairRunArgs {
     int split, slice_elems, env_elems, chunk;
     int every, maxiter;
     long long ticks;  // wait limit, in ticks of the 100 MHz clock
+    int looks;        // the clock is read when a wait's count of looks & looks is 0
 };
 
 __global__ void k_pair_run_init(const unsigned long long *__restrict__ src, PairRunArgs a) {
@@ -627,7 +630,7 @@ __device__ __forceinline__ void pair_settle() {
 // One look at a wait that has not ended; false once it must be given up.
 __device__ __forceinline__ bool pair_wait(const PairRunArgs &a, long long t0, int &n) {
     __builtin_amdgcn_s_sleep(1);
-    if ((++n & 15) != 0) return true;
+    if ((++n & a.looks) != 0) return true;
     return wall_clock64() - t0 < a.ticks && !(pair_get(a.done) & PAIR_RUN_BAILED);
 }
 
@@ -1192,7 +1195,16 @@ bool pair_run_ready(PairPlan *p, int nnet, long long nmsg, int nports) {
     return true;
 }
 
-void pair_run_off(PairPlan *p) { p->run_state = -1; }
+bool pair_run_paused(PairPlan *p) {
+    if (p->run_pause == 0) return false;
+    --p->run_pause;
+    return true;
+}
+
+void pair_run_ended(PairPlan *p, bool gave_up) {
+    p->run_next = gave_up ? std::min(2 * std::max(p->run_next, 1), 1 << 20) : 0;
+    p->run_pause = p->run_next / 2;
+}
 
 int pair_run_steps(PairPlan *p, hipStream_t st, const std::vector<int> &steps) {
     if (steps.size() != 4 * p->recs.size()) return 1;
@@ -1231,6 +1243,7 @@ int pair_run(const PairPlan *p, hipStream_t st, bool sequential, const void *sit
     a.every = sequential ? 0 : RUN_CHUNK;
     a.maxiter = rp.maxiter;
     a.ticks = 100ll * wait_us;
+    a.looks = wait_us < 1000 ? 0 : 15;  // a look takes about 0.7 us
     const long long n = std::max(a.nm, (long long)sweeps * PAIR_CTRL_LINES);
     hipLaunchKernelGGL(k_pair_run_init, dim3((unsigned)std::min<long long>((n + 255) / 256, 1024)),
                        dim3(256), 0, st, (const unsigned long long *)src, a);

@@ -109,3 +109,48 @@ def test_waits_cut_short(pkg):
         a, b = (_run(pkg, t, s, m, "f64", o, order=order, **kw) for o in (1, 0))
         for u, v in zip(a[:3], b[:3]):
             np.testing.assert_array_equal(u, v)
+        with pkg.Engine(t, s, dtype="f64") as e:
+            e.set_option("pair_run", 1)
+            e.set_messages(m)
+            e.run(**kw) if order is None else e.run_sequential(order, **kw)
+            assert e.get_option("pair_run_give_up") == 1
+
+
+@pytest.mark.parametrize("order", ["jacobi", "sequential"])
+@pytest.mark.parametrize("launch,maxiter", [(1, 80), (2, 300), (2, 600), (3, 600)])
+def test_a_later_launch_gives_up(pkg, order, launch, maxiter):
+    """The run goes on launch by launch behind the launches that came to their end."""
+    print(f"case pair run gives up {order} launch {launch} of {maxiter} sweeps", flush=True)
+    g = pkg.named_grid((4, 3))
+    t, s, m = _net(pkg, g, 2, 2, "f64")
+    seq = None if order == "jacobi" else [t.slot(*x) for x in pkg.forest_cover_edge_sequence(g)]
+    for kw in ({"maxiter": maxiter}, {"maxiter": maxiter, "tol": 0.0},
+               {"maxiter": maxiter, "tol": 0.0, "criterion": "maxabs"}):
+        want = _run(pkg, t, s, m, "f64", 0, order=seq, **kw)
+        with pkg.Engine(t, s, dtype="f64") as e:
+            e.set_option("pair_run_give_up", launch)
+            e.set_messages(m)
+            r = e.run(**kw) if seq is None else e.run_sequential(seq, **kw)
+            got = (e.messages(), np.array(r.sweeps), np.array(r.at_iteration), np.array(r.delta),
+                   *e.residuals())
+            assert e.get_option("pair_run_give_up") == 1
+        for x, y in zip(got, want):
+            np.testing.assert_array_equal(x, y)
+
+
+def test_runs_after_one_that_gave_up(pkg):
+    """The next run goes launch by launch, the one after it tries again; given up again, two do;
+    after a run that ends, the count starts anew."""
+    print("case pair run tries again", flush=True)
+    t, s, m = _net(pkg, pkg.named_grid((4, 3)), 2, 2, "f64")
+    with pkg.Engine(t, s, dtype="f64") as e:
+        def run():
+            e.set_messages(m)
+            e.run(maxiter=20)
+            return e.get_option("pair_run_give_up")
+        e.set_option("pair_run_give_up", 1)
+        assert [run() for _ in range(8)] == [1, 1, 2, 2, 2, 3, 3, 3]
+        e.set_option("pair_run_give_up", 0)
+        assert [run() for _ in range(3)] == [3, 3, 3]  # left out twice more, then a whole run
+        e.set_option("pair_run_give_up", 1)
+        assert [run() for _ in range(3)] == [4, 4, 5]
