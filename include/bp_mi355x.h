@@ -348,9 +348,10 @@ int bp_last_run_ms(bp_context *ctx, double *ms);
  * memory).  Both return after the result is written; bp_last_run_ms then gives the device
  * time of the contraction's launches.  bp_cn_plan_info (any output may be NULL): the
  * result's rank, labels and entries, the input entries, the products' FP64 FLOPs, their
- * algorithmic bytes (every operand read once, every result written once) and the device
- * workspace.  bp_contract_network plans, executes and frees in
- * one call (out_cap: capacity of `out` in entries, out_labels: room for 64 labels). */
+ * algorithmic bytes (every operand of a launch read once, every result written once; two
+ * products fused into one launch leave out the result between them) and the device workspace.
+ * bp_contract_network plans, executes and frees in one call (out_cap: capacity of `out` in
+ * entries, out_labels: room for 64 labels). */
 typedef struct bp_cn_plan bp_cn_plan;
 enum { BP_CN_ORDER_LEFT = 0, BP_CN_ORDER_GREEDY = 1, BP_CN_ORDER_CHEAPEST = 2 };
 int bp_cn_plan_create(bp_context *ctx, int nt, const int *ranks, const int *labels,

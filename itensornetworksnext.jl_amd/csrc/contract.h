@@ -1032,11 +1032,10 @@ static int cn_build_plan(int nt, const int *ranks, const int *labels, int n_labe
                 }
                 const double m = (double)st.M / st.O;  // rows of the block form
                 p.flops += 2.0 * m * st.V * st.U * st.S * st.O + 2.0 * (double)st.M * st.N * st.K;
-                // the plan's figures are those of the two pairwise steps
-                const long long x = (long long)m * st.V * st.S * st.O;
-                p.bytes += 8.0 * ((double)ops[a].size + (double)ops[b].size + 2.0 * (double)x +
+                // the product of the first two stays in LDS
+                p.bytes += 8.0 * ((double)ops[a].size + (double)ops[b].size +
                                   (double)ops[b2].size + (double)R.size);
-                p.max_interm = std::max(p.max_interm, std::max(x, R.size));
+                p.max_interm = std::max(p.max_interm, R.size);
                 CnStep none;
                 none.a = a;
                 none.b = b;

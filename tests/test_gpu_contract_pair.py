@@ -73,3 +73,19 @@ def test_peps_norm(pkg, orc, shape, D, d):
         have = [x for x in have + labs if x not in shared]
     want = float(want)
     assert abs(got - want) <= 1e-12 * abs(want)
+
+
+def test_plan_figures(pkg):
+    """A fused pair's bytes: three operands and the result; FLOPs of both products.  Beyond the
+    fused kernel's extents (17 labels shared by A and B1) the product between counts twice."""
+    print("case contract pair figures", flush=True)
+    m, v, s, o, n = 300, 3, 2, 3, 9
+    for u, between in ((9, 0), (17, 2)):
+        size = {"m": m, "u": u, "v": v, "s": s, "o": o, "n": n}
+        labels = ["muv", "uso", "vsn"]
+        plan = pkg.ContractionPlan([tuple(size[x] for x in t) for t in labels],
+                                   [tuple(t) for t in labels], order=(0, 1, 3, 2))
+        moved = m * u * v + u * s * o + v * s * n + m * o * n + between * m * v * s * o
+        assert plan.bytes == 8.0 * moved
+        assert plan.flops == 2.0 * (m * v * u * s * o + m * o * v * s * n)
+        plan.close()
