@@ -1,5 +1,6 @@
-// pair.h -- sweep kernel for vertices of degree <= 4 and bond dimensions <= 8, FP64, complex
-// FP64 or FP32, in the unpadded site layout of the generic kernel (kernel: pair.hip).
+// pair.h -- sweep kernel for vertices of degree <= 4 and bond dimensions <= 8 (complex: <= 5 on
+// two bonds of a pair), FP64 or complex FP64, in the unpadded site layout of the generic kernel
+// (kernel: pair.hip).
 #pragma once
 
 #include <string>
@@ -12,7 +13,7 @@
 #define PAIR_RUN_SWEEPS 256  // sweeps of one pair_run launch
 #define PAIR_RUN_BAILED 2  // bit of the network's done flag: pair_run gave up
 
-enum { PAIR_F64 = 0, PAIR_C128 = 1, PAIR_F32 = 2 };
+enum { PAIR_F64 = 0, PAIR_C128 = 1 };
 
 // One vertex as the kernel reads it.  Its ports are split into two pairs of consecutive
 // tensor axes, positions (0, 1) and (2, 3): degree 4 (p0 p1)(p2 p3), degree 3 (p0 p1)(p2),

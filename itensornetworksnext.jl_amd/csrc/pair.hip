@@ -1,4 +1,4 @@
-// pair.hip -- BP messages of a vertex from two pair environments, on FP64 (or FP32) MFMA.
+// pair.hip -- BP messages of a vertex from two pair environments, on FP64 MFMA.
 //
 // The ports of a vertex are split into two pairs; with n = (i, j) running over the two bond
 // indices of a pair, the site tensor of each physical slice is an n0 x n1 matrix A_s.  With
@@ -29,7 +29,6 @@
 #include "pair.h"
 
 typedef double v4d __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 template <int TY>
 struct PairTy;
@@ -48,17 +47,6 @@ struct PairTy<PAIR_F64> {
 template <>
 struct PairTy<PAIR_C128> : PairTy<PAIR_F64> {
     static constexpr bool CX = true;
-};
-template <>
-struct PairTy<PAIR_F32> {
-    using E = float;
-    using V = v4f;
-    static constexpr bool CX = false;
-    static __device__ __forceinline__ V mma(E a, E b, V c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
-    static constexpr int ROW = 0;  // register r holds rows of the whole tile
 };
 
 // waves of the largest workgroup with NT tile columns
@@ -380,10 +368,9 @@ struct PairCore {
             mx = wave_max_v(sqrt((y - xo) * (y - xo) + (yi - xoi) * (yi - xoi)));
             fid = 1.0 - (dr * dr + di * di) / (nn * oo);
         } else {
-            const double yn = (double)y, yo = (double)xo;
-            const double dn = wave_sum_v(yn * yo), nn = wave_sum_v(yn * yn),
-                         oo = wave_sum_v(yo * yo);
-            mx = wave_max_v(fabs(yn - yo));
+            const double dn = wave_sum_v(y * xo), nn = wave_sum_v(y * y),
+                         oo = wave_sum_v(xo * xo);
+            mx = wave_max_v(fabs(y - xo));
             const double c = dn / sqrt(nn * oo);
             fid = 1.0 - c * c;
         }
@@ -403,8 +390,8 @@ struct PairCore {
             }
             return {real ? yr : 0.0, real ? yi : 0.0};
         } else {
-            const double S = wave_sum_v(real ? (double)x : 0.0);
-            return {real ? (E)(S != 0.0 ? (double)x / S : (double)x) : E(0), E(0)};
+            const double S = wave_sum_v(real ? x : 0.0);
+            return {real ? (S != 0.0 ? x / S : x) : 0.0, 0.0};
         }
     }
 };
@@ -498,7 +485,7 @@ __global__ __launch_bounds__(64 * pair_waves(NT)) void k_pair(
                     zv[2 * rec.vertex + 1] = zi;
                 }
             } else {
-                const double z = wave_sum_v(real ? (double)v.re * (double)ml[lane] : 0.0);
+                const double z = wave_sum_v(real ? v.re * ml[lane] : 0.0);
                 if (lane == 0) zv[rec.vertex] = z;
             }
             continue;
@@ -1029,7 +1016,7 @@ int pair_plan_build(PairPlan *p, int dtype, int plain, int nv, int nnet, const i
     p->all = (int)p->recs.size() == nv;
     for (int n = 0; n < nnet; ++n) p->covers = p->covers && lead[n] >= 0;
     p->nt = (maxn + 15) / 16;
-    const size_t esz = dtype == PAIR_F32 ? 4 : dtype == PAIR_C128 ? 16 : 8;
+    const size_t esz = dtype == PAIR_C128 ? 16 : 8;
     // Few tile columns leave few waves: share the slices between two more each.  Three columns
     // a half are six waves, which four SIMDs take in two turns; twelve are even, but take the
     // LDS of two workgroups, so only where the vertices are at most one to a CU (us a sweep of
@@ -1060,8 +1047,7 @@ int pair_plan_build(PairPlan *p, int dtype, int plain, int nv, int nnet, const i
         pair_release(p);
         return 5;
     }
-    const void *fn = dtype == PAIR_F64 ? pair_fn<PAIR_F64>(p->nt)
-                     : dtype == PAIR_C128 ? pair_fn<PAIR_C128>(p->nt) : pair_fn<PAIR_F32>(p->nt);
+    const void *fn = dtype == PAIR_F64 ? pair_fn<PAIR_F64>(p->nt) : pair_fn<PAIR_C128>(p->nt);
     if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)PAIR_LDS_MAX) != hipSuccess) {
         pair_release(p);
@@ -1108,9 +1094,7 @@ static int pair_any(const PairPlan *p, hipStream_t st, const void *sites, const 
                     const int *items, int n, double *zv) {
     if (p->dtype == PAIR_F64)
         return pair_go<PAIR_F64>(p, st, sites, src, dst, ctl, rf, ra, fold, items, n, zv);
-    if (p->dtype == PAIR_C128)
-        return pair_go<PAIR_C128>(p, st, sites, src, dst, ctl, rf, ra, fold, items, n, zv);
-    return pair_go<PAIR_F32>(p, st, sites, src, dst, ctl, rf, ra, fold, items, n, zv);
+    return pair_go<PAIR_C128>(p, st, sites, src, dst, ctl, rf, ra, fold, items, n, zv);
 }
 
 int pair_sweep(const PairPlan *p, hipStream_t st, const void *sites, const void *src, void *dst,
@@ -1139,8 +1123,7 @@ static const void *pair_run_fn(int nt) {
 }
 
 static const void *pair_run_any(const PairPlan *p) {
-    return p->dtype == PAIR_F64 ? pair_run_fn<PAIR_F64>(p->nt)
-           : p->dtype == PAIR_C128 ? pair_run_fn<PAIR_C128>(p->nt) : nullptr;
+    return p->dtype == PAIR_F64 ? pair_run_fn<PAIR_F64>(p->nt) : pair_run_fn<PAIR_C128>(p->nt);
 }
 
 static size_t pair_run_lds(const PairPlan *p) {
