@@ -1085,21 +1085,20 @@ static int resolve_path(bp_context *c) {
     return c->path == BP_PATH_VERTEX ? -1 : BP_PATH_MIXED;
 }
 
-// Allocate whatever workspace the next sweeps need, before any graph capture (no
-// allocation may happen inside a captured region).
+// FP32 networks of bond dimensions 9..12 beside ones of 5..8 sweep on two streams: the former
+// read their sites from HBM with one workgroup (D = 12) on a CU, the latter are products and fit
+// beside them, at any number of vertices.  us a sweep, one stream / two, lattices of D = 12
+// and 8: 4x4 each 80.4 / 74.5, 8x8 81.8 / 75.7, 11x11 88.3 / 79.5, 16x16 133 / 137 (the D = 12
+// slices alone fill the CUs twice over, evenly), 24x24 229 / 230, 32x32 416 / 406; of D = 10 and
+// 6: 11x11 73.8 / 70.7, 16x16 96.6 / 87.1; 16 networks of D = 4..12: 14.30 / 13.54 ms a call.
 static bool sweep_forks(const bp_context *c) {
-    return c->side && c->vplan_ok && c->dtype == BP_F32 && c->vplan.nv16 >= 256 &&
-           c->vplan.nv >= 256;
+    return c->vplan_ok && c->dtype == BP_F32 && c->vplan.nv16 > 0 && c->vplan.nv > 0;
 }
 
+// Allocate whatever workspace the next sweeps need, before any graph capture (no
+// allocation may happen inside a captured region).
 static int prepare_sweep(bp_context *c) {
-    // FP32 networks of bond dimensions 9..12 beside ones of up to 8, a chip's worth of vertices
-    // each: the former read their sites from HBM with one workgroup on a CU, the latter are
-    // products and fit beside them (16 networks of D = 4..12: 14.30 ms a call one after the
-    // other, 13.54 like this).  Smaller buckets leave
-    // room anyway and keep one stream (not measured).
-    if (!c->side && c->vplan_ok && c->dtype == BP_F32 && c->vplan.nv16 >= 256 &&
-        c->vplan.nv >= 256) {
+    if (!c->side && sweep_forks(c)) {
         HIPCHK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
         HIPCHK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
         HIPCHK(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
@@ -1243,7 +1242,7 @@ static int sweep_once(bp_context *c, const NetCtl &done, bool *folded = nullptr,
     if (path == BP_PATH_VERTEX && c->dtype == BP_F64) {
         RETCHK(v64_sweep(c, (const double *)src, (double *)dst, done, fold));
     } else if (path == BP_PATH_VERTEX || path == BP_PATH_MIXED) {
-        const bool fork = sweep_forks(c);
+        const bool fork = c->side && sweep_forks(c);
         const hipStream_t st = fork ? c->side : c->stream;
         if (fork) {
             HIPCHK(hipEventRecord(c->ev_fork, c->stream));

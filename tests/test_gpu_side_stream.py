@@ -1,5 +1,5 @@
-"""FP32 engines whose large-bond bucket (9..12) and small-bond buckets hold 256 vertices or more
-each sweep them on two streams (a fork and a join in every sweep, captured or not).  Every
+"""FP32 engines with a large-bond bucket (9..12) beside one of bond dimensions 5..8 sweep them on
+two streams (a fork and a join in every sweep, captured or not), whatever their sizes.  Every
 network runs the same kernels as in an engine of its own, which has one bucket and one stream:
 the messages, sweeps and deltas agree bit for bit, run after run."""
 import numpy as np
@@ -9,10 +9,15 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("use_graph", [True, False])
-def test_two_buckets_match_each_alone(pkg, use_graph):
-    print(f"case side stream graph={use_graph}", flush=True)
+@pytest.mark.parametrize("size", ["large", "small", "with D = 3"])
+def test_two_buckets_match_each_alone(pkg, size, use_graph):
+    print(f"case side stream {size} graph={use_graph}", flush=True)
     nets = [(pkg.named_grid((16, 17)), 10), (pkg.named_grid((18, 16)), 6),
             (pkg.heavy_hex_lattice(5, 12), 12), (pkg.heavy_hex_lattice(4, 8), 8)]
+    if size != "large":
+        nets = [(pkg.named_grid((2, 2)), 9), (pkg.named_grid((1, 3)), 12), (pkg.named_grid((3, 2)), 5)]
+    if size == "with D = 3":
+        nets.append((pkg.named_grid((4, 4)), 3))
     tops = [pkg.build_topology(g, D, 2) for g, D in nets]
     sites = [pkg.peps.random_sites(t, 3 + i, scale=pkg.peps.peps_scale(2, D))
              for i, (t, (_, D)) in enumerate(zip(tops, nets))]
