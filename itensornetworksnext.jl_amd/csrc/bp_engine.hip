@@ -1928,7 +1928,13 @@ static int ensure_h_state(bp_context *c) {
 //
 // us a call, launch by launch / here: 4x4 D = 2 386 / 213, 10x10 D = 4 complex 265 / 206, 23x17
 // D = 5 387 / 338, sequential 10x10 D = 4 2598 / 874.  A network takes it at any size that is
-// resident as a whole: where its sweeps are not latency, they keep the slices in LDS.
+// resident as a whole: where its sweeps are not latency, they keep the slices in LDS (us a
+// sweep, D = 5 at 20x20 17.0 / 11.8, D = 6 at 16x16 19.7 / 14.5).
+//
+// Sweeps in a run from which it pays, us a run of n sweeps to a tolerance: Jacobi from 4 (10x10
+// D = 4 n = 1 34 / 37, 3 52 / 46, 4 61 / 51; 23x17 D = 5 n = 2 60 / 63, 3 77 / 77, 4 95 / 89;
+// 16x16 D = 6 n = 2 66 / 69, 3 87 / 84, 4 107 / 99); sequential from the first (10x10 D = 4
+// n = 1 351 / 131, 16x16 D = 6 1019 / 590).
 static int pair_run_chunks(bp_context *c, bool sequential, const RunParams &rp, int *launched,
                            bool *over) {
     static std::mutex busy[64];
@@ -2647,7 +2653,7 @@ int bp_run_sequential(bp_context *c, const int *order, int norder, int maxiter, 
     std::vector<SeqLevel> levels;
     int it = 0, at = -1;
     double delta = INFINITY;
-    if (cap >= 2 && c->run_wait_us != 0 && pair_used(c) &&
+    if (c->run_wait_us != 0 && pair_used(c) &&
         pair_run_ready(&c->pair, c->nnet, c->nmsg, c->nports) &&
         seq_steps(c, order, norder, level, &steps)) {
         RunParams rp;

@@ -88,7 +88,8 @@ def test_sequential_runs(pkg, shape, D, dtype):
     shuffled = [int(q) for q in np.random.default_rng(5).permutation(t.nports)]
     for name, order in (("forest", forest), ("reversed", forest[::-1]), ("shuffled", shuffled),
                         ("sorted", sorted(forest))):
-        for kw in ({"maxiter": 60, "tol": 1e-9}, {"maxiter": 2}, {"maxiter": 7, "tol": 1e-30},
+        for kw in ({"maxiter": 60, "tol": 1e-9}, {"maxiter": 1}, {"maxiter": 1, "tol": 1e-9},
+                   {"maxiter": 2}, {"maxiter": 7, "tol": 1e-30},
                    {"maxiter": 60, "tol": 1e-8, "criterion": "maxabs"}):
             print(f"case pair run sequential {shape} D={D} {dtype} {name} {kw}", flush=True)
             a, b = (_run(pkg, t, s, m, dtype, o, order=order, **kw) for o in (250000, 0))
