@@ -559,6 +559,12 @@ static void scratch_release(bp_context *c, bool all = false) {
 // pageable buffer, the page faults of its zeroed memory and of `out`, and the conversion came
 // one after the other (9.4 MB of FP32 messages: a run at 256x256 D = 3
 // took 5.33 ms a call, now 4.64).
+//
+// The lines, us a call into newly allocated memory: FP32 in chunks from 256 KB (pageable / one
+// thread: 240 KB 31 / 37, 506 KB 51 / 52, 1 MB 88 / 77, 4 MB 406 / 221), FP64, which is not
+// converted, from 2 MB (1 MB 60 / 62, 2 MB 119 / 119, 4 MB 238 / 192); four threads from 2^19
+// values (one / four: FP32 1 MB 77 / 82, 2 MB 125 / 110, 8 MB 543 / 318, FP64 4 MB 192 / 153).
+// Chunks of 1, 2 and 4 MB: 212, 188 and 202 for 4 MB, 641, 606 and 595 for 16 MB of FP32.
 static int download_doubles(bp_context *c, const void *dev, bool f32, long long n, double *out) {
     constexpr size_t CHUNK = (size_t)2 << 20;  // bytes
     const size_t es = f32 ? sizeof(float) : sizeof(double);
@@ -799,7 +805,10 @@ static void free_buckets(bp_context *c) {
 
 // The pair kernel (pair.hip) sweeps the vertices it takes on the automatic path of FP64 and
 // complex contexts; a forced generic path and unnormalised updates stay on the generic
-// kernel.  Measured per sweep against it: see pair_plan_build.
+// kernel.  It is the faster one wherever it takes a vertex (us a sweep, generic / pair, square
+// lattices, d = 2): FP64 D = 2 4x4 20.7 / 8.5, 32x32 85 / 12.9, 256x256 4453 / 468; D = 4 4x4
+// 22.7 / 8.7, 256x256 5663 / 555; D = 5 64x64 494 / 107; complex D = 2 128x128 1316 / 187, D = 5
+// 4x4 27.9 / 19.0, 64x64 705 / 283.
 static bool pair_used(const bp_context *c) {
     return c->pair_ok && c->normalize && c->path == BP_PATH_AUTO &&
            (c->dtype == BP_F64 || c->is_cplx());
@@ -974,6 +983,9 @@ static int launch_edge_scalars(bp_context *c, const T *msgs) {
 // kernel, or the vertex bucket plus the generic kernel for the remaining networks.
 
 
+// Padded products per slice up to which the pair kernel stands in for the FP64 D <= 8 kernel:
+// between square lattices of D = 6 (324), faster at any size, and of D = 7 (832), slower above
+// 256 vertices.
 static constexpr double PAIR_MFMA_MAX = 400.0;
 
 // Bits of the networks' largest bond dimensions (up to 31).
@@ -1012,11 +1024,14 @@ static int ensure_v64(bp_context *c) {
                                      lmask) == 0)
                 c->v64_kind = 2;
         }
-        // The pair kernel in its place where it is the faster one: its time grows with the
-        // products it pads to 16 x 16, the other's is that of bond dimension 8.  us per sweep,
-        // d = 2, pair / other: D = 6 (324 products per slice) 23 / 36 at 16x16 and 71 / 82 at
-        // 32x32; D = 7 (832) 33 / 36 and 118 / 83; D = 8 of degree 3 (152) 21 / 41 at 8x16 hex
-        // (bond dimensions that the autotuner has timed stay with what it chose)
+        // The pair kernel in its place where it is the faster one at every size: its time grows
+        // with the products it pads to 16 x 16, the other's is that of bond dimension 8.  us a
+        // sweep, d = 2, pair / other at 4x4, 16x16, 20x20, 32x32: D = 6 (324 products per slice)
+        // 19.4 / 35.2, 19.7 / 37.7, 32.2 / 43.1, 77 / 84; D = 7 (832) 34.0 / 35.0, 34.5 / 37.6,
+        // 67 / 44, 132 / 83; D = 8 of degree 3 (152) 23.5 / 42.7 at 8x16 hex.  Bond dimensions
+        // that the autotuner has timed stay with what it chose.  Single sweeps decide: a resident
+        // network of D = 7 or 8 (up to 256 vertices) would take 28.4 or 32.9 us a sweep of a
+        // many-sweep launch against 37.6 or 38.2.
         RETCHK(ensure_pair(c));
         const unsigned timed = c->dtype == BP_F64 ? c->vx_timed & net_dim_mask(c) : 0u;
         if (c->v64_kind == 1 && c->pair_ok && c->pair.covers && timed == 0u &&
