@@ -264,8 +264,9 @@ int bp_local_energy_device(bp_context *ctx, const double *ops_v, const double *o
  *                      default 0x1FFC0);
  *   "small_bond"       1 (default): FP32 networks whose bond dimensions are all <= 4 run on
  *                      the small-bond kernels; 0: padded to 8 on the D <= 8 kernels;
- *   "fold_bookkeeping" 1 (default): when one D <= 8 vertex launch covers every network, the
- *                      sweep kernels also do the per-network convergence bookkeeping;
+ *   "fold_bookkeeping" 1 (default): when one launch covers every network (the D <= 8 vertex
+ *                      kernels, the FP64 and complex pair kernel; the small-bond kernels on a
+ *                      single network), the sweep kernels also do the convergence bookkeeping;
  *                      0: a separate bookkeeping kernel after every sweep (same results);
  *   "pair_run"         longest wait in us (default 250000) inside the launches that run many
  *                      sweeps of a small FP64 or complex network at once, after which the run
