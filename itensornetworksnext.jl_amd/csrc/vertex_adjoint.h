@@ -609,6 +609,9 @@ void k_vd_site(const float *__restrict__ vsites, const float *__restrict__ msgs,
 }
 
 // ---- vertex scalars: every port absorbed (the chain of the site form), then <E, A> in FP64.
+// 4 mode products in registers, two transposes through LDS, no open: 32 x 32, D = 8 15.2 us (33.6
+// MB of slices), against 38.8 for the message form, whose message out of port 0 (opened in FP32,
+// 5 times further from FP64) gave them before.
 template <int NS>
 __global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void k_vd_scalar(const float *__restrict__ vsites, const float *__restrict__ msgs,
