@@ -67,7 +67,8 @@ def test_autotune_cache_roundtrip(pkg, tmp_path):
 
 
 def test_autotune_fp64_generic_buckets(pkg, orc):
-    """FP64 (generic kernel only): tuned buckets keep 1e-10 parity with the oracle."""
+    """FP64 on a lattice that the pair kernel takes whole: the choice between the D <= 8 kernel
+    and that one keeps 1e-10 parity with the oracle (a bucket of the generic kernel: below)."""
     _say("case autotune fp64")
     t = pkg.build_topology(pkg.heavy_hex_lattice(2, 4), 5, 2)
     s = pkg.peps.random_sites(t, 9, scale=pkg.peps.peps_scale(2, 5))
