@@ -272,9 +272,9 @@ int bp_local_energy_device(bp_context *ctx, const double *ops_v, const double *o
  *                      sweeps of a small FP64 or complex network at once, after which the run
  *                      is repeated launch by launch, as are the next 1, 2, 4, .. runs while
  *                      it happens again; 0: launch by launch (same messages);
- *   "pair_run_give_up" reads how many of these launches have given up a wait; set to n > 0, the
- *                      n-th launch of every run waits for nothing and so gives up (tests of
- *                      the way back), 0 (default): none does;
+ *   "pair_run_give_up" n > 0: the n-th of these launches in every run waits for nothing and so
+ *                      gives up (tests of the way back); 0 (default): none does;
+ *   "pair_run_gave_up" (read only) how many of them have given up a wait;
  *   "keep_workspace"   MiB of device workspace that the context keeps between gate layers
  *                      (default 512; a layer at 32x32, D = 8 takes 368), and up to 32 MiB of
  *                      pinned staging for gates and message downloads; setting it gives back

@@ -1818,7 +1818,8 @@ int bp_get_option(bp_context *c, const char *name, int *value) {
     if (strcmp(name, "normalize") == 0) { *value = c->normalize; return BP_OK; }
     if (strcmp(name, "small_bond") == 0) { *value = c->vx_small; return BP_OK; }
     if (strcmp(name, "pair_run") == 0) { *value = c->run_wait_us; return BP_OK; }
-    if (strcmp(name, "pair_run_give_up") == 0) { *value = c->run_gave_up; return BP_OK; }
+    if (strcmp(name, "pair_run_give_up") == 0) { *value = c->run_give_up; return BP_OK; }
+    if (strcmp(name, "pair_run_gave_up") == 0) { *value = c->run_gave_up; return BP_OK; }
     if (strcmp(name, "keep_workspace") == 0) { *value = c->keep_mib; return BP_OK; }
     return set_err(BP_ERR_ARG, "unknown option %s", name);
 }

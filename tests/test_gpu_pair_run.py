@@ -114,7 +114,7 @@ def test_waits_cut_short(pkg):
             e.set_option("pair_run", 1)
             e.set_messages(m)
             e.run(**kw) if order is None else e.run_sequential(order, **kw)
-            assert e.get_option("pair_run_give_up") == 1
+            assert e.get_option("pair_run_gave_up") == 1
 
 
 @pytest.mark.parametrize("order", ["jacobi", "sequential"])
@@ -134,7 +134,7 @@ def test_a_later_launch_gives_up(pkg, order, launch, maxiter):
             r = e.run(**kw) if seq is None else e.run_sequential(seq, **kw)
             got = (e.messages(), np.array(r.sweeps), np.array(r.at_iteration), np.array(r.delta),
                    *e.residuals())
-            assert e.get_option("pair_run_give_up") == 1
+            assert e.get_option("pair_run_gave_up") == 1
         for x, y in zip(got, want):
             np.testing.assert_array_equal(x, y)
 
@@ -148,7 +148,7 @@ def test_runs_after_one_that_gave_up(pkg):
         def run():
             e.set_messages(m)
             e.run(maxiter=20)
-            return e.get_option("pair_run_give_up")
+            return e.get_option("pair_run_gave_up")
         e.set_option("pair_run_give_up", 1)
         assert [run() for _ in range(8)] == [1, 1, 2, 2, 2, 3, 3, 3]
         e.set_option("pair_run_give_up", 0)
